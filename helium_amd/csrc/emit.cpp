@@ -78,6 +78,29 @@ template <int NV> __device__ __forceinline__ void ld_vec(const f16_t* p, float (
 #pragma unroll
     for (int k = 0; k < NV; k++) e[k] = (float)v[k];
 }
+// Rows whose length is no multiple of the vector: NV elements from an address aligned to one element only (the hardware
+// takes 16-byte accesses at any such address), `n` of them inside the row; the rest read as zero and are not stored.
+template <class T> struct RawOf { typedef T type; };
+template <> struct RawOf<bf16_t> { typedef u16 type; };
+template <class T, int N> struct AnyVec { typedef typename Vec<T, N>::type type __attribute__((aligned(sizeof(T)))); };
+__device__ __forceinline__ float raw_value(const float*, float v) { return v; }
+__device__ __forceinline__ u32 raw_value(const u32*, u32 v) { return v; }
+__device__ __forceinline__ float raw_value(const bf16_t*, u16 v) { return __builtin_bit_cast(float, (u32)v << 16); }
+__device__ __forceinline__ float raw_value(const f16_t*, f16_t v) { return (float)v; }
+template <int NV, class T> __device__ __forceinline__ typename Vec<typename RawOf<T>::type, NV>::type ld_raw_n(const T* p, u32 n) {
+    typedef typename RawOf<T>::type R;
+    typename Vec<R, NV>::type v;
+    if (n >= NV) v = *(const typename AnyVec<R, NV>::type*)p;
+    else
+#pragma unroll
+    for (int k = 0; k < NV; k++) v[k] = k < n ? ((const R*)p)[k] : (R)0;
+    return v;
+}
+template <int NV, class T, class E> __device__ __forceinline__ void ld_vec_n(const T* p, E (&e)[NV], u32 n) {
+    const auto v = ld_raw_n<NV>(p, n);
+#pragma unroll
+    for (int k = 0; k < NV; k++) e[k] = raw_value(p, v[k]);
+}
 __device__ __forceinline__ float ld_one(const float* p) { return *p; }
 __device__ __forceinline__ u32 ld_one(const u32* p) { return *p; }
 __device__ __forceinline__ float ld_one(const bf16_t* p) { return __builtin_bit_cast(float, (u32)(*(const u16*)p) << 16); }
@@ -122,6 +145,16 @@ __device__ __forceinline__ void st_one(float* p, float v) { *p = v; }
 __device__ __forceinline__ void st_one(u32* p, u32 v) { *p = v; }
 __device__ __forceinline__ void st_one(bf16_t* p, float v) { *p = (bf16_t)v; }
 __device__ __forceinline__ void st_one(f16_t* p, float v) { *p = (f16_t)v; }
+template <int NV, bool STREAM = false, class T, class E> __device__ __forceinline__ void st_vec_n(T* p, const E (&e)[NV], u32 n) {
+    if (n >= NV) {
+        typename Vec<T, NV>::type v;
+#pragma unroll
+        for (int k = 0; k < NV; k++) v[k] = (T)e[k];
+        if constexpr (STREAM) __builtin_nontemporal_store(v, (typename AnyVec<T, NV>::type*)p); else *(typename AnyVec<T, NV>::type*)p = v;
+    } else
+#pragma unroll
+    for (int k = 0; k < NV; k++) if (k < n) st_one(p + k, e[k]);
+}
 // stores v and returns what a load of that element would give back (the value rounded to the element type)
 template <class T> __device__ __forceinline__ float store_and_keep(T* p, float v) {
     T t;
@@ -299,7 +332,7 @@ bool streams_out(const Arg& a) {
     return a.is_output && storage_bytes(a.dtype, (size_t)a.numel) >= (size_t(4) << 20);
 }
 
-int pick_nv(const Program& p, int max_bytes) {
+int pick_nv(const Program& p, int max_bytes, bool any_alignment) {
     const int n = (int)p.dims.size();
     const int64_t N = p.N();
     int widest = 1;  // bytes of the widest element moved along full rows
@@ -313,16 +346,17 @@ int pick_nv(const Program& p, int max_bytes) {
     if (p.acc_expr >= 0) widest = std::max(widest, 4);
     int nv = std::max(1, max_bytes / widest);
     auto ok = [&](int v) {
-        if (N % v) return false;
+        if (any_alignment ? N < v : N % v != 0) return false;
         for (auto& e : p.exprs) {
             if (e.kind != Expr::Load || !e.access.chain.empty()) continue;
             if (e.access.stride[n - 1] != 1) continue;
             if (e.access.dtype == HE_BOOL) return false;
-            for (int d = 0; d + 1 < n; d++)
+            for (int d = 0; d + 1 < n && !any_alignment; d++)
                 if (e.access.stride[d] % v) return false;
         }
         for (auto& o : p.outs) {
             if (!o.reduce && o.dtype == HE_BOOL) return false;
+            if (any_alignment) continue;
             if (!o.reduce && !o.stride.empty() && o.stride[n - 1] == 1)
                 for (int d = 0; d + 1 < n; d++)
                     if (o.stride[d] % v) return false;
@@ -460,9 +494,11 @@ std::string emit_exprs(const Program& p, const EmitCtx& cx) {
         if (cx.phase != 0) {
             const bool deferred = is_deferred_load(p, e, NV, cx.defer_row_varying_only);
             if (cx.phase == 1) {
-                if (deferred)
+                if (deferred && cx.count.empty())
                     s << "{ const size_t o = " << coord_sum(e.access.stride) << ";\nR.raw" << i << " = *(const " << raw_type(e.access.dtype, NV)
                       << "*)(a" << e.access.arg << " + o); }\n";
+                else if (deferred)
+                    s << "R.raw" << i << " = ld_raw_n<" << NV << ">(a" << e.access.arg << " + " << coord_sum(e.access.stride) << ", " << cx.count << ");\n";
                 continue;
             }
             if (deferred) {
@@ -487,10 +523,12 @@ std::string emit_exprs(const Program& p, const EmitCtx& cx) {
                 }
                 const int64_t sn = p.dims[n - 1] > 1 ? a.stride[n - 1] : 0;
                 const std::string ptr = "a" + std::to_string(a.arg);
+                // (columns past the row's end read the row's last one: their values go nowhere)
+                const std::string kth = cx.count.empty() ? "(size_t)k" : "(size_t)(k < " + cx.count + " ? (u32)k : " + cx.count + " - 1u)";
                 if (cx.row_part == 1) s << T << " " << v << "[" << NV << "] = {};\nif (col_ok) { const size_t o = " << coord_sum(a.stride) << ";\n";
                 else s << T << " " << v << "[" << NV << "];\n{ const size_t o = " << coord_sum(a.stride) << ";\n";
                 if (!a.chain.empty()) {
-                    s << "#pragma unroll\nfor (int k = 0; k < " << NV << "; k++) { u32 lin = (u32)(o + (size_t)k * " << sn
+                    s << "#pragma unroll\nfor (int k = 0; k < " << NV << "; k++) { u32 lin = (u32)(o + " << kth << " * " << sn
                       << "ull);\n";
                     for (auto& g : a.chain) emit_generic_map(s, g);
                     if (a.dtype == HE_BOOL)
@@ -498,16 +536,17 @@ std::string emit_exprs(const Program& p, const EmitCtx& cx) {
                     else
                         s << "\n" << v << "[k] = ld_one(" << ptr << " + lin); }\n";
                 } else if (a.dtype == HE_BOOL) {
-                    s << "#pragma unroll\nfor (int k = 0; k < " << NV << "; k++) { const size_t l = o + (size_t)k * " << sn
+                    s << "#pragma unroll\nfor (int k = 0; k < " << NV << "; k++) { const size_t l = o + " << kth << " * " << sn
                       << "ull; " << v << "[k] = ((" << ptr << "[l >> 5] >> (l & 31)) & 1u) != 0; }\n";
                 } else if (sn == 1 && NV > 1) {
-                    s << "ld_vec<" << NV << ">(" << ptr << " + o, " << v << ");\n";
+                    if (cx.count.empty()) s << "ld_vec<" << NV << ">(" << ptr << " + o, " << v << ");\n";
+                    else s << "ld_vec_n<" << NV << ">(" << ptr << " + o, " << v << ", " << cx.count << ");\n";
                 } else if (sn == 0) {
                     s << "const " << T << " t = ld_one(" << ptr << " + o);\n#pragma unroll\nfor (int k = 0; k < " << NV
                       << "; k++) " << v << "[k] = t;\n";
                 } else {
                     s << "#pragma unroll\nfor (int k = 0; k < " << NV << "; k++) " << v << "[k] = ld_one(" << ptr
-                      << " + o + (size_t)k * " << sn << "ull);\n";
+                      << " + o + " << kth << " * " << sn << "ull);\n";
                 }
                 s << "}\n";
                 break;

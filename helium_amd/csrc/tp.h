@@ -172,6 +172,9 @@ struct EmitCtx {
     // Loads of these arguments take the given expression (a value the surrounding code holds in a register) instead of
     // reading memory.
     const std::map<int, std::string>* arg_values = nullptr;
+    // Rows whose length is no multiple of nv: an expression for how many columns from n0 on the row still has. Vector
+    // accesses then assume the alignment of one element only, and the last vector of a row is loaded element by element.
+    std::string count;
 };
 // Per expression: whether its value ignores the row coordinate `m`.
 std::vector<char> row_invariant_exprs(const Program& p);
@@ -180,8 +183,9 @@ bool is_uniform_pow(const Program& p, int id);
 // Members of the struct phase 1 fills: one native vector per deferred Load of the program.
 std::string emit_raw_members(const Program& p, int nv, bool row_varying_only = false);
 std::string emit_exprs(const Program& p, const EmitCtx& cx);
-// Largest vector width (elements) legal for every full-row access and store of the program.
-int pick_nv(const Program& p, int max_bytes);
+// Largest vector width (elements) legal for every full-row access and store of the program; with `any_alignment` the one
+// that is legal when accesses are guarded (EmitCtx::count).
+int pick_nv(const Program& p, int max_bytes, bool any_alignment = false);
 // Whether an output tensor is written with streaming stores (st_vec<NV, true>): 4 MiB or more, i.e. too large to be
 // read back out of L2 by whoever comes next.
 bool streams_out(const Arg& a);

@@ -139,6 +139,38 @@ def test_fused_gemm_on_cpu(name, build, tile):
         compare(got, want)
 
 
+# Extents that no tile, chunk or vector divides: rows at any element's address, partial chunks along each extent, tiles
+# outside the matrix, the last columns of an epilogue.
+RAGGED = [
+    ("nn_odd", lambda: gemm_cases.plain(97, 131, 67), "64,64,64,2,2"),
+    ("nn_odd_batched", lambda: gemm_cases.plain(33, 45, 71, batch=3), "64,64,64,2,2"),
+    ("nn_a_direct_b_any_alignment", lambda: gemm_cases.plain(70, 77, 200), "64,64,64,2,2"),
+    ("nn_direct_with_edges", lambda: gemm_cases.plain(70, 72, 136), "64,64,64,2,2,3"),
+    ("nt_odd", lambda: gemm_cases.transposed_b(70, 99, 75, batch=2), "64,64,64,2,2"),
+    ("nt_direct_with_edges", lambda: gemm_cases.transposed_b(70, 99, 136), "64,64,64,2,2,4"),
+    ("tn_odd", lambda: gemm_cases.transposed_a(67, 101, 75), "64,64,64,2,2"),
+    ("tn_direct_with_edges", lambda: gemm_cases.transposed_a(72, 104, 75), "64,64,64,2,2"),
+    ("tt_odd", lambda: gemm_cases.transposed_a(67, 101, 75, both=True), "64,64,64,2,2"),
+    ("f32_nn_odd", lambda: gemm_cases.plain(37, 67, 43, dtype="f32"), "64,64,32,2,2"),
+    ("f32_nt_odd", lambda: gemm_cases.transposed_b(37, 67, 43, dtype="f32"), "64,64,32,2,2"),
+    ("f32_tn_direct_with_edges", lambda: gemm_cases.transposed_a(36, 68, 43, dtype="f32"), "64,64,32,2,2"),
+    ("mainloop_and_epilogue_odd", lambda: gemm_cases.bias_relu_colsum(67, 77, 75, mainloop=True), "64,64,64,2,2"),
+    ("row_bias_odd", lambda: gemm_cases.bias_relu_colsum(67, 75, 72, bias_axis=2, batch=2), "64,64,64,2,2"),
+    ("reductions_odd", lambda: gemm_cases.all_reductions(67, 77, 75), "64,64,64,2,2"),
+    ("readme_epilogue_odd", lambda: readme_fusion(75, False, True), "64,64,64,2,2"),
+    ("narrower_than_a_chunk", lambda: gemm_cases.plain(40, 5, 7), "64,64,64,2,2"),
+]
+
+
+@pytest.mark.parametrize("name,build,tile", RAGGED, ids=[c[0] for c in RAGGED])
+def test_ragged_products_on_cpu(name, build, tile):
+    g, inputs, outs = build()
+    _, got = run_emulated(g, inputs, tile)
+    f32 = name.startswith("f32")
+    want = oracle.outputs(g.nodes, inputs, round_mainloop_to=None if f32 else "bf16")
+    compare(got, want, **(dict(rel=1e-4, eps=1e-5) if f32 else {}))
+
+
 def test_argument_order_is_producers_then_leaves():
     g, inputs, outs = gemm_cases.bias_relu_colsum(64, 64, 64, mainloop=True)
     k = ha.TileKernel.fused(g)
