@@ -27,6 +27,7 @@ struct Tile {
     int bm = 256, bn = 256, bk = 64;  // workgroup tile
     int wm = 2, wn = 4;               // waves along m / n (wm * wn * 64 threads)
     int stages = 2;                   // LDS stages (direct global->LDS loads use a deeper ring)
+    int wk = 1;                       // groups of wm * wn waves that share the tile's k range (their sums meet in LDS)
 };
 
 const char* kGemmPrelude = R"HIP(
@@ -81,8 +82,10 @@ template <int S> __device__ __forceinline__ u32x4 chunk_from(u32x4 v) {
 
 // Kernel body; problem and tile constants are #defines in front of it.
 const char* kGemmBody = R"HIP(
-#define NWAVES (WAVES_M * WAVES_N)
+#define NWAVES (WAVES_M * WAVES_N)  /* of one k group: WAVES_K of them take every WAVES_K-th k-tile each, in a ring of their own */
 #define NTHREADS (NWAVES * 64)
+#define ALL_WAVES (NWAVES * WAVES_K)
+#define ALL_THREADS (NTHREADS * WAVES_K)
 #define WTM (BM / WAVES_M)        /* wave tile */
 #define WTN (BN / WAVES_N)
 #define MB (WTM / 32)             /* 32x32 MFMA blocks per wave tile */
@@ -98,7 +101,7 @@ const char* kGemmBody = R"HIP(
 #define A_PER_THREAD (BM * A_CHUNKS / NTHREADS)
 #define B_PER_THREAD (BK * B_CHUNKS / NTHREADS)
 #define EP (WTN + 4)              /* float pitch of the epilogue strip */
-#define EPI_STEPS ((32 * WTN) / (64 * NVE))  /* NVE-wide steps a lane takes through one 32-row block */
+#define EPI_STEPS ((32 * WTN) / (64 * NVE * WAVES_K))  /* NVE-wide steps a lane takes through one 32-row block */
 #if NSTAGES * STAGE_BYTES < NWAVES * 32 * EP * 4
 #error "the epilogue strip does not fit in the operand stages"
 #endif
@@ -406,29 +409,46 @@ __device__ __forceinline__ void direct_tile(const unsigned char* __restrict__ rd
 #ifndef KERNEL_ATTRS
 /* NWAVES / 4 waves per SIMD and workgroup: with four waves each one owns the full 512-register budget; WGS_PER_CU
    workgroups are meant to share a CU */
-#define KERNEL_ATTRS __attribute__((amdgpu_waves_per_eu(NWAVES / 4 * WGS_PER_CU, NWAVES / 4 * WGS_PER_CU)))
+#define KERNEL_ATTRS __attribute__((amdgpu_waves_per_eu(ALL_WAVES / 4 * WGS_PER_CU, ALL_WAVES / 4 * WGS_PER_CU)))
 #endif
-extern "C" __global__ __launch_bounds__(NTHREADS) KERNEL_ATTRS
+extern "C" __global__ __launch_bounds__(ALL_THREADS) KERNEL_ATTRS
 void fused_matmul(KERNEL_PARAMS) {
-    __shared__ __attribute__((aligned(16))) unsigned char lds[NSTAGES * STAGE_BYTES];
-    const u32 tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ __attribute__((aligned(16))) unsigned char lds[WAVES_K * NSTAGES * STAGE_BYTES];
+#if WAVES_K > 1
+    const u32 kgroup = __builtin_amdgcn_readfirstlane(threadIdx.x / NTHREADS), tid = threadIdx.x % NTHREADS;
+#else
+    constexpr u32 kgroup = 0;
+    const u32 tid = threadIdx.x;
+#endif
+    unsigned char* const ring = lds + kgroup * (NSTAGES * STAGE_BYTES);
+    const u32 lane = tid & 63, wave = tid >> 6;
     const u32 wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
     u32 tile_m, tile_n;
     TILE_ORDER
 #if SPLIT_K > 1
     // blockIdx.y is the k-range index, not a batch index: this workgroup multiplies k-tiles [kt0, kt0 + KT)
     const u32 bz = 0, split = blockIdx.y, kt0 = split * KT_PER_SPLIT;
-    const u32 KT = kt0 >= KT_ALL ? 0u : (KT_ALL - kt0 < KT_PER_SPLIT ? KT_ALL - kt0 : KT_PER_SPLIT);
+    const u32 KT_RANGE = kt0 >= KT_ALL ? 0u : (KT_ALL - kt0 < KT_PER_SPLIT ? KT_ALL - kt0 : KT_PER_SPLIT);
 #else
     const u32 bz = blockIdx.y, kt0 = 0;
-    constexpr u32 KT = KT_ALL;
+    constexpr u32 KT_RANGE = KT_ALL;
+#endif
+    // k-tiles of this wave's group, and how often the workgroup's waves meet at the loop's barrier (a group of one wave
+    // shares its stages with nobody and meets nobody)
+#if WAVES_K > 1
+    const u32 KT = KT_RANGE > kgroup ? (KT_RANGE - kgroup + WAVES_K - 1) / WAVES_K : 0u;
+    const u32 K_ROUNDS = NWAVES == 1 ? KT : (KT_RANGE + WAVES_K - 1) / WAVES_K;
+#define K_MINE (NWAVES == 1 || kt < KT)
+#else
+    const u32 KT = KT_RANGE, K_ROUNDS = KT;
+#define K_MINE true
 #endif
     const u32 m0 = tile_m * BM, n0 = tile_n * BN;
     EPILOGUE_EARLY
     // Optional rotation of the k loop per workgroup (tuning knob, off by default: workgroups that share an A or B
     // panel read the same k range at the same time, which is what lets them share it through L2).
     const u32 k_shift = KT ? (STAGGER_EXPR) % KT : 0u;
-    auto k_tile = [&](u32 kt) { u32 x = kt + k_shift; return kt0 + (x >= KT ? x - KT : x); };
+    auto k_tile = [&](u32 kt) { u32 x = kt + k_shift; return kt0 + (x >= KT ? x - KT : x) * WAVES_K + kgroup; };
 
     f32x16 acc[MB][NB];
 #pragma unroll
@@ -492,7 +512,7 @@ void fused_matmul(KERNEL_PARAMS) {
     };
     auto stage_store = [&](u32 kt, u32 buf) {
         const u32 k0 = k_tile(kt) * BK; (void)k0;
-        unsigned char* la = lds + buf * STAGE_BYTES;
+        unsigned char* la = ring + buf * STAGE_BYTES;
         unsigned char* lb = la + A_TILE_BYTES;
         (void)la; (void)lb;
 #if !DIRECT_A
@@ -572,18 +592,24 @@ void fused_matmul(KERNEL_PARAMS) {
         if (st < KT) {
 #pragma unroll
             for (int i = 0; i < A_DPW + B_DPW; i++)
-                direct_issue(lds + st * STAGE_BYTES, A_TILE_AT(k_tile(st) * BK), B_TILE_AT(k_tile(st) * BK), GK - k_tile(st) * BK, wpos, i);
+                direct_issue(ring + st * STAGE_BYTES, A_TILE_AT(k_tile(st) * BK), B_TILE_AT(k_tile(st) * BK), GK - k_tile(st) * BK, wpos, i);
         }
 #endif
 #if STAGED
-    stage_load(0);
-    stage_store(0, 0);
+#if SPLIT_K > 1 || WAVES_K > 1
+    if (KT)
+#endif
+    {
+        stage_load(0);
+        stage_store(0, 0);
+    }
 #endif
     Frags frags;
     init_frags(frags);
-    for (u32 kt = 0; kt < KT; kt++) {
+    for (u32 kt = 0; kt < K_ROUNDS; kt++) {
 #if DIRECT_LOADS
         // tile kt must have landed; up to NSTAGES - 2 younger tiles may still be in flight
+        // (a group whose tiles are used up has nothing in flight)
         const u32 younger = KT - 1 - kt < NSTAGES - 2 ? KT - 1 - kt : NSTAGES - 2;
         // (0x0070: no wait on the export counter, lgkmcnt(0) so that this wave's LDS reads and staged LDS stores are done)
         if (younger >= 3) __builtin_amdgcn_s_waitcnt(0x0070 | WAITCNT_VM(3 * (A_DPW + B_DPW)));
@@ -593,13 +619,18 @@ void fused_matmul(KERNEL_PARAMS) {
 #endif
         // every wave's share of tile kt is in LDS (direct loads waited for above, staged stores made before the
         // barrier) and nobody still reads the stage that this iteration refills
-#if DIRECT_LOADS
+#if WAVES_K > 1 && NWAVES == 1
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#elif DIRECT_LOADS
         // The bare barrier: __syncthreads() carries a fence for which the compiler drains every outstanding load,
         // the ones for younger stages included, and a ring deeper than two stages would gain nothing.
         __builtin_amdgcn_s_barrier();
 #else
         __syncthreads();
 #endif
+        if (!K_MINE) continue;
         const u32 next = kt + NSTAGES - 1;
         const bool more = next < KT;
 #if STAGED
@@ -609,10 +640,10 @@ void fused_matmul(KERNEL_PARAMS) {
 #endif
 #if DIRECT_LOADS
         const u32 knext = more ? k_tile(next) * BK : 0u;
-        direct_tile(lds + (kt % NSTAGES) * STAGE_BYTES, lds + (next % NSTAGES) * STAGE_BYTES, A_TILE_AT(knext),
+        direct_tile(ring + (kt % NSTAGES) * STAGE_BYTES, ring + (next % NSTAGES) * STAGE_BYTES, A_TILE_AT(knext),
                     B_TILE_AT(knext), GK - knext, more, acc, wpos, frags);
 #else
-        compute_tile(lds + (kt % NSTAGES) * STAGE_BYTES, acc, wpos, frags, [](int) {});
+        compute_tile(ring + (kt % NSTAGES) * STAGE_BYTES, acc, wpos, frags, [](int) {});
 #endif
 #if STAGED
         STAGE_SCHED_BARRIER
@@ -624,7 +655,9 @@ void fused_matmul(KERNEL_PARAMS) {
     __syncthreads();
 
     // ---- epilogue: accumulators -> wave-private LDS strip -> row-major NV-wide vectors -----------------------
-    float* strip = (float*)lds + wave * (32 * EP);
+    // (with several k groups: a strip per group, and the groups share the steps through the sum of their strips)
+    float* strip = (float*)lds + (kgroup * NWAVES + wave) * (32 * EP);
+    const float* const strip0 = (const float*)lds + wave * (32 * EP);
     EPILOGUE_SETUP
 #pragma unroll
     for (int i = 0; i < MB; i++) {
@@ -635,26 +668,31 @@ void fused_matmul(KERNEL_PARAMS) {
                 const u32 row = (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3), col = j * 32 + (lane & 31);
                 strip[row * EP + col] = acc[i][j][e];
             }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#if WAVES_K > 1
+#define STRIPS_MEET __syncthreads();
+#else
+#define STRIPS_MEET __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); __builtin_amdgcn_wave_barrier(); __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#endif
+        STRIPS_MEET
 #pragma unroll
-        for (int step = 0; step < (32 * WTN) / (64 * NVE); step++) {
+        for (int step = 0; step < EPI_STEPS; step++) {
             EPILOGUE_PREFETCH
-            const u32 idx = (step * 64 + lane) * NVE;
+            const u32 idx = ((step * WAVES_K + kgroup) * 64 + lane) * NVE;
             const u32 row = idx / WTN, col = idx % WTN;
             const u32 m = m0 + wave_m * WTM + i * 32 + row;
             const u32 nn = n0 + wave_n * WTN + col;
             float acc_v[NVE];
 #pragma unroll
-            for (int k = 0; k < NVE; k++) acc_v[k] = strip[row * EP + col + k];
+            for (int k = 0; k < NVE; k++) acc_v[k] = strip0[row * EP + col + k];
+#pragma unroll
+            for (int g = 1; g < WAVES_K; g++)
+#pragma unroll
+                for (int k = 0; k < NVE; k++) acc_v[k] += strip0[g * (NWAVES * 32 * EP) + row * EP + col + k];
             const bool ok = m < GM && nn < GN;  // kept a run-time test even when every tile is full: with it folded away the
             // compiler merges the unrolled steps, hoists every step's loads and spills (2.3x slower on the 40-op epilogue)
             EPILOGUE_BODY
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        STRIPS_MEET
     }
     EPILOGUE_FINISH
 }
@@ -738,7 +776,10 @@ int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch) {
     // 64x64 tiles fill the chip before a split k range has to: the partial tiles of a split cost a second pass over
     // the output (a 3136 x 512 x 4608 convolution: 51 us with 128x128 tiles and four k ranges, 34 us with 64x64 tiles)
     if (((M + 63) / 64) * ((N + 63) / 64) >= 192) return 1;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 8, 1024}));
+    // So do the waves of a workgroup that share a small tile's k range (small_tile): such a product costs about 2.7 us and
+    // 0.2 us for every tile that a wave takes, the second launch of a split one 4 us (32 x 512 x 4608: 6.3 us against 10).
+    if (k_tiles <= 192) return 1;
+    return (int)std::max<int64_t>(1, std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 96, 1024}));
 }
 
 bool operand_b_prefers_nk(const tp::Program& op_b) {
@@ -794,6 +835,44 @@ void validate_gemm_epilogue(const tp::Program& epi) {
     }
 }
 
+// Tiles for a product that has too few of the usual ones to fill the chip: 32x32 to 64x64, one wave computes the whole
+// tile, and four or eight waves of the workgroup take every fourth or eighth k-tile each (Tile::wk). What bounds such a
+// product is the chain of its k-tiles, each a round trip to memory and a few matrix instructions of latency (a 32x32x2 f32
+// instruction alone takes 64 cycles): the waves' chains run side by side, wait for nobody inside the loop, and meet once, in
+// LDS, ahead of the epilogue. False where the tiles chosen otherwise are faster. Measured (us, before -> after; rows x
+// columns x k; before: 64x64 or 128x128 tiles of four waves):
+//   f32   64x512x784 57.3 -> 7.0   64x10x512 38.9 -> 5.2   256x512x512 10.4 -> 5.2   300x700x2000 46.1 -> 13.7
+//   bf16  64x512x784 6.5 -> 3.2    128x256x2304 12.5 -> 4.3   32x512x4608 20.4 -> 6.3   512x512x2048 8.5 -> 6.0
+// and where the line lies: 32x32 tiles (two workgroups of four waves fit a CU) as long as they are one round of the CUs
+// (512x1024x512 bf16, 512 of them: 3.9 against 4.0; 1000x1000x1000, 1024 of them: 11.3 against 6.9; f32 up to 640, its
+// instructions being longer: 768x768x768 17.9 -> 14.9, 1024x1024x1024 23.5 -> 23.8), then 64x32 or 32x64 (640x640x4096
+// bf16 19.9 -> 13.6, 512x1024x1024 f32 22.7 -> 12.4), and 64x64 where k is long (1024x1024x4096 bf16 21.0 -> 16.5, 768x768x3072
+// 15.9 -> 11.9, but 768x768x768 4.7 -> 5.2).
+bool small_tile(const GemmProblem& pr, bool f32, Tile* t) {
+    if (pr.split_k > 1) return false;  // shared over workgroups instead, with tiles that go with it
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((pr.M + bm - 1) / bm) * ((pr.N + bn - 1) / bn) * pr.batch; };
+    const int64_t k_tiles = (pr.K + t->bk - 1) / t->bk;
+    constexpr int64_t kCus = 256;
+    int bm = 32, bn = 32, wk = 4;
+    const bool tall = tiles(64, 32) <= tiles(32, 64);
+    if (tiles(32, 32) <= kCus) {
+        if (k_tiles >= 8) wk = 8;
+    } else if (k_tiles >= 8 && tiles(tall ? 64 : 32, tall ? 32 : 64) <= kCus) {
+        (tall ? bm : bn) = 64;
+    } else if (f32 && k_tiles >= 24 && tiles(32, 32) <= kCus * 5 / 2) {
+        // 32x32
+    } else if (k_tiles >= 24 && tiles(64, 64) <= kCus) {
+        bm = bn = 64;
+    } else {
+        return false;
+    }
+    t->bm = bm;
+    t->bn = bn;
+    t->wm = t->wn = 1;
+    t->wk = wk;
+    return true;
+}
+
 GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     const GemmProblem& pr = prob_;
     HE_REQUIRE(pr.M > 0 && pr.N > 0 && pr.K > 0 && pr.batch > 0, HE_ERR_INVALID, "empty GEMM");
@@ -815,10 +894,10 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     const bool want_direct = !tuning::get("HELIUM_HIP_GEMM_NO_DIRECT");
     const int esz = 16 / epc;  // bytes per multiplicand
     if (const char* env = tuning::get("HELIUM_HIP_GEMM_TILE")) {
-        int v[6] = {256, 256, 64, 2, 4, 2};
-        int n = sscanf(env, "%d,%d,%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5]);
-        HE_REQUIRE(n >= 5, HE_ERR_INVALID, "HELIUM_HIP_GEMM_TILE wants bm,bn,bk,wm,wn[,stages]");
-        t = {v[0], v[1], v[2], v[3], v[4], v[5]};
+        int v[7] = {256, 256, 64, 2, 4, 2, 1};
+        int n = sscanf(env, "%d,%d,%d,%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6]);
+        HE_REQUIRE(n >= 5, HE_ERR_INVALID, "HELIUM_HIP_GEMM_TILE wants bm,bn,bk,wm,wn[,stages[,k groups]]");
+        t = {v[0], v[1], v[2], v[3], v[4], v[5], v[6]};
     } else {
         if (f32) t.bk = 32;  // same bytes per tile row as 64 two-byte multiplicands
         // A skinny product (few output columns, many rows: a convolution with 64 output channels) takes tiles as
@@ -832,7 +911,9 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         // than the unused half of a 256x64 tile costs (7x7 stem: 885 us with 128x128 tiles, 408 with 256x32, 276 with 256x64).
         const bool narrow = !f32 && pr.N <= 32 && pr.N > 16 && pr.M >= 256 * 256;
         const bool gathered_by_element = pr.conv_a.on && pr.conv_a.C % epc != 0;
-        if (skinny || (narrow && gathered_by_element)) {
+        if (small_tile(pr, f32, &t)) {
+            // (t is set)
+        } else if (skinny || (narrow && gathered_by_element)) {
             t.bm = 256;
             t.bn = 64;
             t.wm = 4;
@@ -915,10 +996,11 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     HE_REQUIRE(!pr.out_rows.on || (pr.split_k == 1 && pr.batch == 1 && pr.epi.outs.size() == 1 && !pr.epi.outs[0].reduce), HE_ERR_INVALID,
                "scattered output rows need a plain epilogue and a whole k range");
     HE_REQUIRE(t.bm % (t.wm * 32) == 0 && t.bn % (t.wn * 32) == 0 && (t.bk == 64 || t.bk == 32) && (!f32 || t.bk == 32), HE_ERR_INVALID, "bad GEMM tile");
-    const int threads = t.wm * t.wn * 64;
+    const int threads = t.wm * t.wn * 64;  // of one k group
+    HE_REQUIRE(t.wk >= 1 && threads * t.wk <= 512, HE_ERR_INVALID, "GEMM workgroups have at most 8 waves");
     HE_REQUIRE(threads == 64 || threads == 128 || threads == 256 || threads == 512, HE_ERR_INVALID, "GEMM workgroups have 1, 2, 4 or 8 waves");
     HE_REQUIRE((t.bm * t.bk / epc) % threads == 0 && (t.bk * t.bn / epc) % threads == 0, HE_ERR_INVALID, "bad GEMM tile");
-    HE_REQUIRE(t.stages >= 2 && t.stages <= 5 && t.stages * (t.bm + t.bn) * t.bk * (16 / epc) <= 160 * 1024, HE_ERR_INVALID,
+    HE_REQUIRE(t.stages >= 2 && t.stages <= 5 && t.wk * t.stages * (t.bm + t.bn) * t.bk * (16 / epc) <= 160 * 1024, HE_ERR_INVALID,
                "GEMM tile exceeds LDS");
     const int wtn = t.bn / t.wn;
     // Reductions of the epilogue never meet in memory: every workgroup (for row sums: every wave) parks its partial
@@ -1026,7 +1108,8 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     // (rows that are no multiple of 4 elements: guarded vectors, loaded and stored element by element only at a row's end)
     const bool any_e = nve < 4 && nve_any > nve;
     if (any_e) nve = nve_any;
-    while (nve > 1 && ((32 * wtn) % (64 * nve) != 0)) nve /= 2;
+    while (nve > 1 && ((32 * wtn) % (64 * nve * t.wk) != 0)) nve /= 2;
+    HE_REQUIRE((32 * wtn) % (64 * nve * t.wk) == 0, HE_ERR_INVALID, "bad GEMM tile");
     const std::string epi_count = any_e && nve > 1 ? "(GN - n0)" : "";
     const int lanes_per_row = wtn / nve;           // lanes that share one row of the strip in one step
     const int colsets = std::max(1, lanes_per_row / 64);  // distinct column sets a lane visits
@@ -1041,14 +1124,14 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     // waves of both must fit the register file, so the allocation is held to the budget of twice the waves.
     std::string wgs_per_cu_attr;
     {
-        const int lds_bytes = t.stages * (t.bm + t.bn) * t.bk * esz;
+        const int lds_bytes = t.wk * t.stages * (t.bm + t.bn) * t.bk * esz;
         const int acc_regs = t.bm * t.bn / threads;
         int wgs = tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU") ? atoi(tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU")) : (lds_bytes * 2 <= 160 * 1024 && acc_regs <= 32 ? 2 : 1);
-        if (threads < 256) wgs = 1;
+        if (threads * t.wk < 256) wgs = 1;
         wgs_per_cu_attr = "\n#define WGS_PER_CU " + std::to_string(std::max(1, wgs));
     }
     s << "#define BM " << t.bm << "\n#define BN " << t.bn << "\n#define BK " << t.bk << "\n#define WAVES_M " << t.wm
-      << "\n#define WAVES_N " << t.wn << wgs_per_cu_attr << "\n#define NSTAGES " << t.stages << "\n#define NVE " << nve << "\n#define MMA_BF16 " << (pr.mma_dtype == HE_BF16 ? 1 : 0) << "\n#define MMA_F32 " << (f32 ? 1 : 0)
+      << "\n#define WAVES_N " << t.wn << "\n#define WAVES_K " << t.wk << wgs_per_cu_attr << "\n#define NSTAGES " << t.stages << "\n#define NVE " << nve << "\n#define MMA_BF16 " << (pr.mma_dtype == HE_BF16 ? 1 : 0) << "\n#define MMA_F32 " << (f32 ? 1 : 0)
       << "\n#define STAGGER_EXPR " << (tuning::measuring() && tuning::get("HELIUM_HIP_GEMM_STAGGER") ? tuning::get("HELIUM_HIP_GEMM_STAGGER") : "0u")
       << "\n#define ISSUE_FRONT " << (issue_front ? 1 : 0)
       // measurement only (HELIUM_HIP_TUNING=measure): bit 0 drops the direct loads, bit 1 the fragment reads, bit 2 the
@@ -1252,7 +1335,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         std::string pass;
         for (size_t a = 0; a < pr.epi.args.size(); a++) pass += "a" + std::to_string(a) + ", ";
         prefetch << "{ const int q1 = i * EPI_STEPS + step + EPI_DEPTH;\nif (q1 < MB * EPI_STEPS) {\nconst int i1 = q1 / EPI_STEPS, s1 = q1 % EPI_STEPS;\n"
-                 << "const u32 idx1 = (s1 * 64 + lane) * NVE;\nconst u32 m1 = m0 + wave_m * WTM + i1 * 32 + idx1 / WTN, nn1 = n0 + wave_n * WTN + idx1 % WTN;\n"
+                 << "const u32 idx1 = ((s1 * WAVES_K + kgroup) * 64 + lane) * NVE;\nconst u32 m1 = m0 + wave_m * WTM + i1 * 32 + idx1 / WTN, nn1 = n0 + wave_n * WTN + idx1 % WTN;\n"
                  << "if (m1 < GM && nn1 < GN) epi_load(" << pass << "bz, m1, nn1, Rb[q1 % (EPI_DEPTH + 1)]);\n} }\n";
     }
     for (size_t a = 0; a < pr.epi.args.size(); a++)
@@ -1262,7 +1345,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         std::string pass;
         for (size_t a = 0; a < pr.epi.args.size(); a++) pass += "a" + std::to_string(a) + ", ";
         setup << "RawE Rb[EPI_DEPTH + 1];\n#pragma unroll\nfor (int q1 = 0; q1 < EPI_DEPTH && q1 < MB * EPI_STEPS; q1++) {\nconst int i1 = q1 / EPI_STEPS, s1 = q1 % EPI_STEPS;\n"
-              << "const u32 idx1 = (s1 * 64 + lane) * NVE;\nconst u32 m1 = m0 + wave_m * WTM + i1 * 32 + idx1 / WTN, nn1 = n0 + wave_n * WTN + idx1 % WTN;\n"
+              << "const u32 idx1 = ((s1 * WAVES_K + kgroup) * 64 + lane) * NVE;\nconst u32 m1 = m0 + wave_m * WTM + i1 * 32 + idx1 / WTN, nn1 = n0 + wave_n * WTN + idx1 % WTN;\n"
               << "if (m1 < GM && nn1 < GN) epi_load(" << pass << "bz, m1, nn1, Rb[q1]);\n}\n";
     }
     if (hoisted) {
@@ -1377,7 +1460,8 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
             if (o.reduce && o.fold_m && o.fold_n) nsc++;
         }
         if (ncol + nsc) {
-            HE_REQUIRE((size_t)(ncol * t.wm * t.bn + nsc * t.wm * t.wn) * 4 <= (size_t)t.stages * (t.bm + t.bn) * t.bk * esz, HE_ERR_INTERNAL,
+            const int rows_of = t.wm * t.wk;  // waves that hold sums of one column
+            HE_REQUIRE((size_t)(ncol * rows_of * t.bn + nsc * rows_of * t.wn) * 4 <= (size_t)t.wk * t.stages * (t.bm + t.bn) * t.bk * esz, HE_ERR_INTERNAL,
                        "reduction exchange exceeds the tile's LDS");
             finish << "__syncthreads();\nfloat* red = (float*)lds;\n";
             int ci = 0, si = 0;
@@ -1390,10 +1474,10 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                            << oi << "[c][k];\n";
                     for (int off = lanes_per_row; off < 64; off *= 2) finish << "r += __shfl_xor(r, " << off << ", 64);\n";
                     finish << "const u32 col = ((c * 64 + lane) * NVE) % WTN + k;\n";
-                    finish << "if (lane < " << std::min(lanes_per_row, 64) << ") red[" << ci * t.wm * t.bn << " + wave_m * BN + wave_n * WTN + col] = r;\n}\n}\n";
+                    finish << "if (lane < " << std::min(lanes_per_row, 64) << ") red[" << ci * rows_of * t.bn << " + (kgroup * WAVES_M + wave_m) * BN + wave_n * WTN + col] = r;\n}\n}\n";
                     ci++;
                 } else {
-                    finish << "{ float r = wave_reduce<0, 64>(rs" << oi << ");\nif (lane == 0) red[" << ncol * t.wm * t.bn + si * t.wm * t.wn << " + wave] = r; }\n";
+                    finish << "{ float r = wave_reduce<0, 64>(rs" << oi << ");\nif (lane == 0) red[" << ncol * rows_of * t.bn + si * rows_of * t.wn << " + kgroup * NWAVES + wave] = r; }\n";
                     si++;
                 }
             }
@@ -1404,14 +1488,14 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                 if (!o.reduce || !o.fold_m) continue;
                 const RedOut& ro = red_of(oi);
                 if (!o.fold_n) {
-                    finish << "for (u32 c = tid; c < BN; c += NTHREADS) {\nfloat r = 0.0f;\n#pragma unroll\nfor (int w = 0; w < WAVES_M; w++) r += red["
-                           << ci * t.wm * t.bn << " + w * BN + c];\nif (n0 + c < GN) " << (fold_in_kernel ? "HE_WS_STORE(red_ws + " : "red_ws[") << ro.off
+                    finish << "for (u32 c = threadIdx.x; c < BN; c += ALL_THREADS) {\nfloat r = 0.0f;\n#pragma unroll\nfor (int w = 0; w < WAVES_K * WAVES_M; w++) r += red["
+                           << ci * rows_of * t.bn << " + w * BN + c];\nif (n0 + c < GN) " << (fold_in_kernel ? "HE_WS_STORE(red_ws + " : "red_ws[") << ro.off
                            << "ull + ((size_t)bz * " << ro.parts << "u + tile_m) * GN + n0 + c" << (fold_in_kernel ? ", r);" : "] = r;") << "\n}\n";
                     ci++;
                 } else {
                     const int64_t per_b = ro.parts / o.b_div;  // partials per batch index: one per tile
-                    finish << "if (tid == 0) {\nfloat r = 0.0f;\n#pragma unroll\nfor (int w = 0; w < WAVES_M * WAVES_N; w++) r += red["
-                           << ncol * t.wm * t.bn + si * t.wm * t.wn << " + w];\n" << (fold_in_kernel ? "HE_WS_STORE(red_ws + " : "red_ws[") << ro.off
+                    finish << "if (threadIdx.x == 0) {\nfloat r = 0.0f;\n#pragma unroll\nfor (int w = 0; w < ALL_WAVES; w++) r += red["
+                           << ncol * rows_of * t.bn + si * rows_of * t.wn << " + w];\n" << (fold_in_kernel ? "HE_WS_STORE(red_ws + " : "red_ws[") << ro.off
                            << "ull + (size_t)(bz / " << o.b_div << "u) * " << ro.parts << "u + (size_t)(bz % " << o.b_div << "u) * " << per_b << "u + tile_m * "
                            << tiles_n << "u + tile_n" << (fold_in_kernel ? ", r);" : "] = r;") << "\n}\n";
                     si++;
@@ -1421,7 +1505,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                 // every partial of this workgroup has left the CU before its tickets are taken; whoever takes the last
                 // ticket of a counter finds all partials in memory, adds them in tile order, and leaves the counter at
                 // zero for the next launch
-                finish << "HE_WS_DRAIN();\n__syncthreads();\n__shared__ u32 red_last[2];\nif (tid == 0) {\n"
+                finish << "HE_WS_DRAIN();\n__syncthreads();\n__shared__ u32 red_last[2];\nif (threadIdx.x == 0) {\n"
                        << "u32* c0 = red_cnt + (size_t)bz * " << tiles_n << "u + tile_n;\nconst bool l0 = HE_WS_TICKET(c0) == " << tiles_m - 1 << "u;\nif (l0) HE_WS_STORE(c0, 0u);\nred_last[0] = l0;\n";
                 if (nsc) {
                     // (scalar outputs of one kernel share b_div: one counter per element group)
@@ -1441,14 +1525,14 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                     char scale[64];
                     snprintf(scale, sizeof scale, "%.9ef", o.rop == tp::ROp::Mean ? (float)o.mean_scale : 1.0f);
                     if (!o.fold_n) {
-                        finish << "if (red_last[0]) {\nfor (u32 c = tid; c < BN; c += NTHREADS) {\nif (n0 + c < GN) {\nfloat r = 0.0f;\n#pragma unroll 8\nfor (u32 p = 0; p < "
+                        finish << "if (red_last[0]) {\nfor (u32 c = threadIdx.x; c < BN; c += ALL_THREADS) {\nif (n0 + c < GN) {\nfloat r = 0.0f;\n#pragma unroll 8\nfor (u32 p = 0; p < "
                                << ro.parts << "u; p++) r += HE_WS_LOAD(red_ws + " << ro.off << "ull + ((size_t)bz * " << ro.parts << "u + p) * GN + n0 + c);\na"
                                << o.arg << "[(size_t)bz * GN + n0 + c] = r * " << scale << ";\n}\n}\n}\n";
                     } else {
                         // one thread per partial (at most 4096), then the waves' sums in order
-                        finish << "if (red_last[1]) {\nfloat r = 0.0f;\nfor (u32 p = tid; p < " << ro.parts << "u; p += NTHREADS) r += HE_WS_LOAD(red_ws + " << ro.off
-                               << "ull + (size_t)(bz / " << o.b_div << "u) * " << ro.parts << "u + p);\nr = wave_reduce<0, 64>(r);\n__syncthreads();\nif (lane == 0) red[wave] = r;\n__syncthreads();\n"
-                               << "if (tid == 0) {\nfloat total = 0.0f;\nfor (int w = 0; w < WAVES_M * WAVES_N; w++) total += red[w];\na" << o.arg << "[bz / " << o.b_div
+                        finish << "if (red_last[1]) {\nfloat r = 0.0f;\nfor (u32 p = threadIdx.x; p < " << ro.parts << "u; p += ALL_THREADS) r += HE_WS_LOAD(red_ws + " << ro.off
+                               << "ull + (size_t)(bz / " << o.b_div << "u) * " << ro.parts << "u + p);\nr = wave_reduce<0, 64>(r);\n__syncthreads();\nif (lane == 0) red[kgroup * NWAVES + wave] = r;\n__syncthreads();\n"
+                               << "if (threadIdx.x == 0) {\nfloat total = 0.0f;\nfor (int w = 0; w < ALL_WAVES; w++) total += red[w];\na" << o.arg << "[bz / " << o.b_div
                                << "u] = total * " << scale << ";\n}\n}\n";
                     }
                 }
@@ -1669,14 +1753,14 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     HE_REQUIRE(tiles < (1ll << 31) && pr.batch < 65536, HE_ERR_INVALID, "GEMM grid too large");
     grid_[0] = (uint32_t)tiles;
     grid_[1] = (uint32_t)(pr.split_k > 1 ? pr.split_k : pr.batch);
-    threads_ = (uint32_t)threads;
+    threads_ = (uint32_t)(threads * t.wk);
     for (auto& r : reds) reduce_outs_.push_back(pr.map_e[pr.epi.outs[r.out].arg]);
     reduce_floats_ = red_floats;
     std::string reduce_args;
     for (int a : reduce_all_args_ ? pr.map_e : reduce_outs_) reduce_args += (reduce_args.empty() ? "" : ",") + std::to_string(a);
-    describe_ = strfmt("gemm [%lld,%lld,%lld]x[%lld] tile=%dx%dx%d stages=%d waves=%dx%d threads=%d grid=%ux%u rawA=%d rawB=%d NVA=%d NVB=%d NVE=%d "
+    describe_ = strfmt("gemm [%lld,%lld,%lld]x[%lld] tile=%dx%dx%d stages=%d waves=%dx%d threads=%d k_groups=%d grid=%ux%u rawA=%d rawB=%d NVA=%d NVB=%d NVE=%d "
                        "direct=%d%d mma=%s epilogue_exprs=%zu outs=%zu split_k=%d reduce_ws=%llu reduce_grid=%u reduce_args=[%s] reduce_counters=%llu",
-                       (long long)pr.batch, (long long)pr.M, (long long)pr.K, (long long)pr.N, t.bm, t.bn, t.bk, t.stages, t.wm, t.wn, threads,
+                       (long long)pr.batch, (long long)pr.M, (long long)pr.K, (long long)pr.N, t.bm, t.bn, t.bk, t.stages, t.wm, t.wn, threads * t.wk, t.wk,
                        grid_[0], grid_[1], (int)raw_a, (int)raw_b, nva, nvb, nve, (int)direct_a, (int)direct_b, dtype_name(pr.mma_dtype), pr.epi.exprs.size(),
                        pr.epi.outs.size(), pr.split_k, (unsigned long long)reduce_floats_, reduce_grid_, reduce_args.c_str(), (unsigned long long)reduce_counters_);
     kernel_.reset(new JitKernel(source_, "fused_matmul", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));

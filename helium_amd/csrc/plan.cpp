@@ -1141,9 +1141,13 @@ int filter_gradient_split_k(const GemmProblem& pr, bool element_gather) {
     //    (5 tiles x 50 shares against 9 x 56 of 128x128), at batch 64 45.8 -> 43.6, the stride-2 56x56x64 -> 128 layer 50.8 -> 44.5;
     //  - 512 output channels keep 256x256 tiles, whose count, not that of 128x128 tiles, decides the shares as long as a
     //    share keeps 12 k-tiles: the 7x7x512 layer 36 x 4 = 144 workgroups 77.4 us, 36 x 7 = 252 workgroups 70.3.
+    //  - a short k (few pixels) and 32x32 tiles for every CU at most: the waves of a workgroup share the k range, and there are
+    //    no partial tiles to add up (gemm.cpp: small_tile).
+    const bool wide128 = !element_gather && pr.M > 64 && pr.M <= 128 && pr.N >= 512;
+    if (!wide128 && !element_gather && ((pr.M + 31) / 32) * ((pr.N + 31) / 32) <= 256 && k_tiles <= 96) return 1;
     if (tuning::get("HELIUM_HIP_GEMM_NO_WIDE_CONV_TILES")) {
         // (the shares as they were, for comparison)
-    } else if (!element_gather && pr.M > 64 && pr.M <= 128 && pr.N >= 512) {
+    } else if (wide128) {
         const int64_t wide = (pr.N + 255) / 256;
         split = (int)std::max<int64_t>(1, std::min<int64_t>({256 / wide, k_tiles / 4, 1024}));
     } else if (!element_gather && pr.M >= 512 && pr.N >= 512) {

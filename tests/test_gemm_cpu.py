@@ -171,6 +171,31 @@ def test_ragged_products_on_cpu(name, build, tile):
     compare(got, want, **(dict(rel=1e-4, eps=1e-5) if f32 else {}))
 
 
+# Waves that share a tile's k range: group counts that do not divide the k-tiles, groups without a tile, groups of several
+# waves, operands through registers and by direct loads, every kind of reduction over the groups' shares of the rows.
+K_GROUPS = [
+    ("nn_odd_four_groups", lambda: gemm_cases.plain(97, 131, 467), "32,32,64,1,1,2,4"),
+    ("nn_direct_three_stages", lambda: gemm_cases.plain(64, 72, 456), "32,32,64,1,1,3,4"),
+    ("reductions_eight_groups", lambda: gemm_cases.all_reductions(70, 72, 300), "32,32,64,1,1,2,8"),
+    ("mainloop_two_groups_of_four_waves", lambda: gemm_cases.bias_relu_colsum(67, 77, 175, mainloop=True), "64,64,64,2,2,2,2"),
+    ("direct_two_groups_of_four_waves", lambda: gemm_cases.plain(128, 128, 320), "64,64,64,2,2,2,2"),
+    ("f32_linear_layer_one_k_tile", lambda: gemm_cases.linear_layer(48, 40, 72), "32,32,32,1,1,4,4"),
+    ("f32_eight_groups_one_k_tile", lambda: gemm_cases.plain(37, 67, 10, dtype="f32"), "32,32,32,1,1,2,8"),
+    ("tt_64x32_waves", lambda: gemm_cases.transposed_a(67, 101, 275, both=True), "64,32,64,1,1,2,4"),
+    ("nt_64x64_waves", lambda: gemm_cases.transposed_b(70, 99, 1160), "64,64,64,1,1,2,4"),
+]
+
+
+@pytest.mark.parametrize("name,build,tile", K_GROUPS, ids=[c[0] for c in K_GROUPS])
+def test_products_with_k_groups_on_cpu(name, build, tile):
+    g, inputs, outs = build()
+    k, got = run_emulated(g, inputs, tile)
+    assert "k_groups=" + tile.split(",")[-1] in k.description and sorted(got) == sorted(outs)
+    f32 = name.startswith("f32")
+    want = oracle.outputs(g.nodes, inputs, round_mainloop_to=None if f32 else "bf16")
+    compare(got, want, **(dict(rel=1e-4, eps=1e-5) if f32 else {}))
+
+
 def test_argument_order_is_producers_then_leaves():
     g, inputs, outs = gemm_cases.bias_relu_colsum(64, 64, 64, mainloop=True)
     k = ha.TileKernel.fused(g)
