@@ -10,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libhelium_hip.so")
+COMPILER = os.path.join(HERE, "helium_rtc")  # the kernel compiler that the library runs as a child process
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 
 
@@ -46,6 +47,12 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(link), flush=True)
     subprocess.check_call(link)
+    # (an old-style run path comes before the environment's: the compiler of this toolchain, whatever else is on the path)
+    tool = [hipcc, "-x", "c++", *flags, os.path.join(CSRC, "compiler", "main.cpp"), "-o", COMPILER, f"-L{ROCM}/lib", "-lhiprtc",
+            f"-Wl,-rpath,{ROCM}/lib", "-Wl,--disable-new-dtags"]
+    if verbose:
+        print(" ".join(tool), flush=True)
+    subprocess.check_call(tool)
     return LIB
 
 

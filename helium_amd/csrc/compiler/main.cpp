@@ -1,0 +1,42 @@
+// The kernel compiler as a process of its own: source text on stdin, `name option...` as arguments, the code object on
+// stdout behind one status byte ('o': code object, 'e': the compiler's log). rtc.cpp says why it is not called in-process.
+#include <hip/hiprtc.h>
+#include <unistd.h>
+
+#include <string>
+#include <vector>
+
+static int answer(char status, const char* data, size_t bytes) {
+    std::string out(1, status);
+    out.append(data, bytes);
+    for (size_t done = 0; done < out.size();) {
+        const ssize_t n = write(1, out.data() + done, out.size() - done);
+        if (n <= 0) return 2;
+        done += (size_t)n;
+    }
+    return 0;
+}
+static int refuse(const std::string& why) { return answer('e', why.data(), why.size()); }
+
+int main(int argc, char** argv) {
+    if (argc < 2) return 2;
+    std::string source;
+    char buf[1 << 16];
+    for (ssize_t n; (n = read(0, buf, sizeof buf)) > 0;) source.append(buf, (size_t)n);
+    hiprtcProgram prog;
+    hiprtcResult r = hiprtcCreateProgram(&prog, source.c_str(), (std::string(argv[1]) + ".hip").c_str(), 0, nullptr, nullptr);
+    if (r != HIPRTC_SUCCESS) return refuse(std::string("hiprtcCreateProgram: ") + hiprtcGetErrorString(r));
+    std::vector<const char*> options(argv + 2, argv + argc);
+    r = hiprtcCompileProgram(prog, (int)options.size(), options.data());
+    size_t n = 0;
+    if (r != HIPRTC_SUCCESS) {
+        hiprtcGetProgramLogSize(prog, &n);
+        std::string log(n, '\0');
+        if (n) hiprtcGetProgramLog(prog, &log[0]);
+        return refuse(std::string(hiprtcGetErrorString(r)) + "\n" + log);
+    }
+    if (hiprtcGetCodeSize(prog, &n) != HIPRTC_SUCCESS || n == 0) return refuse("no code object");
+    std::string code(n, '\0');
+    if ((r = hiprtcGetCode(prog, &code[0])) != HIPRTC_SUCCESS) return refuse(std::string("hiprtcGetCode: ") + hiprtcGetErrorString(r));
+    return answer('o', code.data(), code.size());
+}

@@ -56,3 +56,23 @@ def test_cache_can_be_switched_off(tmp_path):
     out = subprocess.run([sys.executable, "-c", CHILD], env=env, capture_output=True, text=True, timeout=300, cwd=tmp_path)
     assert out.returncode == 0, out.stderr
     assert out.stdout.split()[:2] == ["1", "0"] and not os.listdir(tmp_path)
+
+
+def test_the_compiler_does_not_depend_on_what_the_program_imported_first(tmp_path):
+    """torch carries a HIP compiler of its own; kernels come from the toolchain's all the same."""
+    made = []
+    for first in ("", "import torch\n"):
+        d = tmp_path / ("with" if first else "without")
+        out = subprocess.run([sys.executable, "-c", first + CHILD], env=dict(os.environ, HELIUM_HIP_CACHE_DIR=str(d)), capture_output=True,
+                             text=True, timeout=300)
+        assert out.returncode == 0, out.stderr
+        made.append({f: open(os.path.join(d, f), "rb").read() for f in os.listdir(d)})
+    assert len(made[0]) == 1 and made[0] == made[1]
+
+
+def test_what_the_compiler_has_against_a_source_reaches_the_caller():
+    code = ("import sys; sys.path.insert(0, %r)\nfrom helium_amd import device\n"
+            "try:\n    device.rtc_compile('extern \"C\" __global__ void broken() { no_such_name(); }', 'broken')\n"
+            "except Exception as e:\n    print(e)\n" % ROOT)
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, HELIUM_HIP_CACHE_DIR="off"), capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0 and "broken" in out.stdout and "no_such_name" in out.stdout, out.stdout + out.stderr
