@@ -102,13 +102,11 @@ int he_plan_instruction_kernel(he_plan_t plan, int index, he_tile_kernel_t* kern
 int he_plan_precompile(he_plan_t plan) {
     return he::guard([&] {
         HE_REQUIRE(plan, HE_ERR_INVALID, "bad argument");
-        {
-            // the kernels the executor would run: its assignment of instructions to streams shapes some of them
-            he::exec::Prepared as_executed;
-            as_executed.graph = plan->graph;
-            as_executed.plan = plan->plan;
-            he::exec::assign_streams(&as_executed);
-        }
+        // the kernels the executor would run: its assignment of instructions to streams shapes some of them, and joins others
+        he::exec::Prepared as_executed;
+        as_executed.graph = plan->graph;
+        as_executed.plan = plan->plan;
+        he::exec::assign_streams(&as_executed);
         std::vector<std::future<void>> jobs;
         for (auto& step : plan->plan->steps)
             for (auto& instr : step.instrs)
@@ -121,6 +119,7 @@ int he_plan_precompile(he_plan_t plan) {
                         }
                     }));
         for (auto& j : jobs) j.get();
+        he::exec::build_schedule(&as_executed);
     });
 }
 int he_plan_destroy(he_plan_t plan) {
@@ -132,7 +131,8 @@ int he_execute_graph(he_graph_t graph, const uint32_t* input_nodes, const he_ten
                      uint32_t* output_nodes, he_tensor_t* output_tensors, int max_outputs, int* num_outputs) {
     return he::guard([&] {
         HE_REQUIRE(graph && num_outputs && (num_inputs == 0 || (input_nodes && input_tensors)), HE_ERR_INVALID, "bad argument");
-        std::map<he::ir::NodeId, he::exec::TensorRef> inputs;
+        he::exec::NamedTensors inputs;
+        inputs.reserve((size_t)num_inputs);
         for (int i = 0; i < num_inputs; i++) {
             HE_REQUIRE(input_tensors[i], HE_ERR_INVALID, "null input tensor %d", i);
             const he::ir::Node& n = graph->g->get(input_nodes[i]);
@@ -140,7 +140,7 @@ int he_execute_graph(he_graph_t graph, const uint32_t* input_nodes, const he_ten
             const he::exec::Tensor& t = *input_tensors[i]->t;
             HE_REQUIRE(t.dtype == n.desc.dtype && (int64_t)t.len == he::ir::num_elements(n.desc.shape), HE_ERR_INVALID,
                        "tensor for input node %u does not match its descriptor", input_nodes[i]);
-            inputs[input_nodes[i]] = input_tensors[i]->t;
+            inputs.emplace_back(input_nodes[i], input_tensors[i]->t);
         }
         // the optimised copy of the graph and its plan are made on the first call and kept with the handle
         std::shared_ptr<const he::exec::Prepared> prepared;

@@ -694,6 +694,7 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
     for (int d = 0; d < n; d++) s << (d ? "," : "") << p.dims[d];
     s << "] NV=" << NV << " TX=" << TX << " TY=" << TY << " RPT=" << RPT << "\n";
     s << kPrelude;
+    L.prelude_bytes = (size_t)s.tellp();
     s << "#define NV " << NV << "\n#define TX " << TX << "\n#define TY " << TY << "\n#define RPT " << RPT
       << "\n#define TR " << TR << "\n#define DIM_N " << N << "u\n#define DIM_M " << M << "u\n";
     s << "extern \"C\" __global__ __launch_bounds__(" << threads << ") void " << entry << "(";

@@ -111,9 +111,10 @@ void DevicePool::note_use(Tensor& t, uint64_t scope) {
     note_locked(t, scope);
 }
 
-void DevicePool::note_uses(const std::map<ir::NodeId, TensorRef>& tensors, uint64_t scope) {
+void DevicePool::note_uses(const std::vector<TensorRef>& tensors, uint64_t scope) {
     std::lock_guard<std::mutex> lk(mu_);
-    for (auto& kv : tensors) note_locked(*kv.second, scope);
+    for (auto& t : tensors)
+        if (t) note_locked(*t, scope);
 }
 
 Allocation DevicePool::allocate(size_t bytes, uint64_t scope) {
@@ -252,6 +253,7 @@ TensorRef create_tensor_with_data(const void* data, int dtype, size_t len) {
     }
     t->uploaded = true;
     t->ready = DevicePool::global().take_event();
+    t->ready->on = st.h2d;
     HE_HIP(hipEventRecord(t->ready->e, st.h2d));
     return t;
 }
@@ -281,8 +283,14 @@ struct HostTimer {
         acc[i] += std::chrono::duration<double, std::micro>(n - t).count();
         t = n;
     }
-    void restart() {
-        if (on()) t = std::chrono::steady_clock::now();
+    void report() {
+        if (!on()) return;
+        static thread_local double sum[8] = {0};
+        static thread_local int calls = 0;
+        for (int i = 0; i < 8; i++) sum[i] += acc[i];
+        if (++calls % 100 != 0) return;
+        fprintf(stderr, "[exec timing] per graph, us: setup %.1f, storage %.1f, launches %.1f, finish %.1f\n", sum[2] / 100, sum[3] / 100, sum[4] / 100, sum[5] / 100);
+        for (double& v : sum) v = 0;
     }
 };
 // Join events of an execution are destroyed one execution later on the same thread: by then they were recorded and
@@ -292,8 +300,6 @@ void retire_join_events(const std::vector<hipEvent_t>& events) {
     for (hipEvent_t e : garbage) (void)hipEventDestroy(e);
     garbage = events;
 }
-thread_local double g_host_acc[8] = {0};
-thread_local int g_host_calls = 0;
 std::atomic<int> g_fan_out{1};
 
 // Whether the independent instructions of a step are worth a stream each. Putting work on a second stream costs a
@@ -478,6 +484,10 @@ std::shared_ptr<const Prepared> prepare(const ir::OpGraph& graph_in) {
         for (auto& instr : step.instrs)
             if (!instr->compiled()) jobs.push_back(std::async(std::launch::async, [instr] { instr->precompile(); }));
     for (auto& j : jobs) j.get();
+    build_schedule(pr.get());
+    if (getenv("HELIUM_HIP_PLAN_DEBUG") && pr->schedule)
+        fprintf(stderr, "[plan] schedule: %d instructions, %zu launches, %.1f MB of intermediate values\n", pr->schedule->instrs, pr->schedule->launches.size(),
+                pr->schedule->arena_bytes / 1e6);
     if (getenv("HELIUM_HIP_PLAN_DEBUG")) {
         size_t fanned = 0, multi = 0;
         for (size_t k = 0; k < pr->plan->steps.size(); k++) {
@@ -489,22 +499,206 @@ std::shared_ptr<const Prepared> prepare(const ir::OpGraph& graph_in) {
     return pr;
 }
 
-std::map<NodeId, TensorRef> execute_graph(const ir::OpGraph& graph_in, const std::map<NodeId, TensorRef>& inputs,
-                                          ExecStats* stats) {
-    return execute_prepared(*prepare(graph_in), inputs, stats);
+namespace {
+// The thread's streams wait for a tensor that something outside this execution fills (an upload, another thread's graph).
+void wait_for_tensor(const Tensor& t, hipStream_t stream, hipStream_t main, ExecStats* stats) {
+    // (what the main stream recorded is ahead of this execution on both of its streams)
+    if (!t.ready || t.ready->on == main || t.ready_seen.load(std::memory_order_acquire)) return;
+    // a producer seen finished once stays finished: no wait is queued for it again
+    if (hipEventQuery(t.ready->e) == hipSuccess) {
+        const_cast<Tensor&>(t).ready_seen.store(true, std::memory_order_release);
+        return;
+    }
+    HE_HIP(hipStreamWaitEvent(stream, t.ready->e, 0));
+    stats->event_waits++;
 }
 
-std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std::map<NodeId, TensorRef>& caller_inputs,
-                                             ExecStats* stats) {
-    HostTimer ht;
-    // the ids of a rewritten graph differ from the caller's: inputs are renamed on the way in, outputs on the way out
-    std::map<NodeId, TensorRef> renamed;
-    if (!prepared.input_of.empty())
-        for (auto& kv : caller_inputs) {
-            auto it = prepared.input_of.find(kv.first);
-            if (it != prepared.input_of.end()) renamed[it->second] = kv.second;
+// HELIUM_HIP_INSTR_TIMING=<n>: every launch is timed on its own (the device is drained before and after it), and the n
+// slowest of the second execution are listed with the bytes they read and write. A debugging aid: it serialises.
+struct LaunchTimes {
+    static int wanted() {
+        static const int n = getenv("HELIUM_HIP_INSTR_TIMING") ? atoi(getenv("HELIUM_HIP_INSTR_TIMING")) : 0;
+        return n;
+    }
+    struct Time {
+        double us;
+        size_t launch;
+    };
+    std::vector<Time> times;
+    std::chrono::steady_clock::time_point t0;
+    void start() {
+        HE_HIP(hipDeviceSynchronize());
+        t0 = std::chrono::steady_clock::now();
+    }
+    void stop(size_t launch) {
+        HE_HIP(hipDeviceSynchronize());
+        times.push_back({std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t0).count(), launch});
+    }
+    void report(const Schedule& S) {
+        static std::atomic<int> reports{0};
+        if (times.empty() || reports.fetch_add(1) != 1) return;  // the second execution: kernels are compiled and loaded by then
+        std::sort(times.begin(), times.end(), [](const Time& a, const Time& b) { return a.us > b.us; });
+        double total = 0;
+        for (auto& t : times) total += t.us;
+        fprintf(stderr, "[instr timing] %zu launches, %.1f us in all; slowest:\n", times.size(), total);
+        for (int i = 0; i < wanted() && i < (int)times.size(); i++) {
+            const Schedule::Launch& L = S.launches[times[i].launch];
+            int64_t bytes = 0;
+            for (uint32_t a : L.args) bytes += (int64_t)S.slots[a].bytes;
+            fprintf(stderr, "  #%-4zu %8.1f us %8.1f MB %6.2f TB/s  %s\n", times[i].launch, times[i].us, bytes / 1e6, bytes / times[i].us / 1e6,
+                    L.kernel ? L.kernel->describe().substr(0, 320).c_str() : "permute");
         }
-    const std::map<NodeId, TensorRef>& inputs = prepared.input_of.empty() ? caller_inputs : renamed;
+    }
+};
+
+NamedTensors execute_scheduled(const Prepared& prepared, const NamedTensors& inputs, bool one_stream, ExecStats* stats) {
+    HostTimer ht;
+    const Schedule& S = *prepared.schedule;
+    DevicePool& pool = DevicePool::global();
+    Streams& st = thread_streams();
+    const hipStream_t main = st.s[0];
+    const bool use_side = S.uses_side && !one_stream && st.s.size() >= 2 && !LaunchTimes::wanted();
+    static const bool launch_events = getenv("HELIUM_HIP_NO_LAUNCH_EVENTS") == nullptr;
+    ExecStats local;
+    std::vector<TensorRef> tensors(S.slots.size());  // the caller's and the results
+    for (auto& in : inputs) {
+        auto it = std::lower_bound(S.inputs.begin(), S.inputs.end(), in.first, [](const Schedule::Named& a, NodeId n) { return a.node < n; });
+        if (it != S.inputs.end() && it->node == in.first) tensors[it->slot] = in.second;
+    }
+    for (auto& in : S.inputs) HE_REQUIRE(tensors[in.slot], HE_ERR_INVALID, "missing storage for input node %u", in.node);
+    EventRef done = pool.take_event();
+    done->on = main;
+    const uint64_t scope = pool.begin_scope((uint64_t)(uintptr_t)&st);
+    bool done_recorded = false, side_used = false, side_joined = false;
+    std::vector<EventRef> events;  // of this execution, given back when it has been queued
+    auto record = [&](hipStream_t on) {
+        events.push_back(pool.take_event());
+        HE_HIP(hipEventRecord(events.back()->e, on));
+        return events.back()->e;
+    };
+    auto join_side = [&] {
+        if (!side_used || side_joined) return;
+        HE_HIP(hipStreamWaitEvent(main, record(st.s[1]), 0));
+        local.event_waits++;
+        side_joined = true;
+    };
+    std::vector<TensorRef> blocks;
+    try {
+        pool.note_uses(tensors, scope);
+        ht.lap(2);
+        std::vector<void*> at(S.slots.size(), nullptr);
+        char* arena = nullptr;
+        if (S.arena_bytes) {
+            blocks.push_back(allocate_tensor(HE_U32, (size_t)(S.arena_bytes / 4), scope));
+            arena = (char*)blocks.back()->ptr;
+        }
+        for (size_t i = 0; i < S.slots.size(); i++) {
+            const Schedule::Slot& s = S.slots[i];
+            if (s.where == Schedule::Slot::Result) tensors[i] = allocate_tensor(s.dtype, s.len, scope);
+            at[i] = s.where == Schedule::Slot::Arena ? arena + s.offset : tensors[i]->ptr;
+        }
+        ht.lap(3);
+        hipEvent_t main_end = nullptr, early_end = nullptr;  // what the next wait of the other stream is for
+        std::vector<void*> ptrs;
+        LaunchTimes timing;
+        for (size_t i = 0; i < S.launches.size(); i++) {
+            const Schedule::Launch& L = S.launches[i];
+            const bool on_side = use_side && L.stream == 1;
+            const hipStream_t stream = on_side ? st.s[1] : main;
+            if (on_side) {
+                // the side stream's first work of this execution comes after the end of the thread's previous one
+                if (!side_used && st.has_run) HE_HIP(hipStreamWaitEvent(stream, st.exec_end->e, 0));
+                side_used = true;
+                if (L.waits_for_main) {
+                    HE_HIP(hipStreamWaitEvent(stream, main_end, 0));
+                    local.event_waits++;
+                }
+            } else if (use_side && L.waits_for_early) {
+                HE_HIP(hipStreamWaitEvent(stream, early_end, 0));
+                local.event_waits++;
+            }
+            for (uint32_t in : L.new_inputs) wait_for_tensor(*tensors[in], stream, main, &local);
+            const bool closes = L.closes && launch_events;
+            if (closes) {
+                join_side();
+                set_pending_stop_event(done->e);
+            } else if (use_side && L.marks_end && launch_events) {
+                events.push_back(pool.take_event());
+                main_end = events.back()->e;
+                set_pending_stop_event(main_end);
+            }
+            ptrs.resize(L.args.size());
+            for (size_t a = 0; a < L.args.size(); a++) ptrs[a] = at[L.args[a]];
+            if (LaunchTimes::wanted()) timing.start();
+            try {
+                if (L.kernel) L.kernel->execute(ptrs.data(), stream);
+                else L.permute->execute(ptrs[0], ptrs[1], stream);
+            } catch (...) {
+                (void)take_pending_stop_event();
+                throw;
+            }
+            if (LaunchTimes::wanted()) timing.stop(i);
+            // (still pending: a launch too large for the entry point that takes an event)
+            const bool taken = take_pending_stop_event() == nullptr;
+            if (closes) done_recorded = taken;
+            else if (use_side && L.marks_end && !(taken && launch_events)) main_end = record(stream);
+            if (use_side && i + 1 == S.early_launches) early_end = record(stream);
+        }
+        ht.lap(4);
+        join_side();
+        // Drop of the executor (cuda.rs:232-260): when everything queued above has run, the scope's freed blocks become available
+        // to everyone. The main stream carries the event the pool polls.
+        if (!done_recorded) HE_HIP(hipEventRecord(done->e, main));
+        timing.report(S);
+    } catch (...) {
+        // The scope must end, and only after the work already queued.
+        try {
+            side_joined = false;
+            join_side();
+            HE_HIP(hipEventRecord(done->e, main));
+            st.exec_end = done;
+            st.has_run = true;
+            pool.end_scope_after(scope, done);
+        } catch (...) {
+            (void)hipDeviceSynchronize();
+            pool.end_scope(scope);
+        }
+        throw;
+    }
+    // The same event orders this thread's next execution after this one, and it is the ready event of every tensor the caller
+    // gets (enumerate_output_tensors, cuda.rs:142-153, records one per tensor).
+    for (size_t i = 0; i < S.slots.size(); i++)
+        if (S.slots[i].where == Schedule::Slot::Result) tensors[i]->ready = done;
+    st.exec_end = done;
+    st.has_run = true;
+    pool.end_scope_after(scope, std::move(done));
+    local.steps = S.steps;
+    local.instrs = S.instrs;
+    local.streams_used = side_used ? 2 : 1;
+    if (stats) *stats = local;
+    NamedTensors result;
+    result.reserve(S.outputs.size());
+    for (auto& o : S.outputs) result.emplace_back(o.node, tensors[o.slot]);
+    ht.lap(5);
+    ht.report();
+    return result;
+}
+}  // namespace
+
+NamedTensors execute_prepared(const Prepared& prepared, const NamedTensors& named_inputs, ExecStats* stats) {
+    const int fan_mode = g_fan_out.load();
+    if (prepared.schedule && fan_mode != 2) return execute_scheduled(prepared, named_inputs, fan_mode == 0, stats);
+    // Step by step, the instructions of a step over the thread's streams.
+    // The ids of a rewritten graph differ from the caller's: inputs are renamed on the way in, outputs on the way out
+    std::map<NodeId, TensorRef> inputs;
+    for (auto& kv : named_inputs) {
+        if (prepared.input_of.empty()) {
+            inputs[kv.first] = kv.second;
+            continue;
+        }
+        auto it = prepared.input_of.find(kv.first);
+        if (it != prepared.input_of.end()) inputs[it->second] = kv.second;
+    }
     const std::shared_ptr<const ir::OpGraph>& graph = prepared.graph;
     const std::shared_ptr<const plan::Plan>& plan = prepared.plan;
     const std::set<NodeId>& alive = prepared.alive;
@@ -514,8 +708,11 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
         HE_REQUIRE(inputs.count(in), HE_ERR_INVALID, "missing storage for input node %u", in);
     const uint64_t scope = pool.begin_scope((uint64_t)(uintptr_t)&st);
     std::map<NodeId, TensorRef> tensors = inputs;
-    pool.note_uses(tensors, scope);
-    ht.lap(2);
+    {
+        std::vector<TensorRef> held;
+        for (auto& kv : inputs) held.push_back(kv.second);
+        pool.note_uses(held, scope);
+    }
     ExecStats local;
     std::set<const Tensor*> synced;        // input tensors whose ready event a stream already waited on
     std::vector<size_t> prev_streams;      // streams the previous step ran on
@@ -542,7 +739,6 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
     };
     // An execution whose steps hold one instruction each runs on stream 0 alone: its last launch can carry the
     // execution's event itself.
-    const int fan_mode = g_fan_out.load();
     auto step_width = [&](size_t k) {
         const plan::Step& step = plan->steps[k];
         const bool fan = !step.in_order && (fan_mode == 2 || (fan_mode == 1 && prepared.fan_out[k]));
@@ -559,32 +755,12 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
         }
         if (!one_stream || getenv("HELIUM_HIP_NO_LAUNCH_EVENTS")) closing = nullptr;
     }
-    // The side stream (side_stream_split): stream 1 runs the chains that nothing on the main stream waits for.
-    const Prepared::Side& S = prepared.side;
-    const bool side_mode = fan_mode == 1 && !S.side.empty() && st.s.size() >= 2;
-    // (the end event follows the join of the two streams: the last launch carries it only if it runs on the main stream)
-    if (side_mode && (getenv("HELIUM_HIP_NO_LAUNCH_EVENTS") || S.side.back())) closing = nullptr;
-    if (side_mode && !getenv("HELIUM_HIP_NO_LAUNCH_EVENTS") && !S.side.back()) closing = S.order.back();
-    std::vector<uint8_t> issued(side_mode ? S.order.size() : 0, 0);
-    std::vector<TensorRef> held;           // what side instructions touch stays allocated until the streams have joined
-    std::set<const Tensor*> synced_side;   // input tensors whose ready event the side stream waited on
-    bool main_dirty = false;               // the main stream has taken work since the side stream last waited for it
-    bool side_joined = false;              // the main stream has waited for the end of the side stream's work
-    std::vector<EventRef> launch_events;   // completion events of main-stream launches that a side instruction follows
-    bool main_end_known = false;           // ... and whether the last of them marks the main stream's latest launch
     EventRef done = pool.take_event();
+    done->on = st.s[0];
     bool done_recorded = false;
-    struct InstrTime {
-        double us;
-        int64_t bytes;
-        const plan::Instr* instr;
-        size_t order;  // position in the execution
-    };
-    std::vector<InstrTime> instr_times;
-    static const int instr_timing = getenv("HELIUM_HIP_INSTR_TIMING") ? atoi(getenv("HELIUM_HIP_INSTR_TIMING")) : 0;
     // One instruction on stream `w` of the thread's pool: storage for what it writes, waits for inputs made outside
     // this execution, its launches.
-    auto run_instr = [&](const plan::Instr& instr, size_t w, bool on_side, std::vector<const Tensor*>& waited) {
+    auto run_instr = [&](const plan::Instr& instr, size_t w, std::vector<const Tensor*>& waited) {
         hipStream_t stream = st.s[w];
         // a stream's first work of this execution comes after the end of the thread's previous execution
         // (stream 0 carried that end itself)
@@ -599,9 +775,8 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
         for (NodeId in : instr.all_inputs()) {
             auto it = tensors.find(in);
             HE_REQUIRE(it != tensors.end(), HE_ERR_INTERNAL, "missing storage for node %u", in);
-            // tensors made outside this execution carry a ready event (uploads, earlier graphs); a wait of the main
-            // stream also covers the side stream, which waits for the main stream before every instruction it takes
-            if (inputs.count(in) && !synced.count(it->second.get()) && !(on_side && synced_side.count(it->second.get()))) {
+            // tensors made outside this execution carry a ready event (uploads, earlier graphs)
+            if (inputs.count(in) && !synced.count(it->second.get())) {
                 Tensor& t = *it->second;
                 // a producer seen finished once stays finished: no wait is queued for it again
                 if (t.ready && !t.ready_seen.load(std::memory_order_acquire)) {
@@ -617,85 +792,21 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
                 waited.push_back(it->second.get());
             }
         }
-        ht.lap(3);
         if (&instr == closing) set_pending_stop_event(done->e);
-        // HELIUM_HIP_INSTR_TIMING=<n>: every instruction is timed on its own (the device is drained before and after
-        // it), and the n slowest of the execution are listed with the bytes they read and write. A debugging aid:
-        // the execution is serialised while it is on.
-        std::chrono::steady_clock::time_point t_instr;
-        if (instr_timing) {
-            HE_HIP(hipDeviceSynchronize());
-            t_instr = std::chrono::steady_clock::now();
-        }
         try {
             instr.execute([&](NodeId n) -> void* { return tensors.at(n)->ptr; }, stream);
         } catch (...) {
             (void)take_pending_stop_event();
             throw;
         }
-        if (instr_timing) {
-            HE_HIP(hipDeviceSynchronize());
-            const double us = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - t_instr).count();
-            int64_t bytes = 0;
-            for (NodeId n : instr.all_inputs()) bytes += (int64_t)tensors.at(n)->bytes;
-            for (NodeId n : instr.all_outputs()) bytes += (int64_t)tensors.at(n)->bytes;
-            instr_times.push_back({us, bytes, &instr, instr_times.size()});
-        }
         // taken by the instruction's last launch, or still pending (a launch too large for that entry point)
         if (&instr == closing) done_recorded = take_pending_stop_event() == nullptr;
-        ht.lap(4);
         local.instrs++;
-    };
-    // A side instruction waits for everything the main stream has taken so far: for the results it reads, and because
-    // the blocks it is given may have been freed by the main stream just now. What it touches is held until the
-    // streams join, so the main stream is never handed a block the side stream still uses. The side instructions that
-    // read its results alone follow at once (a filter gradient's update), which saves them a wait of their own.
-    std::function<void(size_t)> issue_side = [&](size_t idx) {
-        const plan::Instr& instr = *S.order[idx];
-        if (main_dirty) {
-            hipEvent_t e;
-            if (main_end_known) {
-                e = launch_events.back()->e;
-            } else {
-                HE_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-                events.push_back(e);
-                HE_HIP(hipEventRecord(e, st.s[0]));
-            }
-            HE_HIP(hipStreamWaitEvent(st.s[1], e, 0));
-            local.event_waits++;
-            main_dirty = false;
-        }
-        std::vector<const Tensor*> waited_side;
-        run_instr(instr, 1, true, waited_side);
-        synced_side.insert(waited_side.begin(), waited_side.end());
-        for (NodeId n : instr.all_inputs()) held.push_back(tensors.at(n));
-        for (NodeId n : instr.all_outputs()) held.push_back(tensors.at(n));
-        issued[idx] = 1;
-        for (uint32_t d : S.dependents[idx]) {
-            if (issued[d] || S.side[d] != 1) continue;
-            bool ready = true;
-            for (uint32_t dep : S.deps[d]) ready = ready && issued[dep];
-            if (ready) issue_side(d);
-        }
     };
     // Whatever happens below, the scope must end, and only after the work already queued: a failing instruction leaves
     // earlier launches running on up to four streams. On failure stream 0 is ordered after every stream this execution
     // used, the end event is recorded there as usual, and the error goes on to the caller.
-    EventRef early_done;  // the early instructions' end on the side stream, until the main stream has waited for it
     try {
-    if (side_mode && !instr_timing) {
-        for (size_t idx = 0; idx < S.order.size(); idx++) {
-            if (S.side[idx] != 2) continue;
-            std::vector<const Tensor*> waited_side;
-            run_instr(*S.order[idx], 1, true, waited_side);
-            synced_side.insert(waited_side.begin(), waited_side.end());
-            for (NodeId n : S.order[idx]->all_inputs()) held.push_back(tensors.at(n));
-            for (NodeId n : S.order[idx]->all_outputs()) held.push_back(tensors.at(n));
-            issued[idx] = 1;
-            if (!early_done) early_done = pool.take_event();
-        }
-        if (early_done) HE_HIP(hipEventRecord(early_done->e, st.s[1]));
-    }
     for (size_t step_no = 0; step_no < plan->steps.size(); step_no++) {
         auto& step = plan->steps[step_no];
         for (NodeId r : step.tensors_to_release) tensors.erase(r);
@@ -706,53 +817,11 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
         const size_t width = step_width(step_no);
         std::vector<size_t> cur(width);
         for (size_t w = 0; w < width; w++) cur[w] = w;
-        ht.lap(3);
         join(cur);
-        ht.lap(6);
         for (size_t i = 0; i < step.instrs.size(); i++) {
             const plan::Instr& instr = *step.instrs[i];
             if (instr.absorbed()) continue;  // run, and its outputs allocated, by the instruction that carries it
-            if (side_mode) {
-                const size_t idx = S.index.at(&instr);
-                if (issued[idx]) continue;  // went out early, behind the side instruction it reads
-                if (S.side[idx] == 1) {
-                    issue_side(idx);
-                    continue;
-                }
-                issued[idx] = 1;  // (an early instruction left for here - under instruction timing - runs on the main stream)
-                if (early_done) {
-                    bool reads_early = false;
-                    for (uint32_t d : S.deps[idx]) reads_early = reads_early || S.side[d] == 2;
-                    if (reads_early) {
-                        HE_HIP(hipStreamWaitEvent(st.s[0], early_done->e, 0));
-                        local.event_waits++;
-                        early_done.reset();
-                    }
-                }
-                main_dirty = true;
-                main_end_known = false;
-                if (&instr == closing) {
-                    if (used_streams.count(1)) {
-                        prev_streams = {1};
-                        join({0});
-                        prev_streams = {0};
-                    }
-                    side_joined = true;
-                } else if (!instr_timing && !getenv("HELIUM_HIP_NO_LAUNCH_EVENTS")) {
-                    // when a side instruction comes next, this instruction's last launch carries the event it will wait
-                    // for, which saves the main stream a record of its own
-                    size_t next = idx + 1;
-                    while (next < issued.size() && issued[next]) next++;
-                    if (next < issued.size() && S.side[next] == 1) {
-                        launch_events.push_back(pool.take_event());
-                        set_pending_stop_event(launch_events.back()->e);
-                        run_instr(instr, i % width, false, waited);
-                        main_end_known = take_pending_stop_event() == nullptr;
-                        continue;
-                    }
-                }
-            }
-            run_instr(instr, i % width, false, waited);
+            run_instr(instr, i % width, waited);
         }
         // every stream of the next steps is ordered after this step's streams, so one wait per tensor is enough
         synced.insert(waited.begin(), waited.end());
@@ -773,8 +842,6 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
         retire_join_events(events);
         throw;
     }
-    ht.lap(3);
-    if (side_mode && used_streams.count(1) && !side_joined) prev_streams = {0, 1};
     // Drop of the executor (cuda.rs:232-260): when everything queued above has run, the scope's freed blocks
     // become available to everyone. Stream 0 joins the last step and carries the event the pool polls.
     join({0});
@@ -789,38 +856,14 @@ std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std
     local.streams_used = (int)used_streams.size();
     if (stats) *stats = local;
 
-    if (!instr_times.empty()) {
-        static std::atomic<int> reports{0};
-        if (reports.fetch_add(1) == 1) {  // the second execution: kernels are compiled and loaded by then
-            std::sort(instr_times.begin(), instr_times.end(), [](const InstrTime& a, const InstrTime& b) { return a.us > b.us; });
-            double total = 0;
-            for (auto& t : instr_times) total += t.us;
-            fprintf(stderr, "[instr timing] %zu instructions, %.1f us in all; slowest:\n", instr_times.size(), total);
-            const int top = atoi(getenv("HELIUM_HIP_INSTR_TIMING"));
-            for (int i = 0; i < top && i < (int)instr_times.size(); i++) {
-                const std::string d = instr_times[i].instr->describe();
-                const auto k = instr_times[i].instr->kernel();
-                fprintf(stderr, "  #%-4zu %8.1f us %8.1f MB %6.2f TB/s  %s  %s\n", instr_times[i].order, instr_times[i].us, instr_times[i].bytes / 1e6,
-                        instr_times[i].bytes / instr_times[i].us / 1e6, d.substr(0, 60).c_str(), k ? k->describe().substr(0, 260).c_str() : "");
-            }
-        }
-    }
-    std::map<NodeId, TensorRef> result;
+    NamedTensors result;
     for (NodeId out : graph->outputs()) {
         NodeId from = graph->inbound(out)[0];
         auto it = tensors.find(from);
         HE_REQUIRE(it != tensors.end(), HE_ERR_INTERNAL, "output node %u has no storage", out);
-        result[prepared.caller_output.empty() ? out : prepared.caller_output.at(out)] = it->second;
+        result.emplace_back(prepared.caller_output.empty() ? out : prepared.caller_output.at(out), it->second);
     }
-    ht.lap(5);
-    if (HostTimer::on()) {
-        for (int i = 0; i < 8; i++) g_host_acc[i] += ht.acc[i];
-        if (++g_host_calls % 100 == 0) {
-            fprintf(stderr, "[exec timing] per graph, us: copy+optimize %.1f, plan lookup %.1f, setup %.1f, alloc+waits %.1f, joins %.1f, launches %.1f, finish %.1f\n",
-                    g_host_acc[0] / 100, g_host_acc[1] / 100, g_host_acc[2] / 100, g_host_acc[3] / 100, g_host_acc[6] / 100, g_host_acc[4] / 100, g_host_acc[5] / 100);
-            for (double& v : g_host_acc) v = 0;
-        }
-    }
+    std::sort(result.begin(), result.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
     return result;
 }
 

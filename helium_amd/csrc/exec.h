@@ -21,6 +21,7 @@ using ir::NodeId;
 // When the last holder lets go the event returns to the pool's spare list.
 struct SharedEvent {
     hipEvent_t e = nullptr;
+    hipStream_t on = nullptr;  // the stream it was recorded on: work queued there later needs no wait for it
     ~SharedEvent();
 };
 using EventRef = std::shared_ptr<SharedEvent>;
@@ -59,7 +60,7 @@ public:
     // block is free again for whoever comes after all of those that are still live.
     void release(const Allocation& a, uint64_t owner, const std::vector<uint64_t>& used);
     void note_use(struct Tensor& t, uint64_t scope);
-    void note_uses(const std::map<ir::NodeId, std::shared_ptr<struct Tensor>>& tensors, uint64_t scope);
+    void note_uses(const std::vector<std::shared_ptr<struct Tensor>>& tensors, uint64_t scope);  // (null entries are skipped)
     EventRef take_event();          // an event nobody holds any more, or a new one
     void recycle(hipEvent_t event);  // called when an event's last holder lets go
     void stats(uint64_t* driver_bytes, uint64_t* driver_allocs, uint64_t* reuses);
@@ -104,6 +105,40 @@ struct ExecStats {
     int steps = 0, instrs = 0, streams_used = 0, event_waits = 0;
 };
 
+// What an execution of a plan does when its steps do not fan out over streams: launches in order, each with its kernel and
+// the slots (values in memory) its arguments lie in. Built once per graph (schedule.cpp).
+struct Schedule {
+    struct Named {
+        NodeId node;  // in the caller's graph
+        uint32_t slot;
+    };
+    struct Slot {
+        // a tensor of the caller's; a tensor the caller gets; or part of the execution's own block, at `offset`
+        enum Where : uint8_t { Input, Result, Arena } where = Arena;
+        int dtype = HE_F32;
+        size_t len = 0, bytes = 0;
+        uint64_t offset = 0;
+    };
+    struct Launch {
+        std::shared_ptr<KernelBase> kernel;  // or:
+        std::shared_ptr<Permute> permute;
+        std::vector<uint32_t> args;        // slots in the kernel's argument order (permute: source, destination)
+        std::vector<uint32_t> new_inputs;  // input slots that this stream reads for the first time
+        uint8_t stream = 0;                // 0: the main stream, 1: the side stream
+        bool waits_for_main = false;       // the side stream waits for what the main stream has taken so far
+        bool marks_end = false;            // ... whose latest launch this is: it carries an event
+        bool waits_for_early = false;      // the main stream waits for the early launches
+        bool closes = false;               // the last launch, on the main stream: it carries the execution's event
+    };
+    std::vector<Named> inputs, outputs;  // by node
+    std::vector<Slot> slots;
+    std::vector<Launch> launches;
+    size_t early_launches = 0;  // how many at the head of `launches` are early ones
+    uint64_t arena_bytes = 0;
+    int steps = 0, instrs = 0;  // of the plan
+    bool uses_side = false;
+};
+
 // Everything about an execution that depends on the graph alone: the optimised copy, its plan and the tensors that
 // outlive the plan. Built once per graph by `prepare` and shared by every later execution.
 struct Prepared {
@@ -122,7 +157,16 @@ struct Prepared {
         std::vector<uint8_t> side;
         std::vector<std::vector<uint32_t>> deps, dependents;
     } side;
+    std::shared_ptr<const Schedule> schedule;  // null for a plan whose steps fan out
+    NodeId caller_input(NodeId own) const {
+        for (auto& kv : input_of)
+            if (kv.second == own) return kv.first;
+        return own;
+    }
 };
+// Builds pr->schedule, joined kernels included (compiled, not loaded: needs no device).
+void build_schedule(Prepared* pr);
+using NamedTensors = std::vector<std::pair<NodeId, TensorRef>>;
 // 0: every instruction runs on one stream; 1 (default): the instructions of a step fan out over the thread's streams
 // where the work that can overlap outweighs the joins; 2: every step with several instructions fans out, as
 // cuda.rs:190-221 does.
@@ -131,12 +175,8 @@ void set_stream_fan_out(int mode);
 // beside the main chain are told so (plan::Instr::runs_beside_main_chain), which has to happen before their kernels are made.
 void assign_streams(Prepared* pr);
 std::shared_ptr<const Prepared> prepare(const ir::OpGraph& graph);
-std::map<NodeId, TensorRef> execute_prepared(const Prepared& prepared, const std::map<NodeId, TensorRef>& inputs,
-                                             ExecStats* stats = nullptr);
-
-// BackendExt::execute_graph (backend.rs:40-80). `inputs`: storage for every Input node. Returns the storage of
-// every node that feeds an Output node, keyed by the Output node's id.
-std::map<NodeId, TensorRef> execute_graph(const ir::OpGraph& graph, const std::map<NodeId, TensorRef>& inputs,
-                                          ExecStats* stats = nullptr);
+// BackendExt::execute_graph (backend.rs:40-80) for a prepared graph. `inputs`: storage for every Input node. Returns the
+// storage of every node that feeds an Output node, with the Output node's id, in the order of those.
+NamedTensors execute_prepared(const Prepared& prepared, const NamedTensors& inputs, ExecStats* stats = nullptr);
 
 }  // namespace he::exec

@@ -1047,7 +1047,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     // the loads of the partials are three dependent round trips at the very end of the kernel, and a 4096^3 product with
     // the README's epilogue took 155 us this way against 141. Row sums keep the second launch as well.
     // (a program that rides on the fold launch needs that launch)
-    bool fold_in_kernel = !reds.empty() && pr.split_k == 1 && tiles_m * tiles_n * pr.batch <= 64 && !pr.epi.post &&
+    bool fold_in_kernel = !reds.empty() && pr.split_k == 1 && tiles_m * tiles_n * pr.batch <= (t.wk > 1 ? 256 : 64) && !pr.epi.post &&
                           !tuning::get("HELIUM_HIP_GEMM_NO_TICKET_FOLD");
     for (auto& r : reds) {
         const tp::Out& o = pr.epi.outs[r.out];

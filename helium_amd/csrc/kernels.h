@@ -70,6 +70,10 @@ public:
     size_t scratch_bytes_needed() const override;
     void load() override;
     bool loaded() const override;
+    // Whether the kernel can be part of a JoinedKernel: one launch of blocks that know nothing of each other.
+    bool can_join() const {
+        return launch_.grid && launch_.fills.empty() && !launch_.ws_floats && !launch_.finalize_grid && !prog_.post;
+    }
     ~TileKernel() override;
 
 private:
@@ -78,6 +82,27 @@ private:
     tp::PointwiseLaunch launch_;
     std::unique_ptr<JitKernel> kernel_, finalize_;
     ReduceScratch scratch_;
+};
+
+// Independent tile kernels as one launch: each member's blocks follow the previous member's. For kernels that are too small
+// to be worth a launch each.
+class JoinedKernel : public KernelBase {
+public:
+    explicit JoinedKernel(const std::vector<std::shared_ptr<TileKernel>>& members);
+    const std::vector<tp::Arg>& args() const override { return args_; }  // the members' one after the other
+    const std::string& source() const override { return source_; }
+    const std::string& describe() const override { return describe_; }
+    void execute(void* const* ptrs, hipStream_t stream) override;
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    size_t scratch_bytes_needed() const override { return 0; }
+    void load() override { kernel_->load(); }
+    bool loaded() const override { return kernel_->loaded(); }
+
+private:
+    std::vector<tp::Arg> args_;
+    std::string source_, describe_;
+    std::unique_ptr<JitKernel> kernel_;
+    uint32_t grid_ = 0, threads_ = 256;
 };
 
 // Fused GEMM: C = f(A) g(B) with mainloop op chains applied while tiles are staged into LDS and the epilogue

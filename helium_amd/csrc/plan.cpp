@@ -594,6 +594,8 @@ std::shared_ptr<const Plan> generate_plan(const std::shared_ptr<const ir::OpGrap
                 bool is_small = true;
                 for (NodeId n : small->subgraph().nodes()) is_small = is_small && ir::num_elements(g->get(n).desc.shape) <= (1 << 16);
                 if (!is_small) continue;
+                // (a renamed shape alone is no launch: the executor hands the storage on)
+                if (small->subgraph().nodes().size() == 1 && g->get(small->subgraph().nodes()[0]).op.kind == ir::OpKind::Reshape) continue;
                 // the producer that runs last must be the one whose reductions are read (the others are done before it: earlier
                 // steps, or earlier in a step that then runs in order)
                 bool have = false, reads_reduction = false;

@@ -59,6 +59,11 @@ public:
         std::lock_guard<std::mutex> lk(mu_);
         return kernel_;
     }
+    std::shared_ptr<Permute> permute() const {
+        precompile();
+        std::lock_guard<std::mutex> lk(mu_);
+        return permute_;
+    }
     // Beyond the reference: the executor runs this instruction on its side stream, beside the chain of instructions
     // that everything else waits for (exec.cpp: side_stream_split). Told before the kernel is made, a filter gradient
     // then splits its k range over fewer workgroups: it has time, and the CUs it leaves alone keep the main chain going.

@@ -1,4 +1,6 @@
 // Pointwise / reduction instruction: helium/src/cuda/instr/pointwise.rs + pointwise/jit.rs (kernels K2/K3).
+#include <sstream>
+
 #include "kernels.h"
 
 namespace he {
@@ -148,6 +150,53 @@ void TileKernel::run(void* const* ptrs, hipStream_t stream, ReduceScratch::Buf w
         const uint32_t fgrid[3] = {launch_.finalize_grid, 1, 1};
         finalize_->launch(fgrid, block, 0, stream, argv.data(), true);
     }
+}
+
+JoinedKernel::JoinedKernel(const std::vector<std::shared_ptr<TileKernel>>& members) {
+    HE_REQUIRE(!members.empty(), HE_ERR_INTERNAL, "a joined kernel needs a member");
+    // A member's text is its own kernel made a function: it is told its block, and its constants end with it.
+    const std::string head = "extern \"C\" __global__ __launch_bounds__(256) void ", block = "blockIdx.x";
+    const tp::PointwiseLaunch& first = members[0]->launch_info();
+    std::ostringstream s, calls, params;
+    s << first.source.substr(0, first.prelude_bytes);
+    for (size_t k = 0; k < members.size(); k++) {
+        const tp::PointwiseLaunch& L = members[k]->launch_info();
+        HE_REQUIRE(members[k]->can_join() && L.threads == first.threads && L.options == first.options, HE_ERR_INTERNAL, "a kernel that cannot join others");
+        std::string text = L.source.substr(L.prelude_bytes);
+        const size_t at = text.find(head);
+        HE_REQUIRE(at != std::string::npos, HE_ERR_INTERNAL, "unexpected kernel text");
+        const size_t paren = text.find('(', at + head.size());
+        text.replace(at, paren + 1 - at, "static __device__ __forceinline__ void member_" + std::to_string(k) + "(const u32 member_block, ");
+        for (size_t b = text.find(block); b != std::string::npos; b = text.find(block, b)) text.replace(b, block.size(), "member_block");
+        s << text << "#undef NV\n#undef TX\n#undef TY\n#undef RPT\n#undef TR\n#undef DIM_N\n#undef DIM_M\n";
+        calls << (k ? "else " : "");
+        if (k + 1 < members.size()) calls << "if (blockIdx.x < " << grid_ + L.grid << "u) ";
+        calls << "member_" << k << "(blockIdx.x - " << grid_ << "u";
+        for (const tp::Arg& a : members[k]->args()) {
+            params << (args_.empty() ? "" : ", ") << (a.is_output ? "" : "const ") << tp::c_type(a.dtype) << "* __restrict__ p" << args_.size();
+            calls << ", p" << args_.size();
+            args_.push_back(a);
+        }
+        calls << ");\n";
+        HE_REQUIRE((uint64_t)grid_ + L.grid < (1ull << 31), HE_ERR_UNSUPPORTED, "joined grid too large");
+        grid_ += L.grid;
+        describe_ += (k ? "\n" : "") + L.describe;
+    }
+    threads_ = first.threads;
+    s << head << "joined_kernels(" << params.str() << ") {\n" << calls.str() << "}\n";
+    source_ = s.str();
+    describe_ = "joined members=" + std::to_string(members.size()) + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + "\n" + describe_;
+    kernel_.reset(new JitKernel(source_, "joined_kernels", first.options));
+}
+
+void JoinedKernel::execute(void* const* ptrs, hipStream_t stream) {
+    std::vector<void*> argv(args_.size());
+    for (size_t i = 0; i < args_.size(); i++) {
+        HE_REQUIRE(ptrs[i] != nullptr && ((uintptr_t)ptrs[i] & 15) == 0, HE_ERR_INVALID, "kernel argument %zu is null or not 16-byte aligned", i);
+        argv[i] = (void*)&ptrs[i];
+    }
+    const uint32_t grid[3] = {grid_, 1, 1}, block[3] = {threads_, 1, 1};
+    kernel_->launch(grid, block, 0, stream, argv.data(), true);
 }
 
 }  // namespace he

@@ -132,6 +132,7 @@ bool attach_post(Program* main, const Program& post);
 // ---- emission -----------------------------------------------------------------------------------------------
 struct PointwiseLaunch {
     std::string source, entry;
+    size_t prelude_bytes = 0;  // of `source`, ahead of what is this kernel's own
     uint32_t grid = 1, threads = 256;
     int nv = 1, tx = 1, ty = 1, rpt = 1;
     // Outputs that must be filled before the launch: (argument index, 32-bit fill pattern).

@@ -513,3 +513,33 @@ def test_linear_layer_backward_products(gpu, dtype, precision):
     got, steps = run_graph(g, host)
     assert sorted(k for instrs, _ in steps for k, _ in instrs) == ["gemm", "gemm"], steps
     check_against_oracle(g, host, got, steps, matmul_rel=1e-4 if dtype == "f32" else 1e-2)
+
+
+@pytest.mark.parametrize("count", [1, 3, 30])
+def test_small_elementwise_launches_share_launches(gpu, count):
+    """Elementwise instructions of different sizes run as parts of joined launches (more of them than one launch takes),
+    ahead of and behind a product that reads some of them; results that are another value's storage under another shape
+    (of a sum, of an input) come back whole."""
+    rng = np.random.default_rng(count)
+    g = ha.ir.OpGraph()
+    host = {}
+
+    def new(shape):
+        i = g.new_input(shape, "f32")
+        host[i] = rng.uniform(-1, 1, shape).astype(np.float32)
+        return i
+
+    a, b = g.change_data_type(new([40, 24]), "bf16"), g.change_data_type(new([24, 56]), "bf16")
+    product = g.matmul(a, b, "bf16_f32")
+    g.new_output(g.reshape(product, [56, 40]))
+    total = g.reduce(product, "sum", 1)
+    g.new_output(g.reshape(total, [40]))
+    for k in range(count):
+        x = new([3 + k, 5 + 7 * k])
+        g.new_output(g.change_data_type(g.unary(x, "relu"), "bf16"))
+        w = new([40, 1 + k])  # reads the product's row sums
+        g.new_output(g.binary(w, g.broadcast(g.reshape(total, [40, 1]), 2, [(1, 1 + k)]), "mul"))
+    g.new_output(g.reshape(new([6, 10]), [60]))
+    for _ in range(2):
+        got, steps = run_graph(g, host)
+        check_against_oracle(g, host, got, steps, matmul_rel=1e-2)
