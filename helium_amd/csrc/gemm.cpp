@@ -411,9 +411,17 @@ __device__ __forceinline__ void direct_tile(const unsigned char* __restrict__ rd
    workgroups are meant to share a CU */
 #define KERNEL_ATTRS __attribute__((amdgpu_waves_per_eu(ALL_WAVES / 4 * WGS_PER_CU, ALL_WAVES / 4 * WGS_PER_CU)))
 #endif
+#if GEMM_PART
+/* one of several products that share a launch (CompositeKernel), in a namespace of its own */
+__device__ __forceinline__ void gemm_part(KERNEL_PARAMS, unsigned char* lds, const u32 block_x) {
+    constexpr u32 block_y = 0;
+#else
 extern "C" __global__ __launch_bounds__(ALL_THREADS) KERNEL_ATTRS
 void fused_matmul(KERNEL_PARAMS) {
     __shared__ __attribute__((aligned(16))) unsigned char lds[WAVES_K * NSTAGES * STAGE_BYTES];
+    const u32 block_x = blockIdx.x, block_y = blockIdx.y;
+#endif
+    (void)block_y;
 #if WAVES_K > 1
     const u32 kgroup = __builtin_amdgcn_readfirstlane(threadIdx.x / NTHREADS), tid = threadIdx.x % NTHREADS;
 #else
@@ -426,11 +434,11 @@ void fused_matmul(KERNEL_PARAMS) {
     u32 tile_m, tile_n;
     TILE_ORDER
 #if SPLIT_K > 1
-    // blockIdx.y is the k-range index, not a batch index: this workgroup multiplies k-tiles [kt0, kt0 + KT)
-    const u32 bz = 0, split = blockIdx.y, kt0 = split * KT_PER_SPLIT;
+    // block_y is the k-range index, not a batch index: this workgroup multiplies k-tiles [kt0, kt0 + KT)
+    const u32 bz = 0, split = block_y, kt0 = split * KT_PER_SPLIT;
     const u32 KT_RANGE = kt0 >= KT_ALL ? 0u : (KT_ALL - kt0 < KT_PER_SPLIT ? KT_ALL - kt0 : KT_PER_SPLIT);
 #else
-    const u32 bz = blockIdx.y, kt0 = 0;
+    const u32 bz = block_y, kt0 = 0;
     constexpr u32 KT_RANGE = KT_ALL;
 #endif
     // k-tiles of this wave's group, and how often the workgroup's waves meet at the loop's barrier (a group of one wave
@@ -850,7 +858,7 @@ void validate_gemm_epilogue(const tp::Program& epi) {
 // 15.9 -> 11.9, but 768x768x768 4.7 -> 5.2).
 bool small_tile(const GemmProblem& pr, bool f32, Tile* t) {
     if (pr.split_k > 1) return false;  // shared over workgroups instead, with tiles that go with it
-    auto tiles = [&](int64_t bm, int64_t bn) { return ((pr.M + bm - 1) / bm) * ((pr.N + bn - 1) / bn) * pr.batch; };
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((pr.M + bm - 1) / bm) * ((pr.N + bn - 1) / bn) * pr.batch * pr.siblings; };
     const int64_t k_tiles = (pr.K + t->bk - 1) / t->bk;
     constexpr int64_t kCus = 256;
     int bm = 32, bn = 32, wk = 4;
@@ -873,7 +881,7 @@ bool small_tile(const GemmProblem& pr, bool f32, Tile* t) {
     return true;
 }
 
-GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
+GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(std::move(prob)) {
     const GemmProblem& pr = prob_;
     HE_REQUIRE(pr.M > 0 && pr.N > 0 && pr.K > 0 && pr.batch > 0, HE_ERR_INVALID, "empty GEMM");
     HE_REQUIRE(pr.M < (1ll << 31) && pr.N < (1ll << 31) && pr.K < (1ll << 31) &&
@@ -893,7 +901,10 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     const bool chunk_a = run_a % epc == 0, chunk_b = run_b % epc == 0;
     const bool want_direct = !tuning::get("HELIUM_HIP_GEMM_NO_DIRECT");
     const int esz = 16 / epc;  // bytes per multiplicand
-    if (const char* env = tuning::get("HELIUM_HIP_GEMM_TILE")) {
+    if (tiled_like) {
+        const int* v = tiled_like->tile_;
+        t = {v[0], v[1], v[2], v[3], v[4], v[5], v[6]};
+    } else if (const char* env = tuning::get("HELIUM_HIP_GEMM_TILE")) {
         int v[7] = {256, 256, 64, 2, 4, 2, 1};
         int n = sscanf(env, "%d,%d,%d,%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6]);
         HE_REQUIRE(n >= 5, HE_ERR_INVALID, "HELIUM_HIP_GEMM_TILE wants bm,bn,bk,wm,wn[,stages[,k groups]]");
@@ -959,7 +970,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
             t.wn = 4;
             small = true;
         } else if (!f32 && pr.conv_a.on && pr.conv_a.C % epc == 0 && pr.N >= 256 && pr.N % 256 == 0 && pr.split_k == 1 &&
-                   ((pr.M + 255) / 256) * (pr.N / 256) * pr.batch < 128 && ((pr.M + 127) / 128) * (pr.N / 256) * pr.batch >= 192 &&
+                   ((pr.M + 255) / 256) * (pr.N / 256) * pr.batch * pr.siblings < 128 && ((pr.M + 127) / 128) * (pr.N / 256) * pr.batch * pr.siblings >= 192 &&
                    !tuning::get("HELIUM_HIP_GEMM_NO_WIDE_CONV_TILES")) {
             // a convolution (or data gradient) into a multiple of 256 channels whose 256x256 tiles would leave half the chip
             // idle while 128x256 tiles fill three quarters of it or more: the filter travels to half as many workgroups
@@ -975,7 +986,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         // (a split k range multiplies the workgroups: the filter gradients of 256 and 512 channels keep the large tile,
         // 81 -> 70 us and 93 -> 78 us)
         // (... of 512; with 256 output channels eight waves on the small tile do better: 46.8 -> 41.5 and 71.1 -> 67.1 us)
-        if (pr.M <= 128 || pr.N <= 128 || ((pr.M + 255) / 256) * ((pr.N + 255) / 256) * pr.batch * pr.split_k < 128 ||
+        if (pr.M <= 128 || pr.N <= 128 || ((pr.M + 255) / 256) * ((pr.N + 255) / 256) * pr.batch * pr.siblings * pr.split_k < 128 ||
             (pr.conv_b.on && !f32 && pr.conv_b.C % epc == 0 && pr.M <= 256)) {
             t.bm = t.bn = 128;
             t.wm = t.wn = 2;
@@ -987,7 +998,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
             small = true;
             // still fewer workgroups than half the CUs: 64x64 tiles (one MFMA block per wave) spread the work
             // (a split k range multiplies the workgroups instead and keeps the tile's arithmetic intensity)
-            if (pr.M > 64 && pr.N > 64 && ((pr.M + 127) / 128) * ((pr.N + 127) / 128) * pr.batch * pr.split_k < 128) {
+            if (pr.M > 64 && pr.N > 64 && ((pr.M + 127) / 128) * ((pr.N + 127) / 128) * pr.batch * pr.siblings * pr.split_k < 128) {
                 t.bm = t.bn = 64;
                 t.wn = 2;
             }
@@ -1047,7 +1058,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     // the loads of the partials are three dependent round trips at the very end of the kernel, and a 4096^3 product with
     // the README's epilogue took 155 us this way against 141. Row sums keep the second launch as well.
     // (a program that rides on the fold launch needs that launch)
-    bool fold_in_kernel = !reds.empty() && pr.split_k == 1 && tiles_m * tiles_n * pr.batch <= (t.wk > 1 ? 256 : 64) && !pr.epi.post &&
+    bool fold_in_kernel = !reds.empty() && pr.split_k == 1 && tiles_m * tiles_n * pr.batch <= (t.wk > 1 ? 256 : 64) && tiles_m <= 32 && !pr.epi.post &&
                           !tuning::get("HELIUM_HIP_GEMM_NO_TICKET_FOLD");
     for (auto& r : reds) {
         const tp::Out& o = pr.epi.outs[r.out];
@@ -1090,11 +1101,11 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                              (int64_t)pr.conv_a.N * pr.conv_a.H * pr.conv_a.W * pr.conv_a.C < (int64_t(1) << 32) &&
                              !tuning::get("HELIUM_HIP_GEMM_NO_CONV_FAST");
     if (!(direct_a && direct_b)) t.stages = 2;  // register staging is double-buffered only
-    else if (!tuning::get("HELIUM_HIP_GEMM_TILE") && small) {
+    else if (!tuning::get("HELIUM_HIP_GEMM_TILE") && small && !tiled_like) {
         // A grid that leaves CUs idle is bound by the latency of its k-loop: keep as many tiles in flight as LDS holds.
         // With more than one workgroup per CU (a split k range) the LDS is better spent on a second and third
         // workgroup, whose loads hide each other's waits (filter gradient of a 64-channel layer: 66 -> 56 us).
-        const int64_t workgroups = ((pr.M + t.bm - 1) / t.bm) * ((pr.N + t.bn - 1) / t.bn) * pr.batch * pr.split_k;
+        const int64_t workgroups = ((pr.M + t.bm - 1) / t.bm) * ((pr.N + t.bn - 1) / t.bn) * pr.batch * pr.siblings * pr.split_k;
         // (not for a data gradient's gather: at batch 128 the 7x7x512 layer takes 54.2 us with four stages, 49.7 with three,
         // 48.9 with two, the 14x14x256 layer at batch 64 29.3 / 27.5 / 27.8; the forward gather does not care)
         const bool deeper = !(pr.conv_a.on && pr.conv_a.bwd);
@@ -1103,6 +1114,10 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
     // All direct loads of the next tile are issued at the start of a tile's MFMAs (the round trip needs the whole
     // tile to hide); HELIUM_HIP_GEMM_ISSUE=0 spreads them over the k-steps instead.
     const bool issue_front = tuning::get("HELIUM_HIP_GEMM_ISSUE") ? atoi(tuning::get("HELIUM_HIP_GEMM_ISSUE")) != 0 : true;
+    {
+        const int v[7] = {t.bm, t.bn, t.bk, t.wm, t.wn, t.stages, t.wk};
+        memcpy(tile_, v, sizeof v);
+    }
     int nve = std::min(8, tp::pick_nv(pr.epi, 32));
     const int nve_any = std::min(8, tp::pick_nv(pr.epi, 32, true));
     // (rows that are no multiple of 4 elements: guarded vectors, loaded and stored element by element only at a row's end)
@@ -1128,7 +1143,9 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         const int acc_regs = t.bm * t.bn / threads;
         int wgs = tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU") ? atoi(tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU")) : (lds_bytes * 2 <= 160 * 1024 && acc_regs <= 32 ? 2 : 1);
         if (threads * t.wk < 256) wgs = 1;
-        wgs_per_cu_attr = "\n#define WGS_PER_CU " + std::to_string(std::max(1, wgs));
+        wgs_per_cu_ = std::max(1, wgs);
+        lds_bytes_ = (uint32_t)lds_bytes;
+        wgs_per_cu_attr = "\n#define WGS_PER_CU " + std::to_string(wgs_per_cu_);
     }
     s << "#define BM " << t.bm << "\n#define BN " << t.bn << "\n#define BK " << t.bk << "\n#define WAVES_M " << t.wm
       << "\n#define WAVES_N " << t.wn << "\n#define WAVES_K " << t.wk << wgs_per_cu_attr << "\n#define NSTAGES " << t.stages << "\n#define NVE " << nve << "\n#define MMA_BF16 " << (pr.mma_dtype == HE_BF16 ? 1 : 0) << "\n#define MMA_F32 " << (f32 ? 1 : 0)
@@ -1555,7 +1572,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
         // (with several k ranges or batch entries the dealing goes on from one row of the grid to the next: only whole
         // multiples of 8 keep a tile's ranges on one XCD, and filter gradients of 3 to 41 ranges lost up to 1.6x without)
         const bool xcd = ((tm * tn) % 8 == 0 || (pr.split_k == 1 && pr.batch == 1)) && !tuning::get("HELIUM_HIP_GEMM_NO_XCD");
-        o << "{ u32 b = blockIdx.x;\n";
+        o << "{ u32 b = block_x;\n";
         const int64_t whole = tm * tn / 8, over = tm * tn % 8;  // (the first `over` XCDs take one tile more)
         if (xcd) o << "b = (b % 8u) * " << whole << "u" << (over ? " + (b % 8u < " + std::to_string(over) + "u ? b % 8u : " + std::to_string(over) + "u)" : std::string()) << " + b / 8u;\n";
         const int G = tuning::get("HELIUM_HIP_GEMM_GROUP") ? atoi(tuning::get("HELIUM_HIP_GEMM_GROUP")) : 4;
@@ -1763,6 +1780,7 @@ GemmKernel::GemmKernel(GemmProblem prob) : prob_(std::move(prob)) {
                        (long long)pr.batch, (long long)pr.M, (long long)pr.K, (long long)pr.N, t.bm, t.bn, t.bk, t.stages, t.wm, t.wn, threads * t.wk, t.wk,
                        grid_[0], grid_[1], (int)raw_a, (int)raw_b, nva, nvb, nve, (int)direct_a, (int)direct_b, dtype_name(pr.mma_dtype), pr.epi.exprs.size(),
                        pr.epi.outs.size(), pr.split_k, (unsigned long long)reduce_floats_, reduce_grid_, reduce_args.c_str(), (unsigned long long)reduce_counters_);
+    if (pr.siblings > 1) return;  // compiled as a part of the launch that they share
     kernel_.reset(new JitKernel(source_, "fused_matmul", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));
     if (pr.split_k > 1) finalize_.reset(new JitKernel(source_, "fused_matmul_finalize", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));
     if (pr.epi.post) describe_ += strfmt(" carries=%zuexprs/%zuouts", pr.epi.post->exprs.size(), pr.epi.post->outs.size());
@@ -1848,28 +1866,93 @@ void GemmKernel::run(void* const* ptrs, hipStream_t stream, float* ws, uint32_t*
     }
 }
 
-CompositeKernel::CompositeKernel(std::vector<std::unique_ptr<KernelBase>> parts, bool zero_outputs_first)
-    : parts_(std::move(parts)), zero_first_(zero_outputs_first) {
-    HE_REQUIRE(!parts_.empty(), HE_ERR_INTERNAL, "a composite kernel needs a part");
-    for (auto& p : parts_) {
-        HE_REQUIRE(p->args().size() == parts_[0]->args().size(), HE_ERR_INTERNAL, "the parts of a composite kernel take different arguments");
-        // (sources and descriptions one after the other, each introduced by a line that names the part)
-        source_ += "// ---- part " + std::to_string(&p - &parts_[0]) + " of " + std::to_string(parts_.size()) + "\n" + p->source() + "\n";
-        describe_ += (describe_.empty() ? "" : "\n") + p->describe();
+namespace {
+// The names a generated product defines for the preprocessor, those of the shared prelude aside.
+std::vector<std::string> macros_of(const std::string& text) {
+    std::vector<std::string> names;
+    const std::string directive = "#define ";
+    for (size_t at = text.find(directive); at != std::string::npos; at = text.find(directive, at + 1)) {
+        if (at && text[at - 1] != '\n') continue;
+        size_t end = at + directive.size();
+        while (end < text.size() && (isalnum((unsigned char)text[end]) || text[end] == '_')) end++;
+        const std::string name = text.substr(at + directive.size(), end - at - directive.size());
+        if (name.compare(0, 3, "HE_") == 0 || name == "LDS_AS" || name == "GLOBAL_AS" || name == "KERNEL_ATTRS") continue;
+        if (std::find(names.begin(), names.end(), name) == names.end()) names.push_back(name);
     }
-    describe_ = "composite parts=" + std::to_string(parts_.size()) + " zero_first=" + (zero_first_ ? "1" : "0") + "\n" + describe_;
+    return names;
+}
+}  // namespace
+
+CompositeKernel::CompositeKernel(std::vector<GemmProblem> problems, bool zero_the_rest) {
+    HE_REQUIRE(!problems.empty(), HE_ERR_INTERNAL, "a composite kernel needs a part");
+    // The products with the longest k first: their workgroups are the ones that the launch ends with otherwise. All take the
+    // tiles of the first, chosen for as many workgroups as there are products.
+    std::stable_sort(problems.begin(), problems.end(), [](const GemmProblem& x, const GemmProblem& y) { return x.K > y.K; });
+    const int siblings = std::max<int>(2, (int)problems.size());  // (never one: a part is not compiled by itself)
+    for (auto& pr : problems) {
+        HE_REQUIRE(pr.out_rows.on && pr.batch == 1, HE_ERR_INTERNAL, "the parts of a composite kernel write rows of one tensor");
+        pr.siblings = siblings;
+        parts_.emplace_back(new GemmKernel(std::move(pr), parts_.empty() ? nullptr : parts_[0].get()));
+    }
+    const GemmKernel& first = *parts_[0];
+    const std::vector<tp::Arg>& args = first.args();
+    std::ostringstream bodies, s, calls;
+    uint32_t lds = 0;
+    for (size_t k = 0; k < parts_.size(); k++) {
+        GemmKernel& p = *parts_[k];
+        HE_REQUIRE(p.args().size() == args.size() && p.threads_ == first.threads_ && p.grid_[1] == 1, HE_ERR_INTERNAL, "the parts of a composite kernel differ");
+        lds = std::max(lds, p.lds_bytes_);
+        bodies << "#define GEMM_PART 1\nnamespace part_" << k << " {\n" << p.source() << "}\n";
+        for (auto& name : macros_of(p.source())) bodies << "#undef " << name << "\n";
+        bodies << "#undef GEMM_PART\n";
+        // (whole multiples of 8 blocks: the XCD that a part's tile order counts on is its block number's, part or whole)
+        calls << "if (b < " << grid_ + p.grid_[0] << "u) {\n" << "part_" << k << "::gemm_part(";
+        for (size_t a = 0; a < args.size(); a++) calls << "p" << a << ", ";
+        calls << "lds, b - " << grid_ << "u);\nreturn;\n}\n";
+        grid_ = (grid_ + p.grid_[0] + 7) / 8 * 8;
+        if (k + 1 < parts_.size()) calls << "if (b < " << grid_ << "u) return;\n";
+        describe_ += (describe_.empty() ? "" : "\n") + p.describe();
+    }
+    threads_ = first.threads_;
+    if (zero_the_rest) {
+        // what no part writes: the pixels of the classes that no tap reaches, 16 bytes at a time
+        const GemmProblem& pr = first.problem();
+        const auto& r = pr.out_rows;
+        const tp::Arg& out = args[pr.map_e[pr.epi.outs[0].arg]];
+        const int64_t row_chunks = pr.N * (dtype_bits(out.dtype) / 8) / 16, chunks = out.numel / pr.N * row_chunks;
+        HE_REQUIRE(pr.N * (dtype_bits(out.dtype) / 8) % 16 == 0 && chunks < (1ll << 31), HE_ERR_UNSUPPORTED, "gradient rows that are no whole 16-byte chunks");
+        const uint32_t blocks = (uint32_t)std::min<int64_t>((chunks + threads_ - 1) / threads_, 2048);
+        calls << "for (unsigned i = (b - " << grid_ << "u) * " << threads_ << "u + threadIdx.x; i < " << chunks << "u; i += " << (uint64_t)blocks * threads_
+              << "u) {\nconst unsigned pixel = i / " << row_chunks << "u, w = pixel % " << r.W << "u, h = pixel / " << r.W << "u % " << r.H << "u;\nbool written = false;\n";
+        for (auto& p : parts_)
+            calls << "written = written || (h % " << r.sh << "u == " << p->problem().out_rows.a << "u && w % " << r.sw << "u == " << p->problem().out_rows.b << "u);\n";
+        calls << "if (!written) ((zero_chunk_t*)p" << pr.map_e[pr.epi.outs[0].arg] << ")[i] = zero_chunk_t{0u, 0u, 0u, 0u};\n}\n";
+        grid_ += blocks;
+    }
+    s << bodies.str() << "typedef unsigned zero_chunk_t __attribute__((ext_vector_type(4)));\n#define ALL_WAVES " << threads_ / 64 << "\n#define WGS_PER_CU " << first.wgs_per_cu_
+      << "\nextern \"C\" __global__ __launch_bounds__(" << threads_ << ") KERNEL_ATTRS\nvoid fused_matmul_parts(";
+    for (size_t a = 0; a < args.size(); a++)
+        s << (a ? ", " : "") << (args[a].is_output ? "" : "const ") << (args[a].dtype == HE_F32 ? "" : "part_0::") << tp::c_type(args[a].dtype) << "* __restrict__ p" << a;
+    s << ") {\n__shared__ __attribute__((aligned(16))) unsigned char lds[" << lds << "];\nconst unsigned b = blockIdx.x;\n" << calls.str() << "}\n";
+    const std::string text = s.str();
+    source_ = text;
+    // (sources and descriptions one after the other, each introduced by a line that names the part)
+    for (auto& p : parts_) source_ += "// ---- part " + std::to_string(&p - &parts_[0]) + " of " + std::to_string(parts_.size()) + "\n" + p->source() + "\n";
+    describe_ = "composite parts=" + std::to_string(parts_.size()) + " zero_first=" + (zero_the_rest ? "1" : "0") + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + "\n" + describe_;
+    kernel_.reset(new JitKernel(text, "fused_matmul_parts", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));
 }
 
-void CompositeKernel::zero_outputs(void* const* ptrs, hipStream_t stream) const {
-    std::vector<std::pair<void*, std::pair<uint32_t, uint32_t>>> fills;
-    const auto& a = args();
-    for (size_t i = 0; i < a.size(); i++)
-        // (whole words, rounded up: an odd count of 16-bit elements ends in half a word, and blocks are 256-byte granules)
-        if (a[i].is_output) fills.push_back({ptrs[i], {(uint32_t)((storage_bytes(a[i].dtype, (size_t)a[i].numel) + 3) / 4), 0u}});
-    if (!fills.empty()) fill_buffers(fills, stream);
+void CompositeKernel::execute(void* const* ptrs, hipStream_t stream) {
+    std::vector<void*> argv(args().size());
+    for (size_t i = 0; i < argv.size(); i++) {
+        HE_REQUIRE(ptrs[i] != nullptr && ((uintptr_t)ptrs[i] & 15) == 0, HE_ERR_INVALID, "kernel argument %zu is null or not 16-byte aligned", i);
+        argv[i] = (void*)&ptrs[i];
+    }
+    const uint32_t grid[3] = {grid_, 1, 1}, block[3] = {threads_, 1, 1};
+    kernel_->launch(grid, block, 0, stream, argv.data(), true);
 }
 
-// Only the last part's last launch closes the instruction: an event that is pending for it is held back until then.
+// Only an instruction's last launch closes it: an event that is pending for it is held back until then.
 namespace {
 struct HeldStopEvent {
     hipEvent_t e = take_pending_stop_event();
@@ -1880,41 +1963,6 @@ struct HeldStopEvent {
     ~HeldStopEvent() { give_back(); }
 };
 }  // namespace
-
-void CompositeKernel::execute(void* const* ptrs, hipStream_t stream) {
-    HeldStopEvent held;
-    if (zero_first_) zero_outputs(ptrs, stream);
-    for (auto& p : parts_) {
-        if (&p == &parts_.back()) held.give_back();
-        p->execute(ptrs, stream);
-    }
-}
-
-void CompositeKernel::execute_in_scratch(void* const* ptrs, hipStream_t stream, void* scratch, size_t scratch_bytes) {
-    HeldStopEvent held;
-    if (zero_first_) zero_outputs(ptrs, stream);
-    for (auto& p : parts_) {
-        if (&p == &parts_.back()) held.give_back();
-        p->execute_in_scratch(ptrs, stream, scratch, scratch_bytes);  // (one after the other: they may share it)
-    }
-}
-
-size_t CompositeKernel::scratch_bytes_needed() const {
-    size_t need = 0;
-    for (auto& p : parts_) need = std::max(need, p->scratch_bytes_needed());
-    return need;
-}
-
-void CompositeKernel::load() {
-    for (auto& p : parts_) p->load();
-    if (zero_first_) load_fill_kernel();
-}
-
-bool CompositeKernel::loaded() const {
-    for (auto& p : parts_)
-        if (!p->loaded()) return false;
-    return !zero_first_ || fill_kernel_loaded();
-}
 
 // ---------------------------------------------------------------------------------------------------------
 // Convolutions over a repacked few-channel image

@@ -110,6 +110,7 @@ private:
 // helium-playground/src/kernel_generator.rs + templates/matmul.cu).
 struct GemmProblem {
     int64_t batch = 1, M = 0, N = 0, K = 0;
+    int siblings = 1;              // products of about this size in the same launch (CompositeKernel)
     int mma_dtype = HE_BF16;       // multiplicand type: HE_BF16, HE_F16 or HE_F32
     tp::Program op_a, op_b, epi;   // dims [batch,M,K], [batch,K,N] ([batch,N,K] when b_nk), [batch,M,N]
     // B's source is contiguous along k (a transposed matrix, a convolution filter): its program iterates [batch,N,K],
@@ -170,7 +171,8 @@ void validate_gemm_epilogue(const tp::Program& epi);
 
 class GemmKernel : public KernelBase {
 public:
-    explicit GemmKernel(GemmProblem prob);
+    // `tiled_like`: take that kernel's tile
+    explicit GemmKernel(GemmProblem prob, const GemmKernel* tiled_like = nullptr);
     const std::vector<tp::Arg>& args() const override { return prob_.args; }
     const std::string& source() const override { return source_; }
     const std::string& describe() const override { return describe_; }
@@ -183,8 +185,12 @@ public:
     ~GemmKernel() override;
 
 private:
+    friend class CompositeKernel;
     void run(void* const* ptrs, hipStream_t stream, float* ws, uint32_t* counters);
     GemmProblem prob_;
+    int tile_[7] = {0};  // rows, columns, k, waves along rows, columns, LDS stages, k groups
+    int wgs_per_cu_ = 1;
+    uint32_t lds_bytes_ = 0;
     std::string source_, describe_;
     // finalize_: adds up the partial tiles of a split-k product; reduce_: folds the partials of the epilogue's reductions
     std::unique_ptr<JitKernel> kernel_, finalize_, reduce_;
@@ -198,26 +204,26 @@ private:
     ReduceScratch scratch_;
 };
 
-// Several kernels with one argument list, launched one after the other on the same stream (the classes of a strided
-// data gradient). `zero_outputs_first`: the kernels do not write every element of the outputs; the rest is zero.
+// Several products with one argument list in one launch: the classes of a strided data gradient, each of which writes some
+// rows of the output (GemmProblem::OutRows). One after the other they were up to four launches (and a fill), each with a
+// tail of its own. `zero_the_rest`: the parts do not write every row; the launch zeroes the others.
 class CompositeKernel : public KernelBase {
 public:
-    CompositeKernel(std::vector<std::unique_ptr<KernelBase>> parts, bool zero_outputs_first);
+    CompositeKernel(std::vector<GemmProblem> problems, bool zero_the_rest);
     const std::vector<tp::Arg>& args() const override { return parts_[0]->args(); }
-    const std::string& source() const override { return source_; }
+    const std::string& source() const override { return source_; }  // of the launch, then of each part by itself
     const std::string& describe() const override { return describe_; }
     void execute(void* const* ptrs, hipStream_t stream) override;
-    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void* scratch, size_t scratch_bytes) override;
-    size_t scratch_bytes_needed() const override;
-    void load() override;
-    bool loaded() const override;
-    const std::vector<std::unique_ptr<KernelBase>>& parts() const { return parts_; }
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    size_t scratch_bytes_needed() const override { return 0; }
+    void load() override { kernel_->load(); }
+    bool loaded() const override { return kernel_->loaded(); }
 
 private:
-    void zero_outputs(void* const* ptrs, hipStream_t stream) const;
-    std::vector<std::unique_ptr<KernelBase>> parts_;
-    bool zero_first_;
+    std::vector<std::unique_ptr<GemmKernel>> parts_;  // sources only
     std::string source_, describe_;
+    std::unique_ptr<JitKernel> kernel_;
+    uint32_t grid_ = 0, threads_ = 256;
 };
 
 // A convolution (or its filter gradient) over a 16-bit image of 3 or 4 channels, run over a repacked copy of the

@@ -1242,11 +1242,7 @@ std::unique_ptr<KernelBase> make_gemm_kernel(const ir::OpSubgraph& sg, const ir:
     // stride): each multiplies only the taps that reach its pixels.
     bool any_empty = false;
     std::vector<GemmProblem> classes = strided_data_gradient_classes(sg, &any_empty);
-    if (!classes.empty()) {
-        std::vector<std::unique_ptr<KernelBase>> parts;
-        for (auto& pr : classes) parts.emplace_back(new GemmKernel(std::move(pr)));
-        return std::unique_ptr<KernelBase>(new CompositeKernel(std::move(parts), any_empty));
-    }
+    if (!classes.empty()) return std::unique_ptr<KernelBase>(new CompositeKernel(std::move(classes), any_empty));
     GemmProblem pr = gemm_problem_from_ir(sg);
     // A filter gradient that runs beside the main chain takes 0.4 of the workgroups it would take alone: four in ten of
     // the CUs are then busy with it and the main chain's kernels keep the rest, where a launch that fills the chip

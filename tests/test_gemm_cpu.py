@@ -492,6 +492,33 @@ def test_conv_backward_data_on_cpu(name, image, oc, kernel, dtype, stride, dilat
     assert np.abs(got[dx] - want).max() <= tol * max(1.0, np.abs(want).max()), (k.description, np.abs(got[dx] - want).max())
 
 
+@pytest.mark.parametrize("case", [c for c in BWD_DATA_CASES if c[5] != (1, 1) and c[6] == (1, 1)], ids=lambda c: c[0])
+def test_classes_of_a_strided_data_gradient_share_a_launch(case):
+    """The launch itself: every pixel of the gradient is written by it, those that no tap reaches with zeros."""
+    from oracle import helium_ir as oracle_ir
+
+    _, image, oc, kernel, dtype, stride, dilation, mode, _ = case
+    rng = np.random.default_rng(12)
+    params = {"in_channels": image[3], "out_channels": oc, "kernel_size": list(kernel), "stride": list(stride),
+              "dilation": list(dilation), "padding_mode": mode}
+    flow_shape = [image[0], *oracle_ir.conv_output_size(params, image[1:3], kernel), oc]
+    filter_shape = [oc, kernel[0], kernel[1], image[3]]
+    g = ha.ir.OpGraph()
+    dy = g.new_input(flow_shape, dtype); w = g.new_input(filter_shape, dtype)
+    dx = g.conv_backward_data(dy, w, params, image[1:3])
+    g.new_output(dx)
+    inputs = {dy: nm.to_storage(rng.uniform(-1, 1, flow_shape).astype(np.float32), dtype),
+              w: nm.to_storage((rng.uniform(-1, 1, filter_shape) * 0.25).astype(np.float32), dtype)}
+    k = ha.backend.matmul_kernel(g, [dx])
+    grid, threads = (int(v) for v in re.search(r"grid=(\d+) threads=(\d+)", k.description).groups())
+    bufs = [(np.zeros(a["numel"], dtype=nm.NP_STORAGE[a["dtype"]]), 1) if a["is_output"] else (inputs[a["node"]], 0) for a in k.args]
+    (got,) = run_kernel(re.split(r"// ---- part \d+ of \d+\n", k.source)[0], "fused_matmul_parts", grid, threads, bufs)
+    got = nm.from_storage(got, dtype, [got.size]).astype(np.float64)
+    want = oracle_ir.kernel_outputs(g.nodes, inputs, [dx])[dx]
+    want = nm.from_storage(want.reshape(-1), dtype, [want.size]).astype(np.float64)
+    assert np.abs(got - want).max() <= (1e-4 if dtype == "f32" else 2e-2) * max(1.0, np.abs(want).max()), k.description
+
+
 BWD_FILTER_CASES = [
     # name, image NHWC, out channels, kernel, dtype, stride, dilation, mode, tile
     ("3x3_same_bf16", (2, 9, 10, 16), 24, (3, 3), "bf16", (1, 1), (1, 1), "same", "128,128,64,2,2"),
