@@ -27,6 +27,7 @@ struct Tile {
     int bm = 256, bn = 256, bk = 64;  // workgroup tile
     int wm = 2, wn = 4;               // waves along m / n (wm * wn * 64 threads)
     int stages = 2;                   // LDS stages (direct global->LDS loads use a deeper ring)
+    int wgs = 0;                      // workgroups that are meant to share a CU (0: two where LDS and accumulators allow it)
     int wk = 1;                       // groups of wm * wn waves that share the tile's k range (their sums meet in LDS)
 };
 
@@ -881,6 +882,44 @@ bool small_tile(const GemmProblem& pr, bool f32, Tile* t) {
     return true;
 }
 
+// Tiles for a 16-bit product of some hundreds of 128x128 tiles. `staged`: an operand goes through registers; `fused`: it has
+// arithmetic on the way. False: the usual ones. Measured (us; rows x columns x k; before: 128x128 tiles of four waves, or
+// 256x256, one workgroup to a CU):
+//  - 256x256 tiles do about 4/3 of the work per CU and time that 128x128 ones do, so they pay as long as the rounds they take
+//    are filled three quarters as well: 4001x4001x2001 plain, odd, 157 against 193; but 16 times 777x1203x1000 (1.25 rounds of
+//    256x256 tiles) 116 -> 93 on 64x128;
+//  - up to one 128x128 tile for a CU, 64x128 tiles of eight waves, two workgroups to a CU: 1501x1501 with the 40-op epilogue
+//    55 -> 40, a 2048x2048x2048 product with operand arithmetic 41 -> 30; where operands move by direct loads only up to
+//    three quarters of that (2048x1024x1024 11.6 -> 7.3; 2048x2048x512 loses);
+//  - beyond, two 128x128 workgroups to a CU: 2323x2323x2323 78 -> 53, 2324x2324 with the 40-op epilogue 96 -> 60;
+//  - with operand arithmetic, three of 64x128: what bounds these is the chain request - evaluate - store to LDS of every
+//    k-tile, which other workgroups hide. 4 times 777x1203x1000 56 -> 30.
+bool mid_tile(const GemmProblem& pr, bool staged, bool fused, Tile* t) {
+    if (pr.conv_a.on || pr.conv_b.on || pr.split_k > 1 || pr.M <= 64 || pr.N <= 64) return false;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((pr.M + bm - 1) / bm) * ((pr.N + bn - 1) / bn) * pr.batch; };
+    constexpr int64_t kCus = 256;
+    // the share of the workgroups' places that holds elements of the result
+    auto filled = [&](int64_t bm, int64_t bn, int64_t per_cu) {
+        const int64_t n = tiles(bm, bn), places = kCus * per_cu;
+        return (double)pr.batch * pr.M * pr.N / ((double)((n + places - 1) / places * places) * bm * bn);
+    };
+    const int64_t t128 = tiles(128, 128);
+    if (t128 < kCus / 2 || (tiles(256, 256) >= kCus / 2 && filled(256, 256, 1) >= 0.75 * filled(128, 128, 2))) return false;
+    t->bm = t->bn = 128;
+    t->wm = t->wn = 2;
+    if (t128 <= (staged ? kCus : kCus * 3 / 4 - 1)) {
+        t->bm = 64;
+        t->wn = 4;
+        t->wgs = 2;
+    } else if (fused) {
+        t->bm = 64;
+        t->wgs = 3;
+    } else if (t128 > kCus) {
+        t->wgs = 2;
+    }
+    return true;
+}
+
 GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(std::move(prob)) {
     const GemmProblem& pr = prob_;
     HE_REQUIRE(pr.M > 0 && pr.N > 0 && pr.K > 0 && pr.batch > 0, HE_ERR_INVALID, "empty GEMM");
@@ -903,12 +942,12 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
     const int esz = 16 / epc;  // bytes per multiplicand
     if (tiled_like) {
         const int* v = tiled_like->tile_;
-        t = {v[0], v[1], v[2], v[3], v[4], v[5], v[6]};
+        t = {v[0], v[1], v[2], v[3], v[4], v[5], 0, v[6]};
     } else if (const char* env = tuning::get("HELIUM_HIP_GEMM_TILE")) {
         int v[7] = {256, 256, 64, 2, 4, 2, 1};
         int n = sscanf(env, "%d,%d,%d,%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6]);
         HE_REQUIRE(n >= 5, HE_ERR_INVALID, "HELIUM_HIP_GEMM_TILE wants bm,bn,bk,wm,wn[,stages[,k groups]]");
-        t = {v[0], v[1], v[2], v[3], v[4], v[5], v[6]};
+        t = {v[0], v[1], v[2], v[3], v[4], v[5], 0, v[6]};
     } else {
         if (f32) t.bk = 32;  // same bytes per tile row as 64 two-byte multiplicands
         // A skinny product (few output columns, many rows: a convolution with 64 output channels) takes tiles as
@@ -922,7 +961,7 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
         // than the unused half of a 256x64 tile costs (7x7 stem: 885 us with 128x128 tiles, 408 with 256x32, 276 with 256x64).
         const bool narrow = !f32 && pr.N <= 32 && pr.N > 16 && pr.M >= 256 * 256;
         const bool gathered_by_element = pr.conv_a.on && pr.conv_a.C % epc != 0;
-        if (small_tile(pr, f32, &t)) {
+        if (small_tile(pr, f32, &t) || (!f32 && mid_tile(pr, !(raw_a0 && chunk_a && raw_b0 && chunk_b), !(raw_a0 && raw_b0), &t))) {
             // (t is set)
         } else if (skinny || (narrow && gathered_by_element)) {
             t.bm = 256;
@@ -1141,7 +1180,7 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
     {
         const int lds_bytes = t.wk * t.stages * (t.bm + t.bn) * t.bk * esz;
         const int acc_regs = t.bm * t.bn / threads;
-        int wgs = tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU") ? atoi(tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU")) : (lds_bytes * 2 <= 160 * 1024 && acc_regs <= 32 ? 2 : 1);
+        int wgs = tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU") ? atoi(tuning::get("HELIUM_HIP_GEMM_WGS_PER_CU")) : t.wgs ? t.wgs : (lds_bytes * 2 <= 160 * 1024 && acc_regs <= 32 ? 2 : 1);
         if (threads * t.wk < 256) wgs = 1;
         wgs_per_cu_ = std::max(1, wgs);
         lds_bytes_ = (uint32_t)lds_bytes;
