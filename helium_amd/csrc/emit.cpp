@@ -625,7 +625,13 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
         L.source = "";
         return L;
     }
-    const int NV = pick_nv(p, 16);
+    // Rows of odd length: vectors at any element's alignment, the row's last one guarded, where aligned ones would move less
+    // than half as much. A wave that moves 4 bytes per lane keeps too little in flight: a [5000 x 3001] f32 chain with four
+    // operands, its values and two reductions of them 87.6 -> 68.5 us. (Small tensors are not bound by that.)
+    const int nv_aligned = pick_nv(p, 16), nv_any = pick_nv(p, 16, true);
+    const bool guarded = nv_aligned * 4 <= nv_any && ir::num_elements(p.dims) >= 1 << 16 && !tuning::get("HELIUM_HIP_POINTWISE_NO_GUARD");
+    const int NV = guarded ? nv_any : nv_aligned;
+    const std::string row_end = guarded ? "(DIM_N - n0)" : "", row_inside = guarded ? "(u32)NV" : "";
     const int threads = 256;
     // A Mean is the sum scaled by 1/group. The reference scales every term (float * double literal,
     // pointwise/jit.rs:413-418); scaling the finished sum once, also in double, differs from that by rounding only
@@ -808,11 +814,14 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
             EmitCtx cx;
             cx.nv = NV;
             cx.row_part = 1;
+            cx.count = row_end;
             s << emit_exprs(p, cx);
         }
     }
     std::ostringstream& main_stream = s;
-    auto row_body = [&](bool squares, bool from_raw) {
+    // `inside`: the tile lies wholly inside the tensor
+    auto row_body = [&](bool squares, bool from_raw, bool inside) {
+    const std::string& count = inside ? row_inside : row_end;
     std::ostringstream s;
     for (size_t oi = 0; oi < p.outs.size(); oi++)
         if (p.outs[oi].reduce && p.outs[oi].fold_n && !p.outs[oi].fold_m)
@@ -824,6 +833,7 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
     cx.row_part = hoist_rows ? 2 : 0;
     cx.phase = from_raw ? 2 : 0;
     cx.defer_row_varying_only = from_raw;
+    cx.count = count;
     s << emit_exprs(p, cx);
     // outputs
     Shape pst = ir::packed_strides(p.dims);
@@ -842,7 +852,7 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
                 }
                 s << ";\n";
                 if (!(p.dims[n - 1] <= 1 || o.stride[n - 1] == 1)) {
-                    s << "#pragma unroll\nfor (int k = 0; k < NV; k++) st_one(a" << o.arg << " + o + (size_t)k * " << o.stride[n - 1] << "ull, " << v << "[k]);\n}\n";
+                    s << "#pragma unroll\nfor (int k = 0; k < NV; k++) " << (count.empty() ? std::string() : "if (k < " + count + ") ") << "st_one(a" << o.arg << " + o + (size_t)k * " << o.stride[n - 1] << "ull, " << v << "[k]);\n}\n";
                     continue;
                 }
             }
@@ -851,12 +861,14 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
                 s << "#pragma unroll\nfor (int k = 0; k < NV; k++) { const size_t l = o + k; if (" << v
                   << "[k]) atomicOr(a" << o.arg << " + (l >> 5), 1u << (l & 31)); }\n";
             } else {
-                s << "st_vec<NV, " << (streams_out(p.args[o.arg]) ? "true" : "false") << ">(a" << o.arg << " + o, " << v << ");\n";
+                s << (count.empty() ? "st_vec<NV, " : "st_vec_n<NV, ") << (streams_out(p.args[o.arg]) ? "true" : "false") << ">(a" << o.arg << " + o, " << v
+                  << (count.empty() ? "" : ", " + count) << ");\n";
             }
             s << "}\n";
             continue;
         }
         std::string term = v + "[k]";
+        if (guarded && !inside && o.fold_n) term = "(k < " + count + " ? " + term + " : red_identity<" + std::to_string((int)o.rop) + ">())";
         if (o.fold_m && !o.fold_n)
             s << "#pragma unroll\nfor (int k = 0; k < NV; k++) rc" << oi << "[k] = red_op<" << (int)o.rop << ">(rc" << oi
               << "[k], " << term << ");\n";
@@ -922,6 +934,7 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
             lx.row_part = hoist_rows ? 2 : 0;
             lx.phase = 1;
             lx.defer_row_varying_only = true;
+            lx.count = row_inside;
             const std::string issue = emit_exprs(p, lx);
             s << "struct RowRaw {\n" << emit_raw_members(p, NV, true) << "};\n";
             auto name = [](int d) { return d == 0 ? std::string("R") : "R" + std::to_string(d); };
@@ -934,14 +947,15 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
             for (int d = 0; d + 1 < ahead; d++) ahead_tail += name(d) + " = " + name(d + 1) + ";\n";
             ahead_tail += name(ahead - 1) + " = Rn;\n";
         }
-        auto loops = [&](const std::string& body, const std::string& body_from_raw) {
+        auto loops = [&](bool squares) {
+            const std::string body = row_body(squares, false, false);
             if (ragged && few_blocks) {
                 s << head << "const bool ok = col_ok && m < DIM_M;\n" << body << "}\n}\n";
                 return;
             }
             if (ragged) s << "if ((tile_y + 1) * TR <= DIM_M && (tile_x + 1) * (TX * NV) <= DIM_N) {\n";
-            if (pipelined) s << ahead_head << "const bool ok = true;\n" << body_from_raw << "}\n" << ahead_tail << "}\n";
-            else s << head << "const bool ok = true;\n" << body << "}\n}\n";
+            if (pipelined) s << ahead_head << "const bool ok = true;\n" << row_body(squares, true, true) << "}\n" << ahead_tail << "}\n";
+            else s << head << "const bool ok = true;\n" << row_body(squares, false, true) << "}\n}\n";
             if (ragged) s << "} else {\n" << head << "const bool ok = col_ok && m < DIM_M;\n" << body << "}\n}\n}\n";
         };
         // `x.pow_scalar(2.0)` reaches the kernel as Pow with a broadcast 1-element operand. The exponents are read
@@ -953,14 +967,14 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
         std::sort(exps.begin(), exps.end());
         exps.erase(std::unique(exps.begin(), exps.end()), exps.end());
         if (exps.empty()) {
-            loops(row_body(false, false), pipelined ? row_body(false, true) : std::string());
+            loops(false);
         } else {
             s << "bool all_squares = true;\n";
             for (int a : exps) s << "all_squares = all_squares && ld_one(a" << a << ") == 2.0f;\n";
             s << "if (all_squares) {\n";
-            loops(row_body(true, false), pipelined ? row_body(true, true) : std::string());
+            loops(true);
             s << "} else {\n";
-            loops(row_body(false, false), pipelined ? row_body(false, true) : std::string());
+            loops(false);
             s << "}\n";
         }
     }

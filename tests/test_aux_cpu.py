@@ -71,3 +71,23 @@ def test_c3_chain_on_cpu(rows, cols, axis):
         a = got[leaf].astype(np.float64)
         w = w.reshape(-1).astype(np.float64)
         assert np.all(np.abs(a - w) <= 1e-3 * np.maximum(np.abs(w), 1e-6)), (leaf, kernel.description)
+
+
+@pytest.mark.parametrize("shape", [(1, 93, 707), (3, 50, 437), (2, 17, 2003), (1, 8200, 9)])
+def test_rows_of_odd_length_move_as_guarded_vectors(shape):
+    """Vectors at any element's alignment, the last one of a row shorter: values, and reductions in which the columns past
+    a row's end take no part."""
+    g, inputs, outs = all_reductions_graph(list(shape), 11)
+    kernel = ha.TileKernel.auxiliary(g)
+    assert " NV=4 " in kernel.description
+    got = run_tile_kernel_cpu(kernel, inputs, "fused_auxiliary")
+    want = oracle.outputs(g.nodes, inputs)
+    for leaf in outs[:4]:
+        assert np.allclose(got[leaf], want[leaf].reshape(-1), rtol=1e-3, atol=1e-3), (leaf, kernel.description)
+    full = outs[4]
+    assert np.all(np.abs(got[full].astype(np.int32) - want[full].reshape(-1).astype(np.int32)) <= 1)
+
+
+@pytest.mark.parametrize("axis", [1, 2])
+def test_c3_chain_of_odd_rows_on_cpu(axis):
+    test_c3_chain_on_cpu(93, 707, axis)
