@@ -911,6 +911,7 @@ bool mid_tile(const GemmProblem& pr, bool staged, bool fused, Tile* t) {
         t->bm = 64;
         t->wn = 4;
         t->wgs = 2;
+        if (!staged) t->stages = 3;
     } else if (fused) {
         t->bm = 64;
         t->wgs = 3;
@@ -973,6 +974,14 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
             t.bn = 32;
             t.wm = 4;
             t.wn = 1;
+        } else if (!f32 && pr.N <= 64 && pr.M > 64 && pr.split_k == 1 && !pr.conv_b.on && !gathered_by_element) {
+            // ... and the same of fewer rows: tiles as narrow as N, low enough to be several to a CU (a convolution of 25088
+            // pixels into 64 channels, k = 576: 6.6 us with 128x128 tiles, 4.9)
+            t.bm = pr.N <= 32 ? 128 : 64;
+            t.bn = pr.N <= 32 ? 32 : 64;
+            t.wm = pr.N <= 32 ? 4 : 2;
+            t.wn = pr.N <= 32 ? 1 : 2;
+            small = true;
         } else if (!f32 && pr.M <= 32 && pr.M > 16 && pr.N >= 128 && pr.conv_b.on && pr.conv_b.C % epc != 0) {
             // ... and a B operand gathered element by element (the filter gradient of the 7x7 stem on a 3-channel
             // image): the gather is bound by the loads it keeps in flight, so small workgroups, six of which share a
@@ -1040,6 +1049,18 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
             if (pr.M > 64 && pr.N > 64 && ((pr.M + 127) / 128) * ((pr.N + 127) / 128) * pr.batch * pr.siblings * pr.split_k < 128) {
                 t.bm = t.bn = 64;
                 t.wn = 2;
+                // ... and half as wide again, eight waves and three stages, where direct loads feed it and half the CUs still get
+                // one: half the traffic per MFMA for B, twice the waves to issue it, and a second tile in flight while one is
+                // multiplied. 1536x1024x2048 16.3 -> 11.3 us, 1280x1280x1280 10.1 -> 7.9, the 7x7x512 convolution at batch 64
+                // 32.7 -> 28.7, its data gradient 32.8 -> 31.0.
+                if (!f32 && pr.N > 64 && pr.split_k == 1 && !pr.conv_b.on && raw_a0 && raw_b0 && want_direct && (pr.conv_a.on ? pr.conv_a.C % epc == 0 : chunk_a) &&
+                    (pr.b_rows.on || chunk_b) && ((pr.M + 63) / 64) * ((pr.N + 127) / 128) * pr.batch * pr.siblings >= 128) {
+                    t.bn = 128;
+                    t.wn = 4;
+                    t.stages = 3;
+                    t.wgs = 2;
+                    small = false;
+                }
             }
         }
     }
