@@ -33,7 +33,7 @@ bool BlockAllocator::allocate(uint64_t size, uint64_t align, StreamId stream, Bl
             const Block& cand = free_.at(id);
             bool allowed = true;
             for (StreamId s : cand.in_use)
-                allowed = allowed && me && (s == stream || me->ancestors.count(s));
+                allowed = allowed && me && (s == stream || is_ancestor(s, stream, *me));
             if (!allowed) continue;
             const uint64_t offset = cand.start % align ? align - cand.start % align : 0;
             if (offset > cand.size || cand.size - offset < size) continue;
@@ -116,11 +116,21 @@ Block BlockAllocator::remove_free_block(BlockId id) {
 StreamId BlockAllocator::begin_stream(StreamId parent) {
     Stream s;
     auto p = streams_.find(parent);
-    if (parent && p != streams_.end()) {
-        s.ancestors = p->second.ancestors;
-        s.ancestors.insert(parent);
-    }
     const StreamId id = next_stream_++;
+    if (parent && p != streams_.end()) {
+        Chain& c = *p->second.chain;
+        if (c.last == parent) {
+            s.chain = p->second.chain;
+        } else {
+            s.chain = std::make_shared<Chain>();
+            s.chain->before = c.before;
+            for (auto& kv : streams_)
+                if (kv.first <= parent && kv.second.chain == p->second.chain) s.chain->before.insert(kv.first);
+        }
+    } else {
+        s.chain = std::make_shared<Chain>();
+    }
+    s.chain->last = id;
     streams_.emplace(id, std::move(s));
     return id;
 }
@@ -137,7 +147,6 @@ void BlockAllocator::end_stream(StreamId id) {
         block.in_use.erase(id);
         add_free_block(std::move(block));
     }
-    for (auto& kv : streams_) kv.second.ancestors.erase(id);
 }
 
 uint64_t BlockAllocator::free_bytes() const {

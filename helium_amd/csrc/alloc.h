@@ -6,6 +6,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <set>
 #include <unordered_map>
 #include <vector>
@@ -49,10 +50,22 @@ public:
 
 private:
     using BlockId = uint64_t;
+    // Streams that begin one after the other, each with the one before as its parent, form a chain; a stream's ancestors are
+    // its chain's earlier streams and those of the stream the chain branched off from. (A set of ancestors per stream is
+    // copied whenever one begins: a host thread that runs 200 executions ahead of the device paid 12 us per execution.)
+    struct Chain {
+        StreamId last = 0;
+        std::set<StreamId> before;  // ancestors of the chain's first stream
+    };
     struct Stream {
         std::set<BlockId> blocks_in_use;
-        std::set<StreamId> ancestors;
+        std::shared_ptr<Chain> chain;
     };
+    bool is_ancestor(StreamId s, StreamId of, const Stream& me) const {
+        if (s >= of) return me.chain->before.count(s) != 0;
+        auto it = streams_.find(s);
+        return (it != streams_.end() && it->second.chain == me.chain) || me.chain->before.count(s) != 0;
+    }
     void add_free_block(Block block);
     Block remove_free_block(BlockId id);
     std::unordered_map<BlockId, Block> free_;
