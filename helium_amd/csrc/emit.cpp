@@ -31,8 +31,7 @@ typedef _Float16 f16_t;
 #ifndef HE_OPAQUE
 // Hides where a value came from. Negating a just-widened bf16 and narrowing it again makes this compiler (with
 // packed FP32 off) build an integer xor it then cannot select; the barrier keeps the three steps apart.
-__device__ __forceinline__ float he_opaque(float x) { asm volatile("" : "+v"(x)); return x; }
-#define HE_OPAQUE(x) he_opaque(x)
+#define HE_OPAQUE(x) __extension__({ float opaque_ = (x); asm volatile("" : "+v"(opaque_)); opaque_; })
 #endif
 #ifndef HE_FAST_RCP
 #define HE_FAST_RCP(x) __builtin_amdgcn_rcpf(x)

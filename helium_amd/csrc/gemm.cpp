@@ -921,7 +921,7 @@ bool mid_tile(const GemmProblem& pr, bool staged, bool fused, Tile* t) {
     return true;
 }
 
-GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(std::move(prob)) {
+GemmKernel::GemmKernel(GemmProblem prob, const GemmTile* tile) : prob_(std::move(prob)) {
     const GemmProblem& pr = prob_;
     HE_REQUIRE(pr.M > 0 && pr.N > 0 && pr.K > 0 && pr.batch > 0, HE_ERR_INVALID, "empty GEMM");
     HE_REQUIRE(pr.M < (1ll << 31) && pr.N < (1ll << 31) && pr.K < (1ll << 31) &&
@@ -941,8 +941,8 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
     const bool chunk_a = run_a % epc == 0, chunk_b = run_b % epc == 0;
     const bool want_direct = !tuning::get("HELIUM_HIP_GEMM_NO_DIRECT");
     const int esz = 16 / epc;  // bytes per multiplicand
-    if (tiled_like) {
-        const int* v = tiled_like->tile_;
+    if (tile) {
+        const GemmTile& v = *tile;
         t = {v[0], v[1], v[2], v[3], v[4], v[5], 0, v[6]};
     } else if (const char* env = tuning::get("HELIUM_HIP_GEMM_TILE")) {
         int v[7] = {256, 256, 64, 2, 4, 2, 1};
@@ -1161,7 +1161,7 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
                              (int64_t)pr.conv_a.N * pr.conv_a.H * pr.conv_a.W * pr.conv_a.C < (int64_t(1) << 32) &&
                              !tuning::get("HELIUM_HIP_GEMM_NO_CONV_FAST");
     if (!(direct_a && direct_b)) t.stages = 2;  // register staging is double-buffered only
-    else if (!tuning::get("HELIUM_HIP_GEMM_TILE") && small && !tiled_like) {
+    else if (!tuning::get("HELIUM_HIP_GEMM_TILE") && small && !tile) {
         // A grid that leaves CUs idle is bound by the latency of its k-loop: keep as many tiles in flight as LDS holds.
         // With more than one workgroup per CU (a split k range) the LDS is better spent on a second and third
         // workgroup, whose loads hide each other's waits (filter gradient of a 64-channel layer: 66 -> 56 us).
@@ -1174,10 +1174,7 @@ GemmKernel::GemmKernel(GemmProblem prob, const GemmKernel* tiled_like) : prob_(s
     // All direct loads of the next tile are issued at the start of a tile's MFMAs (the round trip needs the whole
     // tile to hide); HELIUM_HIP_GEMM_ISSUE=0 spreads them over the k-steps instead.
     const bool issue_front = tuning::get("HELIUM_HIP_GEMM_ISSUE") ? atoi(tuning::get("HELIUM_HIP_GEMM_ISSUE")) != 0 : true;
-    {
-        const int v[7] = {t.bm, t.bn, t.bk, t.wm, t.wn, t.stages, t.wk};
-        memcpy(tile_, v, sizeof v);
-    }
+    tile_ = {t.bm, t.bn, t.bk, t.wm, t.wn, t.stages, t.wk};
     int nve = std::min(8, tp::pick_nv(pr.epi, 32));
     const int nve_any = std::min(8, tp::pick_nv(pr.epi, 32, true));
     // (rows that are no multiple of 4 elements: guarded vectors, loaded and stored element by element only at a row's end)
@@ -1943,63 +1940,175 @@ std::vector<std::string> macros_of(const std::string& text) {
 }
 }  // namespace
 
-CompositeKernel::CompositeKernel(std::vector<GemmProblem> problems, bool zero_the_rest) {
+void PartsText::add(const GemmKernel& p, const std::vector<std::string>& args) {
+    HE_REQUIRE((!threads || p.threads_ == threads) && p.grid_[1] == 1 && !p.scratch_bytes_needed(), HE_ERR_INTERNAL, "products that cannot share a launch");
+    threads = p.threads_;
+    lds = std::max(lds, p.lds_bytes_);
+    wgs_per_cu = parts ? std::min(wgs_per_cu, p.wgs_per_cu_) : p.wgs_per_cu_;
+    bodies << "#define GEMM_PART 1\nnamespace part_" << parts << " {\n" << p.source() << "}\n";
+    for (auto& name : macros_of(p.source())) bodies << "#undef " << name << "\n";
+    bodies << "#undef GEMM_PART\n";
+    // (whole multiples of 8 blocks: the XCD that a part's tile order counts on is its block number's, part or whole)
+    const uint32_t from = (grid + 7) / 8 * 8;
+    if (from != grid) calls << "if (b < " << from << "u) return;\n";
+    calls << "if (b < " << from + p.grid_[0] << "u) {\npart_" << parts << "::gemm_part(";
+    for (auto& a : args) calls << a << ", ";
+    calls << "lds, b - " << from << "u);\nreturn;\n}\n";
+    grid = from + p.grid_[0];
+    parts++;
+}
+
+void PartsText::add_zeroes(const std::vector<const GemmKernel*>& written, const std::string& out) {
+    // what no part writes: the pixels of the classes that no tap reaches, 16 bytes at a time
+    const GemmProblem& pr = written[0]->problem();
+    const auto& r = pr.out_rows;
+    const tp::Arg& arg = pr.args[pr.map_e[pr.epi.outs[0].arg]];
+    const int64_t row_chunks = pr.N * (dtype_bits(arg.dtype) / 8) / 16, chunks = arg.numel / pr.N * row_chunks;
+    HE_REQUIRE(pr.N * (dtype_bits(arg.dtype) / 8) % 16 == 0 && chunks < (1ll << 31), HE_ERR_UNSUPPORTED, "gradient rows that are no whole 16-byte chunks");
+    const uint32_t blocks = (uint32_t)std::min<int64_t>((chunks + threads - 1) / threads, 2048);
+    calls << "if (b < " << grid + blocks << "u) {\nfor (unsigned i = (b - " << grid << "u) * " << threads << "u + threadIdx.x; i < " << chunks << "u; i += "
+          << (uint64_t)blocks * threads << "u) {\nconst unsigned pixel = i / " << row_chunks << "u, w = pixel % " << r.W << "u, h = pixel / " << r.W << "u % " << r.H
+          << "u;\nbool written = false;\n";
+    for (auto* p : written)
+        calls << "written = written || (h % " << r.sh << "u == " << p->problem().out_rows.a << "u && w % " << r.sw << "u == " << p->problem().out_rows.b << "u);\n";
+    calls << "if (!written) ((zero_chunk_t*)" << out << ")[i] = zero_chunk_t{0u, 0u, 0u, 0u};\n}\nreturn;\n}\n";
+    grid += blocks;
+}
+
+std::string PartsText::text(const std::string& entry, const std::vector<tp::Arg>& args) const {
+    std::ostringstream s;
+    s << bodies.str() << "typedef unsigned zero_chunk_t __attribute__((ext_vector_type(4)));\n#define ALL_WAVES " << threads / 64 << "\n#define WGS_PER_CU " << wgs_per_cu
+      << "\nextern \"C\" __global__ __launch_bounds__(" << threads << ") KERNEL_ATTRS\nvoid " << entry << "(";
+    for (size_t a = 0; a < args.size(); a++)
+        s << (a ? ", " : "") << (args[a].is_output ? "" : "const ") << (args[a].dtype == HE_F32 ? "" : "part_0::") << tp::c_type(args[a].dtype) << "* __restrict__ p" << a;
+    s << ") {\n__shared__ __attribute__((aligned(16))) unsigned char lds[" << lds << "];\nconst unsigned b = blockIdx.x;\n" << calls.str() << "}\n";
+    return s.str();
+}
+
+CompositeKernel::CompositeKernel(std::vector<GemmProblem> problems, bool zero_the_rest) : zero_the_rest_(zero_the_rest) {
     HE_REQUIRE(!problems.empty(), HE_ERR_INTERNAL, "a composite kernel needs a part");
     // The products with the longest k first: their workgroups are the ones that the launch ends with otherwise. All take the
     // tiles of the first, chosen for as many workgroups as there are products.
     std::stable_sort(problems.begin(), problems.end(), [](const GemmProblem& x, const GemmProblem& y) { return x.K > y.K; });
     const int siblings = std::max<int>(2, (int)problems.size());  // (never one: a part is not compiled by itself)
+    PartsText T;
+    std::vector<std::string> names;
+    std::vector<const GemmKernel*> written;
     for (auto& pr : problems) {
         HE_REQUIRE(pr.out_rows.on && pr.batch == 1, HE_ERR_INTERNAL, "the parts of a composite kernel write rows of one tensor");
         pr.siblings = siblings;
-        parts_.emplace_back(new GemmKernel(std::move(pr), parts_.empty() ? nullptr : parts_[0].get()));
+        parts_.emplace_back(new GemmKernel(std::move(pr), parts_.empty() ? nullptr : &parts_[0]->tile_));
+        HE_REQUIRE(parts_.back()->args().size() == args().size(), HE_ERR_INTERNAL, "the parts of a composite kernel differ");
+        for (size_t a = names.size(); a < args().size(); a++) names.push_back("p" + std::to_string(a));
+        T.add(*parts_.back(), names);
+        written.push_back(parts_.back().get());
+        describe_ += "\n" + parts_.back()->describe();
     }
-    const GemmKernel& first = *parts_[0];
-    const std::vector<tp::Arg>& args = first.args();
-    std::ostringstream bodies, s, calls;
-    uint32_t lds = 0;
-    for (size_t k = 0; k < parts_.size(); k++) {
-        GemmKernel& p = *parts_[k];
-        HE_REQUIRE(p.args().size() == args.size() && p.threads_ == first.threads_ && p.grid_[1] == 1, HE_ERR_INTERNAL, "the parts of a composite kernel differ");
-        lds = std::max(lds, p.lds_bytes_);
-        bodies << "#define GEMM_PART 1\nnamespace part_" << k << " {\n" << p.source() << "}\n";
-        for (auto& name : macros_of(p.source())) bodies << "#undef " << name << "\n";
-        bodies << "#undef GEMM_PART\n";
-        // (whole multiples of 8 blocks: the XCD that a part's tile order counts on is its block number's, part or whole)
-        calls << "if (b < " << grid_ + p.grid_[0] << "u) {\n" << "part_" << k << "::gemm_part(";
-        for (size_t a = 0; a < args.size(); a++) calls << "p" << a << ", ";
-        calls << "lds, b - " << grid_ << "u);\nreturn;\n}\n";
-        grid_ = (grid_ + p.grid_[0] + 7) / 8 * 8;
-        if (k + 1 < parts_.size()) calls << "if (b < " << grid_ << "u) return;\n";
-        describe_ += (describe_.empty() ? "" : "\n") + p.describe();
-    }
-    threads_ = first.threads_;
-    if (zero_the_rest) {
-        // what no part writes: the pixels of the classes that no tap reaches, 16 bytes at a time
-        const GemmProblem& pr = first.problem();
-        const auto& r = pr.out_rows;
-        const tp::Arg& out = args[pr.map_e[pr.epi.outs[0].arg]];
-        const int64_t row_chunks = pr.N * (dtype_bits(out.dtype) / 8) / 16, chunks = out.numel / pr.N * row_chunks;
-        HE_REQUIRE(pr.N * (dtype_bits(out.dtype) / 8) % 16 == 0 && chunks < (1ll << 31), HE_ERR_UNSUPPORTED, "gradient rows that are no whole 16-byte chunks");
-        const uint32_t blocks = (uint32_t)std::min<int64_t>((chunks + threads_ - 1) / threads_, 2048);
-        calls << "for (unsigned i = (b - " << grid_ << "u) * " << threads_ << "u + threadIdx.x; i < " << chunks << "u; i += " << (uint64_t)blocks * threads_
-              << "u) {\nconst unsigned pixel = i / " << row_chunks << "u, w = pixel % " << r.W << "u, h = pixel / " << r.W << "u % " << r.H << "u;\nbool written = false;\n";
-        for (auto& p : parts_)
-            calls << "written = written || (h % " << r.sh << "u == " << p->problem().out_rows.a << "u && w % " << r.sw << "u == " << p->problem().out_rows.b << "u);\n";
-        calls << "if (!written) ((zero_chunk_t*)p" << pr.map_e[pr.epi.outs[0].arg] << ")[i] = zero_chunk_t{0u, 0u, 0u, 0u};\n}\n";
-        grid_ += blocks;
-    }
-    s << bodies.str() << "typedef unsigned zero_chunk_t __attribute__((ext_vector_type(4)));\n#define ALL_WAVES " << threads_ / 64 << "\n#define WGS_PER_CU " << first.wgs_per_cu_
-      << "\nextern \"C\" __global__ __launch_bounds__(" << threads_ << ") KERNEL_ATTRS\nvoid fused_matmul_parts(";
-    for (size_t a = 0; a < args.size(); a++)
-        s << (a ? ", " : "") << (args[a].is_output ? "" : "const ") << (args[a].dtype == HE_F32 ? "" : "part_0::") << tp::c_type(args[a].dtype) << "* __restrict__ p" << a;
-    s << ") {\n__shared__ __attribute__((aligned(16))) unsigned char lds[" << lds << "];\nconst unsigned b = blockIdx.x;\n" << calls.str() << "}\n";
-    const std::string text = s.str();
+    const GemmProblem& pr = written[0]->problem();
+    if (zero_the_rest) T.add_zeroes(written, names[pr.map_e[pr.epi.outs[0].arg]]);
+    grid_ = T.grid;
+    threads_ = T.threads;
+    const std::string text = T.text("fused_matmul_parts", args());
     source_ = text;
     // (sources and descriptions one after the other, each introduced by a line that names the part)
     for (auto& p : parts_) source_ += "// ---- part " + std::to_string(&p - &parts_[0]) + " of " + std::to_string(parts_.size()) + "\n" + p->source() + "\n";
-    describe_ = "composite parts=" + std::to_string(parts_.size()) + " zero_first=" + (zero_the_rest ? "1" : "0") + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + "\n" + describe_;
+    describe_ = "composite parts=" + std::to_string(parts_.size()) + " zero_first=" + (zero_the_rest ? "1" : "0") + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + describe_;
     kernel_.reset(new JitKernel(text, "fused_matmul_parts", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));
+}
+
+bool JoinedProducts::can_join(const KernelBase& kernel) {
+    constexpr double kMostWork = 4e9;  // multiply-adds; a larger product does not notice what a launch costs
+    auto small = [](const GemmProblem& pr) { return pr.batch == 1 && (double)pr.M * pr.N * pr.K <= kMostWork; };
+    if (auto* g = dynamic_cast<const GemmKernel*>(&kernel)) return g->problem().split_k == 1 && !g->scratch_bytes_needed() && small(g->problem());
+    if (auto* c = dynamic_cast<const CompositeKernel*>(&kernel)) {
+        for (auto& p : c->parts_)
+            if (!small(p->problem())) return false;
+        return true;
+    }
+    return false;
+}
+
+JoinedProducts::JoinedProducts(const std::vector<std::shared_ptr<KernelBase>>& members) {
+    struct Part {
+        std::unique_ptr<GemmKernel> kernel;
+        size_t member;
+    };
+    std::vector<Part> parts;
+    std::vector<size_t> first_arg;
+    size_t products = 0;
+    for (auto& m : members) {
+        HE_REQUIRE(can_join(*m), HE_ERR_INTERNAL, "a kernel that cannot join others");
+        if (auto* c = dynamic_cast<const CompositeKernel*>(m.get())) products += c->parts_.size();
+        else products++;
+        first_arg.push_back(args_.size());
+        args_.insert(args_.end(), m->args().begin(), m->args().end());
+    }
+    // Each keeps the k groups that it has by itself - the order its sums are made in, and with it every bit of its results -
+    // and takes more waves, or a larger tile of them, where another member's workgroups are larger.
+    uint32_t threads = 0;
+    auto each = [](const KernelBase& m, auto&& f) {
+        if (auto* g = dynamic_cast<const GemmKernel*>(&m)) f(*g);
+        else for (auto& p : dynamic_cast<const CompositeKernel&>(m).parts_) f(*p);
+    };
+    for (auto& m : members) each(*m, [&](const GemmKernel& k) { threads = std::max(threads, k.threads_); });
+    for (size_t m = 0; m < members.size(); m++)
+        each(*members[m], [&](const GemmKernel& k) {
+            GemmTile t = k.tile_;
+            for (uint32_t own = k.threads_; own < threads; own *= 2) {
+                if (t[0] / t[3] > 32) {
+                    t[3] *= 2;
+                } else if (t[1] / t[4] > 32) {
+                    t[4] *= 2;
+                } else {
+                    const bool rows = k.problem().M >= k.problem().N;
+                    t[rows ? 0 : 1] *= 2;
+                    t[rows ? 3 : 4] *= 2;
+                }
+            }
+            if (t != k.tile_) t[5] = 2;
+            GemmProblem pr = k.problem();
+            pr.siblings = std::max<int>(2, (int)products);
+            parts.push_back({std::unique_ptr<GemmKernel>(new GemmKernel(std::move(pr), &t)), m});
+        });
+    // the longest chains of k-tiles first
+    std::stable_sort(parts.begin(), parts.end(), [](const Part& x, const Part& y) {
+        auto chain = [](const GemmKernel& k) { return k.problem().K / k.tile_[2] / k.tile_[6]; };
+        return chain(*x.kernel) > chain(*y.kernel);
+    });
+    PartsText T;
+    for (auto& p : parts) {
+        std::vector<std::string> names;
+        for (size_t a = 0; a < p.kernel->args().size(); a++) names.push_back("p" + std::to_string(first_arg[p.member] + a));
+        T.add(*p.kernel, names);
+        describe_ += "\n" + p.kernel->describe();
+    }
+    for (size_t m = 0; m < members.size(); m++) {
+        auto* c = dynamic_cast<const CompositeKernel*>(members[m].get());
+        if (!c || !c->zero_the_rest_) continue;
+        std::vector<const GemmKernel*> written;
+        for (auto& p : parts)
+            if (p.member == m) written.push_back(p.kernel.get());
+        const GemmProblem& pr = written[0]->problem();
+        T.add_zeroes(written, "p" + std::to_string(first_arg[m] + (size_t)pr.map_e[pr.epi.outs[0].arg]));
+    }
+    // (one round of the chip: beyond that the member with the smallest need of LDS waits for places as large as the largest's - both
+    // gradients of a 1537x1000x777 layer, 608 workgroups of 128 KB, 50 us against 46 one after the other)
+    HE_REQUIRE(T.grid <= 256 * (160 * 1024 / T.lds), HE_ERR_UNSUPPORTED, "products that would not all run at once");
+    grid_ = T.grid;
+    threads_ = T.threads;
+    source_ = T.text("joined_products", args_);
+    describe_ = "joined products=" + std::to_string(parts.size()) + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + describe_;
+    kernel_.reset(new JitKernel(source_, "joined_products", {"-ffp-contract=fast", "-munsafe-fp-atomics"}));
+}
+
+void JoinedProducts::execute(void* const* ptrs, hipStream_t stream) {
+    std::vector<void*> argv(args_.size());
+    for (size_t i = 0; i < argv.size(); i++) {
+        HE_REQUIRE(ptrs[i] != nullptr && ((uintptr_t)ptrs[i] & 15) == 0, HE_ERR_INVALID, "kernel argument %zu is null or not 16-byte aligned", i);
+        argv[i] = (void*)&ptrs[i];
+    }
+    const uint32_t grid[3] = {grid_, 1, 1}, block[3] = {threads_, 1, 1};
+    kernel_->launch(grid, block, 0, stream, argv.data(), true);
 }
 
 void CompositeKernel::execute(void* const* ptrs, hipStream_t stream) {

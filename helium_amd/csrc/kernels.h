@@ -1,9 +1,11 @@
 // Executable kernels built from tile programs: the pointwise/reduction instruction, anchor-less fusion-IR kernels
 // and the fused GEMM.
 #pragma once
+#include <array>
 #include <map>
 #include <mutex>
 #include <memory>
+#include <sstream>
 
 #include "rtc.h"
 #include "tp.h"
@@ -110,7 +112,7 @@ private:
 // helium-playground/src/kernel_generator.rs + templates/matmul.cu).
 struct GemmProblem {
     int64_t batch = 1, M = 0, N = 0, K = 0;
-    int siblings = 1;              // products of about this size in the same launch (CompositeKernel)
+    int siblings = 1;              // products of about this size in the same launch (CompositeKernel, JoinedProducts)
     int mma_dtype = HE_BF16;       // multiplicand type: HE_BF16, HE_F16 or HE_F32
     tp::Program op_a, op_b, epi;   // dims [batch,M,K], [batch,K,N] ([batch,N,K] when b_nk), [batch,M,N]
     // B's source is contiguous along k (a transposed matrix, a convolution filter): its program iterates [batch,N,K],
@@ -169,10 +171,12 @@ int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch);
 // Throws HE_ERR_UNSUPPORTED for an epilogue program the GEMM kernel cannot run.
 void validate_gemm_epilogue(const tp::Program& epi);
 
+using GemmTile = std::array<int, 7>;  // rows, columns, k, waves along rows, along columns, LDS stages, k groups
+
 class GemmKernel : public KernelBase {
 public:
-    // `tiled_like`: take that kernel's tile
-    explicit GemmKernel(GemmProblem prob, const GemmKernel* tiled_like = nullptr);
+    // `tile`: instead of the one that the problem's sizes give
+    explicit GemmKernel(GemmProblem prob, const GemmTile* tile = nullptr);
     const std::vector<tp::Arg>& args() const override { return prob_.args; }
     const std::string& source() const override { return source_; }
     const std::string& describe() const override { return describe_; }
@@ -186,9 +190,11 @@ public:
 
 private:
     friend class CompositeKernel;
+    friend class JoinedProducts;
+    friend struct PartsText;
     void run(void* const* ptrs, hipStream_t stream, float* ws, uint32_t* counters);
     GemmProblem prob_;
-    int tile_[7] = {0};  // rows, columns, k, waves along rows, columns, LDS stages, k groups
+    GemmTile tile_{};
     int wgs_per_cu_ = 1;
     uint32_t lds_bytes_ = 0;
     std::string source_, describe_;
@@ -202,6 +208,16 @@ private:
     std::vector<int> reduce_outs_;  // kernel arguments the reduce launch writes, in its parameter order
     bool reduce_all_args_ = false;  // the reduce launch carries a program and takes every epilogue argument instead
     ReduceScratch scratch_;
+};
+
+// The text of a launch whose blocks are dealt to several products (and to zeroing what the classes of a data gradient leave).
+struct PartsText {
+    std::ostringstream bodies, calls;
+    uint32_t grid = 0, lds = 0, threads = 0;
+    int wgs_per_cu = 1, parts = 0;
+    void add(const GemmKernel& part, const std::vector<std::string>& args);  // `args`: names of its arguments in the launch
+    void add_zeroes(const std::vector<const GemmKernel*>& written, const std::string& out);
+    std::string text(const std::string& entry, const std::vector<tp::Arg>& args) const;
 };
 
 // Several products with one argument list in one launch: the classes of a strided data gradient, each of which writes some
@@ -220,7 +236,31 @@ public:
     bool loaded() const override { return kernel_->loaded(); }
 
 private:
+    friend class JoinedProducts;
     std::vector<std::unique_ptr<GemmKernel>> parts_;  // sources only
+    bool zero_the_rest_;
+    std::string source_, describe_;
+    std::unique_ptr<JitKernel> kernel_;
+    uint32_t grid_ = 0, threads_ = 256;
+};
+
+// Independent products of any kind in one launch (a layer's data and filter gradients): each by itself leaves most of the
+// chip idle while a long chain of k-tiles runs in a few workgroups.
+class JoinedProducts : public KernelBase {
+public:
+    static bool can_join(const KernelBase& kernel);
+    explicit JoinedProducts(const std::vector<std::shared_ptr<KernelBase>>& members);
+    const std::vector<tp::Arg>& args() const override { return args_; }  // the members' one after the other
+    const std::string& source() const override { return source_; }
+    const std::string& describe() const override { return describe_; }
+    void execute(void* const* ptrs, hipStream_t stream) override;
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    size_t scratch_bytes_needed() const override { return 0; }
+    void load() override { kernel_->load(); }
+    bool loaded() const override { return kernel_->loaded(); }
+
+private:
+    std::vector<tp::Arg> args_;
     std::string source_, describe_;
     std::unique_ptr<JitKernel> kernel_;
     uint32_t grid_ = 0, threads_ = 256;

@@ -24,6 +24,7 @@ struct Item {
     std::vector<NodeId> reads, writes;
     uint8_t side = 0;  // Prepared::Side::side
     bool mergeable = false;
+    std::shared_ptr<KernelBase> kernel;  // of several instructions
 };
 
 // Small elementwise launches whose work may share a launch with others': a launch costs the host 2.5 us and the device
@@ -126,6 +127,53 @@ void join_launches(std::vector<Item>* items) {
     *items = std::move(list);
 }
 
+// Joins products that follow each other in the list and do not depend on each other: a layer's data gradient and filter
+// gradient, a block's two convolutions of one activation.
+void join_products(std::vector<Item>* items) {
+    constexpr size_t kMostMembers = 4;
+    std::vector<Item> list;
+    for (Item& it : *items) {
+        const auto joinable = [](const Item& i) {
+            for (auto* instr : i.instrs)
+                if (instr->kind() != plan::InstrKind::Gemm || instr->carried() || !JoinedProducts::can_join(*instr->kernel())) return false;
+            return true;
+        };
+        bool join = !list.empty() && list.back().instrs.size() < kMostMembers && joinable(it) && joinable(list.back());
+        if (join)
+            for (NodeId r : it.reads) join = join && std::find(list.back().writes.begin(), list.back().writes.end(), r) == list.back().writes.end();
+        if (!join) {
+            list.push_back(std::move(it));
+            continue;
+        }
+        Item& group = list.back();
+        group.instrs.push_back(it.instrs[0]);
+        group.reads.insert(group.reads.end(), it.reads.begin(), it.reads.end());
+        group.writes.insert(group.writes.end(), it.writes.begin(), it.writes.end());
+    }
+    items->clear();
+    for (Item& it : list) {
+        if (it.instrs.size() == 1 || it.instrs[0]->kind() != plan::InstrKind::Gemm) {
+            items->push_back(std::move(it));
+            continue;
+        }
+        std::vector<std::shared_ptr<KernelBase>> members;
+        for (auto* i : it.instrs) members.push_back(i->kernel());
+        try {
+            it.kernel = std::make_shared<JoinedProducts>(members);
+            items->push_back(std::move(it));
+        } catch (const Error&) {
+            // no tiles that all of them can take: a launch each, as ever
+            for (auto* i : it.instrs) {
+                Item one;
+                one.instrs = {i};
+                one.reads = i->all_inputs();
+                one.writes = i->all_outputs();
+                items->push_back(std::move(one));
+            }
+        }
+    }
+}
+
 }  // namespace
 
 void build_schedule(Prepared* pr) {
@@ -184,6 +232,9 @@ void build_schedule(Prepared* pr) {
         for (Item& it : items)
             for (NodeId& r : it.reads) r = base(r);
         join_launches(&items);
+        join_products(&items);
+        for (Item& it : items)
+            for (NodeId& r : it.reads) r = base(r);
     } else {
         // The early instructions first, on the side stream, in one launch where they can share it; then the main chain in
         // plan order. A side instruction goes out where the plan has it, and the side instructions that read its results
@@ -239,7 +290,9 @@ void build_schedule(Prepared* pr) {
     for (Item& it : items) {
         Schedule::Launch L;
         L.stream = it.side ? 1 : 0;
-        if (it.instrs.size() > 1) {
+        if (it.kernel) {
+            L.kernel = it.kernel;
+        } else if (it.instrs.size() > 1) {
             std::vector<std::shared_ptr<TileKernel>> members;
             for (auto* i : it.instrs) members.push_back(std::dynamic_pointer_cast<TileKernel>(i->kernel()));
             L.kernel = std::make_shared<JoinedKernel>(std::move(members));
