@@ -6,6 +6,8 @@ import numpy as np
 
 from . import _ffi
 from ._ffi import check, lib
+from . import _native  # (after _ffi: the extension calls the library that it loads)
+from . import device
 from .device import NP_STORAGE, init
 
 _ffi._sig("he_matmul_kernel_create", C.POINTER(C.c_void_p), C.c_void_p, C.POINTER(C.c_uint32), C.c_int)
@@ -38,12 +40,11 @@ def set_option(option, value):
     check(lib.he_backend_set_option(option, int(value)))
 
 
-class Tensor:
-    """TensorStorage: a reference to device storage of `len` elements of `dtype` (Bool: bits)."""
+class Tensor(_native.Tensor):
+    """TensorStorage: a reference to device storage of `len` elements of `dtype` (Bool: bits). Tensor(handle) takes the
+    handle over; free() lets go of it ahead of time."""
 
-    def __init__(self, handle):
-        self.handle = handle
-        self._info = None  # (dtype, len, nbytes, ptr), asked for on first use: a result that is only passed on costs no call
+    _info = None  # (dtype, len, nbytes, ptr), asked for on first use: a result that is only passed on costs no call
 
     def _get(self, i):
         if self._info is None:
@@ -76,17 +77,6 @@ class Tensor:
         out = np.empty(self.nbytes // np.dtype(np_dtype).itemsize, dtype=np_dtype)
         check(lib.he_tensor_download(self.handle, out.ctypes.data_as(C.c_void_p)))
         return out
-
-    def free(self):
-        if self.handle:
-            lib.he_tensor_free(self.handle)
-            self.handle = C.c_void_p()
-
-    def __del__(self):
-        try:
-            self.free()
-        except Exception:
-            pass
 
 
 class Plan:
@@ -149,29 +139,12 @@ class Plan:
 
 def execute_graph(graph, inputs):
     """BackendExt::execute_graph. `inputs`: {input node id: Tensor}. Returns {output node id: Tensor}."""
-    init()
-    n = len(inputs)
-    # array types are cached per size: building a ctypes array type costs more than filling an array
-    in_nodes_t, in_handles_t = _array_types(max(n, 1))
-    nodes = in_nodes_t(*inputs.keys())
-    handles = in_handles_t(*[t.handle for t in inputs.values()])
-    cap = max(1, graph.num_outputs)
-    out_nodes_t, out_handles_t = _array_types(cap)
-    out_nodes = out_nodes_t()
-    out_handles = out_handles_t()
-    count = C.c_int()
-    check(lib.he_execute_graph(graph.handle, nodes, handles, n, out_nodes, out_handles, cap, C.byref(count)))
-    return {out_nodes[i]: Tensor(C.c_void_p(out_handles[i])) for i in range(count.value)}
-
-
-_ARRAY_TYPES = {}
-
-
-def _array_types(n):
-    t = _ARRAY_TYPES.get(n)
-    if t is None:
-        t = _ARRAY_TYPES[n] = (C.c_uint32 * n, C.c_void_p * n)
-    return t
+    if not device._initialised:
+        init()
+    out = _native.execute_graph(graph.handle.value, inputs if isinstance(inputs, dict) else dict(inputs), graph.num_outputs, Tensor)
+    if type(out) is int:
+        check(out)
+    return out
 
 
 def stats():

@@ -6,6 +6,7 @@ host code only.
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -53,6 +54,13 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(tool), flush=True)
     subprocess.check_call(tool)
+    ext = [hipcc, "-x", "c++", *[f for f in flags if f != "-D__HIP_PLATFORM_AMD__"], "-Wno-missing-field-initializers",
+           "-shared", "-I" + sysconfig.get_paths()["include"], "-I" + os.path.join(os.path.dirname(HERE), "include"),
+           os.path.join(CSRC, "python", "native.cpp"), "-o",
+           os.path.join(HERE, "_native" + sysconfig.get_config_var("EXT_SUFFIX")), "-L" + HERE, "-lhelium_hip", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(ext), flush=True)
+    subprocess.check_call(ext)
     return LIB
 
 
