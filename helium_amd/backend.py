@@ -23,6 +23,8 @@ _ffi._sig("he_plan_graph", C.c_void_p, C.POINTER(C.c_void_p))
 _ffi._sig("he_plan_describe_planned", C.c_void_p, restype=C.c_char_p)
 _ffi._sig("he_plan_destroy", C.c_void_p)
 _ffi._sig("he_plan_precompile", C.c_void_p)
+_ffi._sig("he_plan_num_launches", C.c_void_p, C.POINTER(C.c_int))
+_ffi._sig("he_plan_launch_kernel", C.c_void_p, C.c_int, C.POINTER(C.c_void_p))
 _ffi._sig("he_plan_instruction_kernel", C.c_void_p, C.c_int, C.POINTER(C.c_void_p))
 _ffi._sig("he_execute_graph", C.c_void_p, C.POINTER(C.c_uint32), C.POINTER(C.c_void_p), C.c_int, C.POINTER(C.c_uint32),
           C.POINTER(C.c_void_p), C.c_int, C.POINTER(C.c_int))
@@ -127,6 +129,20 @@ class Plan:
     def precompile(self):
         """Compiles the kernels of all instructions (in parallel) into the kernel caches; needs no device."""
         check(lib.he_plan_precompile(self.handle))
+
+    def num_launches(self):
+        """How many launches an execution makes (he_plan_num_launches); 0 when its steps fan out over streams."""
+        n = C.c_int()
+        check(lib.he_plan_num_launches(self.handle, C.byref(n)))
+        return n.value
+
+    def launch_kernel(self, index):
+        """The kernel of the index-th of them (he_plan_launch_kernel), as `kernel` gives an instruction's."""
+        from .kernels import TileKernel
+
+        h = C.c_void_p()
+        check(lib.he_plan_launch_kernel(self.handle, index, C.byref(h)))
+        return TileKernel(h)
 
     def __del__(self):
         try:

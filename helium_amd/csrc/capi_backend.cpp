@@ -1,5 +1,6 @@
 // C ABI of the backend layer: tensors, plans, execute_graph.
 #include <future>
+#include <mutex>
 #include "exec.h"
 
 #include "capi_types.h"
@@ -11,9 +12,37 @@ struct he_plan_s {
     std::shared_ptr<const he::plan::Plan> plan;
     std::shared_ptr<const he::ir::OpGraph> graph;
     std::string text, text_planned;
+    std::mutex mu;  // guards what follows
+    bool precompiled = false;
+    std::shared_ptr<const he::exec::Schedule> schedule;  // of an execution; null before it, and for a plan whose steps fan out
 };
 
 static thread_local he::exec::ExecStats g_last_stats;
+
+// Compiles the kernels the executor would run: its assignment of instructions to streams shapes some of them, and joins others.
+static void precompile(he_plan_t plan) {
+    std::lock_guard<std::mutex> lk(plan->mu);
+    if (plan->precompiled) return;
+    he::exec::Prepared as_executed;
+    as_executed.graph = plan->graph;
+    as_executed.plan = plan->plan;
+    he::exec::assign_streams(&as_executed);
+    std::vector<std::future<void>> jobs;
+    for (auto& step : plan->plan->steps)
+        for (auto& instr : step.instrs)
+            if (!instr->compiled())
+                jobs.push_back(std::async(std::launch::async, [instr] {
+                    try {
+                        instr->precompile();
+                    } catch (const he::Error& e) {
+                        he::fail(e.code, std::string(e.what()) + " (instruction " + instr->describe() + ")");
+                    }
+                }));
+    for (auto& j : jobs) j.get();
+    he::exec::build_schedule(&as_executed);
+    plan->schedule = as_executed.schedule;
+    plan->precompiled = true;
+}
 
 extern "C" {
 
@@ -102,24 +131,25 @@ int he_plan_instruction_kernel(he_plan_t plan, int index, he_tile_kernel_t* kern
 int he_plan_precompile(he_plan_t plan) {
     return he::guard([&] {
         HE_REQUIRE(plan, HE_ERR_INVALID, "bad argument");
-        // the kernels the executor would run: its assignment of instructions to streams shapes some of them, and joins others
-        he::exec::Prepared as_executed;
-        as_executed.graph = plan->graph;
-        as_executed.plan = plan->plan;
-        he::exec::assign_streams(&as_executed);
-        std::vector<std::future<void>> jobs;
-        for (auto& step : plan->plan->steps)
-            for (auto& instr : step.instrs)
-                if (!instr->compiled())
-                    jobs.push_back(std::async(std::launch::async, [instr] {
-                        try {
-                            instr->precompile();
-                        } catch (const he::Error& e) {
-                            he::fail(e.code, std::string(e.what()) + " (instruction " + instr->describe() + ")");
-                        }
-                    }));
-        for (auto& j : jobs) j.get();
-        he::exec::build_schedule(&as_executed);
+        precompile(plan);
+    });
+}
+int he_plan_num_launches(he_plan_t plan, int* launches) {
+    return he::guard([&] {
+        HE_REQUIRE(plan && launches, HE_ERR_INVALID, "bad argument");
+        precompile(plan);
+        *launches = plan->schedule ? (int)plan->schedule->launches.size() : 0;
+    });
+}
+int he_plan_launch_kernel(he_plan_t plan, int index, he_tile_kernel_t* kernel) {
+    return he::guard([&] {
+        HE_REQUIRE(plan && kernel && index >= 0, HE_ERR_INVALID, "bad argument");
+        precompile(plan);
+        HE_REQUIRE(plan->schedule && (size_t)index < plan->schedule->launches.size(), HE_ERR_INVALID, "the plan has no launch %d", index);
+        auto k = std::make_unique<he_tile_kernel_s>();
+        k->k = plan->schedule->launches[index].kernel;
+        HE_REQUIRE(k->k, HE_ERR_INVALID, "launch %d is a permute", index);
+        *kernel = k.release();
     });
 }
 int he_plan_destroy(he_plan_t plan) {

@@ -321,6 +321,13 @@ int he_plan_instruction_kernel(he_plan_t plan, int index, he_tile_kernel_t* kern
 /* Compiles the kernels of every instruction of the plan, in parallel, into the kernel caches: what begin_execute does
  * on first sight of a plan (cuda.rs:98-139, parallel_compile_kernels :262-270). Needs no device. */
 int he_plan_precompile(he_plan_t plan);
+/* The launches of an execution of the plan, in order: small independent instructions share one, so there are fewer of them
+ * than instructions. 0 for a plan whose steps fan out over streams (HE_OPT_STREAM_FAN_OUT) and run step by step.
+ * Compiles what he_plan_precompile compiles. */
+int he_plan_num_launches(he_plan_t plan, int* launches);
+/* The kernel of one of them, as he_plan_instruction_kernel gives an instruction's: the arguments of one that several
+ * instructions share are theirs one after the other. HE_ERR_INVALID for a permute. */
+int he_plan_launch_kernel(he_plan_t plan, int index, he_tile_kernel_t* kernel);
 int he_plan_destroy(he_plan_t plan);
 
 /* BackendExt::execute_graph (backend.rs:40-80): prunes a copy of the graph, takes the cached plan, compiles its

@@ -1,0 +1,63 @@
+"""What an execution launches (schedule.cpp): small independent instructions share launches. The joined kernels run on the
+CPU (tests/cpu_emul.py) against the oracle."""
+import numpy as np
+import pytest
+
+import helium_amd as ha
+from helium_amd.backend import Plan
+from oracle import helium_ir as oracle_ir
+from oracle import numerics as nm
+
+from helpers import run_tile_kernel_cpu
+
+
+class Case:
+    """A graph, its inputs' values in storage form and the kernels that an execution of it launches."""
+
+    def __init__(self, seed=0):
+        self.g, self.host, self.rng = ha.ir.OpGraph(), {}, np.random.default_rng(seed)
+
+    def new(self, shape, dtype="f32"):
+        i = self.g.new_input(list(shape), dtype)
+        self.host[i] = nm.to_storage(self.rng.uniform(-1, 1, shape).astype(np.float32), dtype)
+        return i
+
+    def launches(self):
+        self.g.optimize()
+        self.plan = Plan(self.g)
+        return [self.plan.launch_kernel(i) for i in range(self.plan.num_launches())]
+
+    def check(self, kernels, entries, rel=1e-4):
+        """Runs `kernels` one after the other on the CPU and compares every value that leaves the graph with the oracle's."""
+        pg = self.plan.graph()
+        origin = {n["id"]: n["origin"] for n in pg.nodes}
+        by_id = {n["id"]: n for n in self.g.nodes}
+        val, _ = oracle_ir.evaluate(self.g.nodes, self.host)
+        have = {n["id"]: self.host[origin[n["id"]]] for n in pg.nodes if n["node"] == "input"}
+        made = {}
+        for k, entry in zip(kernels, entries):
+            made.update(run_tile_kernel_cpu(k, {**have, **made}, entry))
+        for node, data in made.items():
+            o = origin[node]
+            want = np.asarray(val[o], dtype=np.float64).reshape(-1)
+            got = nm.from_storage(data, by_id[o]["dtype"], want.shape).astype(np.float64).reshape(-1)
+            tol = 1e-2 if by_id[o]["dtype"] == "bf16" else rel
+            assert (np.abs(got - want) <= tol * np.maximum(np.abs(want), 1.0)).all(), (o, by_id[o], got[:4], want[:4])
+        return made
+
+
+def updates(count, seed=0):
+    """`count` independent elementwise instructions, each of a shape of its own."""
+    c = Case(seed)
+    for k in range(count):
+        c.g.new_output(c.g.change_data_type(c.g.unary(c.new([3 + k, 5 + 7 * k]), "relu"), "bf16"))
+    return c
+
+
+def test_small_instructions_share_a_launch():
+    c = updates(3)
+    kernels = c.launches()
+    assert [k.description.split("\n")[0].split(" grid")[0] for k in kernels] == ["joined members=3"], [k.description for k in kernels]
+    assert len(c.check(kernels, ["joined_kernels"])) == 3
+    with pytest.raises(ha.HeliumError, match="no launch 1"):
+        c.plan.launch_kernel(1)
