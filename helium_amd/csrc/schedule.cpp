@@ -86,7 +86,8 @@ void join_launches(std::vector<Item>* items) {
                 for (size_t i : waiting) {
                     if ((due[i] <= pos) != (pass == 0)) continue;
                     const size_t more = (*items)[i].reads.size() + (*items)[i].writes.size();
-                    if (ready(i) && members.size() < kMostMembers && args + more <= kMostArgs) {
+                    // (one of more arguments than that goes out alone)
+                    if (ready(i) && members.size() < kMostMembers && (members.empty() || args + more <= kMostArgs)) {
                         members.push_back(i);
                         args += more;
                     } else {

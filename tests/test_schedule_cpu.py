@@ -61,3 +61,21 @@ def test_small_instructions_share_a_launch():
     assert len(c.check(kernels, ["joined_kernels"])) == 3
     with pytest.raises(ha.HeliumError, match="no launch 1"):
         c.plan.launch_kernel(1)
+
+
+@pytest.mark.parametrize("terms", [159, 160, 400])
+def test_an_instruction_of_many_arguments_goes_out_alone(terms):
+    """A small sum of as many tensors as a shared launch takes arguments, or more, beside instructions that share one."""
+    c = Case(terms)
+    total = c.new([8, 8])
+    for _ in range(terms - 1):
+        total = c.g.binary(total, c.new([8, 8]), "add")
+    c.g.new_output(total)
+    for k in range(3):
+        c.g.new_output(c.g.unary(c.new([5, 3 + k]), "neg"))
+    kernels = c.launches()
+    members = sorted(len(k.args) for k in kernels)
+    assert members == [6, terms + 1], [k.description for k in kernels]
+    kernels.sort(key=lambda k: len(k.args))
+    made = c.check(kernels, ["joined_kernels", "pointwise_kernel"], rel=1e-5 * terms)
+    assert len(made) == 4
