@@ -767,17 +767,21 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
     const bool any_ticket = L.ws_counters > 0;
     if (any_ws) s << ", float* wsf, u32* wsc";
     s << ") {\n";
-    if (any_col && TY > 1) s << "__shared__ float col_red[TY * TX * NV];\n";
-    if (any_scalar) s << "__shared__ float blk_red[" << threads / 64 << "];\n";
+    auto shared = [&](const char* type, const char* name, const std::string& dims, size_t count) {
+        L.shared.push_back({type, name, dims, count * 4});
+        s << L.shared.back().declaration();
+    };
+    if (any_col && TY > 1) shared("float", "col_red", "[TY * TX * NV]", (size_t)TY * TX * NV);
+    if (any_scalar) shared("float", "blk_red", strfmt("[%d]", threads / 64), threads / 64);
     // rows that one block spans with two or four waves: the waves' parts of a row meet in LDS (two sets taking turns, so
     // one barrier per row is enough), and no atomics - and no fill launch ahead of the kernel - are needed
     const bool rows_meet_in_lds = gx == 1 && TX > 64 && !tuning::get("HELIUM_HIP_NO_ROW_LDS");
     if (rows_meet_in_lds) {
         size_t row_outs = 0;
         for (auto& o : p.outs) row_outs += o.reduce && o.fold_n && !o.fold_m;
-        if (row_outs) s << "__shared__ float row_red[" << row_outs << "][2][" << threads / 64 << "];\n";
+        if (row_outs) shared("float", "row_red", strfmt("[%zu][2][%d]", row_outs, threads / 64), row_outs * 2 * (threads / 64));
     }
-    if (any_ticket) s << "__shared__ u32 ticket_s[" << p.outs.size() << "];\n";
+    if (any_ticket) shared("u32", "ticket_s", strfmt("[%zu]", p.outs.size()), p.outs.size());
     s << "u32 t = blockIdx.x;\nconst u32 tile_x = t % " << gx << "u; t /= " << gx << "u;\nconst u32 tile_y = t % " << gy
       << "u; t /= " << gy << "u;\nconst u32 b = t;\n";
     {

@@ -154,9 +154,12 @@ void TileKernel::run(void* const* ptrs, hipStream_t stream, ReduceScratch::Buf w
 
 JoinedKernel::JoinedKernel(const std::vector<std::shared_ptr<TileKernel>>& members) {
     HE_REQUIRE(!members.empty(), HE_ERR_INTERNAL, "a joined kernel needs a member");
-    // A member's text is its own kernel made a function: it is told its block, and its constants end with it.
+    // A member's text is its own kernel made a function: it is told its block, and its constants end with it. Its LDS arrays
+    // lie in one buffer that all members share (a block runs one of them): arrays of their own would be charged to every
+    // block as a sum, which 24 column reductions of 8 KB each take beyond what a CU has.
     const std::string head = "extern \"C\" __global__ __launch_bounds__(256) void ", block = "blockIdx.x";
     const tp::PointwiseLaunch& first = members[0]->launch_info();
+    size_t lds = 0;
     std::ostringstream s, calls, params;
     s << first.source.substr(0, first.prelude_bytes);
     for (size_t k = 0; k < members.size(); k++) {
@@ -166,12 +169,21 @@ JoinedKernel::JoinedKernel(const std::vector<std::shared_ptr<TileKernel>>& membe
         const size_t at = text.find(head);
         HE_REQUIRE(at != std::string::npos, HE_ERR_INTERNAL, "unexpected kernel text");
         const size_t paren = text.find('(', at + head.size());
-        text.replace(at, paren + 1 - at, "static __device__ __forceinline__ void member_" + std::to_string(k) + "(const u32 member_block, ");
+        text.replace(at, paren + 1 - at, "static __device__ __forceinline__ void member_" + std::to_string(k) + "(const u32 member_block, unsigned char* const lds, ");
+        size_t taken = 0;
+        for (const auto& a : L.shared) {
+            const std::string declared = a.declaration(), type = a.type + " (*)" + a.dims;
+            const size_t where = text.find(declared);
+            HE_REQUIRE(where != std::string::npos, HE_ERR_INTERNAL, "unexpected kernel text");
+            text.replace(where, declared.size(), a.type + " (&" + a.name + ")" + a.dims + " = *(" + type + ")(lds + " + std::to_string(taken) + ");\n");
+            taken += (a.bytes + 15) / 16 * 16;
+        }
+        lds = std::max(lds, taken);
         for (size_t b = text.find(block); b != std::string::npos; b = text.find(block, b)) text.replace(b, block.size(), "member_block");
         s << text << "#undef NV\n#undef TX\n#undef TY\n#undef RPT\n#undef TR\n#undef DIM_N\n#undef DIM_M\n";
         calls << (k ? "else " : "");
         if (k + 1 < members.size()) calls << "if (blockIdx.x < " << grid_ + L.grid << "u) ";
-        calls << "member_" << k << "(blockIdx.x - " << grid_ << "u";
+        calls << "member_" << k << "(blockIdx.x - " << grid_ << "u, lds";
         for (const tp::Arg& a : members[k]->args()) {
             params << (args_.empty() ? "" : ", ") << (a.is_output ? "" : "const ") << tp::c_type(a.dtype) << "* __restrict__ p" << args_.size();
             calls << ", p" << args_.size();
@@ -183,9 +195,12 @@ JoinedKernel::JoinedKernel(const std::vector<std::shared_ptr<TileKernel>>& membe
         describe_ += (k ? "\n" : "") + L.describe;
     }
     threads_ = first.threads;
-    s << head << "joined_kernels(" << params.str() << ") {\n" << calls.str() << "}\n";
+    s << head << "joined_kernels(" << params.str() << ") {\n";
+    if (lds) s << "__shared__ __attribute__((aligned(16))) unsigned char lds[" << lds << "];\n";
+    else s << "unsigned char* const lds = nullptr;\n";
+    s << calls.str() << "}\n";
     source_ = s.str();
-    describe_ = "joined members=" + std::to_string(members.size()) + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + "\n" + describe_;
+    describe_ = "joined members=" + std::to_string(members.size()) + " grid=" + std::to_string(grid_) + " threads=" + std::to_string(threads_) + " lds=" + std::to_string(lds) + "\n" + describe_;
     kernel_.reset(new JitKernel(source_, "joined_kernels", first.options));
 }
 

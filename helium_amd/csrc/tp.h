@@ -133,6 +133,13 @@ bool attach_post(Program* main, const Program& post);
 struct PointwiseLaunch {
     std::string source, entry;
     size_t prelude_bytes = 0;  // of `source`, ahead of what is this kernel's own
+    // The LDS arrays that the kernel (not its fold launch) declares, as they stand in `source`.
+    struct Shared {
+        std::string type, name, dims;
+        size_t bytes;
+        std::string declaration() const { return "__shared__ " + type + " " + name + dims + ";\n"; }
+    };
+    std::vector<Shared> shared;
     uint32_t grid = 1, threads = 256;
     int nv = 1, tx = 1, ty = 1, rpt = 1;
     // Outputs that must be filled before the launch: (argument index, 32-bit fill pattern).

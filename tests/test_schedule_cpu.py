@@ -1,5 +1,7 @@
 """What an execution launches (schedule.cpp): small independent instructions share launches. The joined kernels run on the
 CPU (tests/cpu_emul.py) against the oracle."""
+import re
+
 import numpy as np
 import pytest
 
@@ -79,3 +81,38 @@ def test_an_instruction_of_many_arguments_goes_out_alone(terms):
     kernels.sort(key=lambda k: len(k.args))
     made = c.check(kernels, ["joined_kernels", "pointwise_kernel"], rel=1e-5 * terms)
     assert len(made) == 4
+
+
+def reductions(count, shape, dtype, seed=0):
+    """`count` column reductions (a block's part of each meets in LDS) that differ in their sizes."""
+    c = Case(seed)
+    for k in range(count):
+        c.g.new_output(c.g.reduce(c.g.swap_dims(c.new([shape[0], shape[1], shape[2] - 8 * k], dtype), 1, 2), "mean", 1))
+    return c
+
+
+@pytest.mark.parametrize("count,shape,dtype", [(24, (64, 32, 2048), "bf16"), (24, (128, 32, 1024), "bf16"), (5, (64, 32, 1024), "f32")])
+def test_a_joined_kernel_takes_the_lds_of_its_largest_member(count, shape, dtype):
+    c = reductions(count, shape, dtype)
+    kernels = c.launches()
+    assert len(kernels) == 1 and len(kernels[0].args) == 2 * count, [k.description for k in kernels]
+    own = [c.plan.kernel(i).source for i in range(count)]
+    per_thread = max(int(re.search(r"#define NV (\d+)", s).group(1)) for s in own)
+    assert all("__shared__ float col_red[TY * TX * NV]" in s for s in own)
+    assert f" lds={256 * per_thread * 4}\n" in kernels[0].description and kernels[0].source.count("__shared__") == 1, kernels[0].description
+
+
+def test_members_with_lds_of_their_own_share_one_buffer():
+    """Column reductions of two widths, rows that meet in LDS, a sum over everything, and members without any."""
+    c = Case(7)
+    g = c.g
+    g.new_output(g.reduce(g.swap_dims(c.new([64, 32, 2048], "bf16"), 1, 2), "mean", 1))
+    g.new_output(g.reduce(g.swap_dims(c.new([33, 31, 2000]), 1, 2), "max", 1))
+    g.new_output(g.reduce(c.new([9, 700]), "sum", 1))
+    g.new_output(g.reduce(g.unary(c.new([4, 120]), "neg"), "sum", 2))
+    g.new_output(g.unary(c.new([5, 7]), "exp"))
+    kernels = c.launches()
+    assert len(kernels) == 1 and kernels[0].source.count("__shared__") == 1, [k.description for k in kernels]
+    for name in ("col_red", "row_red", "blk_red"):
+        assert f"(&{name})" in kernels[0].source, name
+    assert len(c.check(kernels, ["joined_kernels"])) == 5
