@@ -27,6 +27,15 @@ struct Item {
     std::shared_ptr<KernelBase> kernel;  // of several instructions
 };
 
+Item item_of(const plan::Instr& instr, uint8_t side) {
+    Item it;
+    it.instrs = {&instr};
+    it.reads = instr.all_inputs();
+    it.writes = instr.all_outputs();
+    it.side = side;
+    return it;
+}
+
 // Small elementwise launches whose work may share a launch with others': a launch costs the host 2.5 us and the device
 // about as much, whatever it does. (Larger ones gain nothing from company, and moving them keeps their operands alive.)
 bool is_mergeable(const plan::Instr& instr) {
@@ -125,7 +134,22 @@ void join_launches(std::vector<Item>* items) {
         out[i] = 1;
     }
     flush(n);
-    *items = std::move(list);
+    // ---- their kernels; a group whose kernel does not compile goes out as its members' own, which have been compiled
+    items->clear();
+    for (Item& it : list) {
+        if (it.instrs.size() < 2) {
+            items->push_back(std::move(it));
+            continue;
+        }
+        std::vector<std::shared_ptr<TileKernel>> members;
+        for (auto* i : it.instrs) members.push_back(std::dynamic_pointer_cast<TileKernel>(i->kernel()));
+        try {
+            it.kernel = std::make_shared<JoinedKernel>(members);
+            items->push_back(std::move(it));
+        } catch (const Error&) {
+            for (auto* i : it.instrs) items->push_back(item_of(*i, it.side));
+        }
+    }
 }
 
 // Joins products that follow each other in the list and do not depend on each other: a layer's data gradient and filter
@@ -164,13 +188,7 @@ void join_products(std::vector<Item>* items) {
             items->push_back(std::move(it));
         } catch (const Error&) {
             // no tiles that all of them can take: a launch each, as ever
-            for (auto* i : it.instrs) {
-                Item one;
-                one.instrs = {i};
-                one.reads = i->all_inputs();
-                one.writes = i->all_outputs();
-                items->push_back(std::move(one));
-            }
+            for (auto* i : it.instrs) items->push_back(item_of(*i, it.side));
         }
     }
 }
@@ -200,14 +218,6 @@ void build_schedule(Prepared* pr) {
     std::sort(S.inputs.begin(), S.inputs.end(), [](const Schedule::Named& a, const Schedule::Named& b) { return a.node < b.node; });
     // ---- launches in the order they go out
     std::vector<Item> items;
-    auto item_of = [&](const plan::Instr& instr, uint8_t side) {
-        Item it;
-        it.instrs = {&instr};
-        it.reads = instr.all_inputs();
-        it.writes = instr.all_outputs();
-        it.side = side;
-        return it;
-    };
     std::map<NodeId, NodeId> view_of;
     auto base = [&](NodeId n) {
         for (auto it = view_of.find(n); it != view_of.end(); it = view_of.find(n)) n = it->second;
@@ -293,10 +303,6 @@ void build_schedule(Prepared* pr) {
         L.stream = it.side ? 1 : 0;
         if (it.kernel) {
             L.kernel = it.kernel;
-        } else if (it.instrs.size() > 1) {
-            std::vector<std::shared_ptr<TileKernel>> members;
-            for (auto* i : it.instrs) members.push_back(std::dynamic_pointer_cast<TileKernel>(i->kernel()));
-            L.kernel = std::make_shared<JoinedKernel>(std::move(members));
         } else if (it.instrs[0]->kind() == plan::InstrKind::Permute) {
             L.permute = it.instrs[0]->permute();
             L.args = {slot(it.instrs[0]->inputs()[0]), slot(it.instrs[0]->outputs()[0])};

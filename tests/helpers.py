@@ -123,3 +123,25 @@ def assert_storage_close(got, want, dtype, what="", max_ulps=2, reduce_rel=None)
         bad = np.flatnonzero(~ok.reshape(-1))[:5]
         raise AssertionError(f"{what}: {(~ok).sum()} of {ok.size} elements differ, e.g. at {bad}: got "
                              f"{np.asarray(got).reshape(-1)[bad]} want {np.asarray(want).reshape(-1)[bad]}")
+
+
+# ---- the package with another kernel compiler --------------------------------------------------------------------
+def run_with_compiler(tmp_path, script, code, **env):
+    """Runs Python text in a process of its own, with a copy of the package whose kernel compiler (the program beside the
+    library) is the shell text `script`; $REAL there is the real one. Returns the finished process."""
+    import os
+    import shutil
+    import subprocess
+    import sys
+
+    import helium_amd
+
+    here = os.path.dirname(helium_amd.__file__)
+    there = tmp_path / "package" / "helium_amd"
+    if not there.exists():
+        shutil.copytree(here, there, ignore=shutil.ignore_patterns("csrc", "build", "_kcache", "__pycache__", "helium_rtc"))
+    compiler = there / "helium_rtc"
+    compiler.write_text("#!/bin/sh\nREAL=%s\n%s\n" % (os.path.join(here, "helium_rtc"), script))
+    compiler.chmod(0o755)
+    return subprocess.run([sys.executable, "-c", "import sys\nsys.path.insert(0, %r)\n%s" % (str(tmp_path / "package"), code)],
+                          env={**os.environ, "HELIUM_HIP_CACHE_DIR": "off", **env}, capture_output=True, text=True, timeout=300)

@@ -10,7 +10,7 @@ from helium_amd.backend import Plan
 from oracle import helium_ir as oracle_ir
 from oracle import numerics as nm
 
-from helpers import run_tile_kernel_cpu
+from helpers import run_tile_kernel_cpu, run_with_compiler
 
 
 class Case:
@@ -116,3 +116,18 @@ def test_members_with_lds_of_their_own_share_one_buffer():
     for name in ("col_red", "row_red", "blk_red"):
         assert f"(&{name})" in kernels[0].source, name
     assert len(c.check(kernels, ["joined_kernels"])) == 5
+
+
+def test_a_join_that_does_not_compile_leaves_its_members_a_launch_each(tmp_path):
+    code = """
+import helium_amd as ha
+from helium_amd.backend import Plan
+g = ha.ir.OpGraph()
+for k in range(4):
+    g.new_output(g.unary(g.new_input([3, 5 + k], "f32"), "relu"))
+plan = Plan(g)
+print(sorted(len(plan.launch_kernel(i).args) for i in range(plan.num_launches())))
+"""
+    refuses = run_with_compiler(tmp_path, 'if [ "$1" = joined_kernels ]; then printf "eno registers left"; else exec "$REAL" "$@"; fi', code)
+    assert refuses.stdout.split("\n")[0] == "[2, 2, 2, 2]", refuses.stdout + refuses.stderr
+    assert run_with_compiler(tmp_path, 'exec "$REAL" "$@"', code).stdout.split("\n")[0] == "[8]"
