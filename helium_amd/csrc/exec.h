@@ -164,6 +164,8 @@ struct Prepared {
         return own;
     }
 };
+// Whether the instruction's launch can be shared with others' (its kernel is made if it is not there yet).
+bool can_share_launch(const plan::Instr& instr);
 // Builds pr->schedule, joined kernels included (compiled, not loaded: needs no device).
 void build_schedule(Prepared* pr);
 using NamedTensors = std::vector<std::pair<NodeId, TensorRef>>;

@@ -9,6 +9,18 @@
 
 namespace he::exec {
 
+// Small elementwise launches whose work may share a launch with others': a launch costs the host 2.5 us and the device
+// about as much, whatever it does. (Larger ones gain nothing from company, and moving them keeps their operands alive.)
+bool can_share_launch(const plan::Instr& instr) {
+    constexpr size_t kMostBytes = 32u << 20;
+    if (instr.kind() != plan::InstrKind::Pointwise) return false;
+    const auto kernel = std::dynamic_pointer_cast<TileKernel>(instr.kernel());
+    if (!kernel || !kernel->can_join()) return false;
+    size_t bytes = 0;
+    for (const tp::Arg& a : kernel->args()) bytes += storage_bytes(a.dtype, (size_t)a.numel);
+    return bytes <= kMostBytes;
+}
+
 namespace {
 
 // An instruction that only renames a shape: its result is its operand's storage.
@@ -34,18 +46,6 @@ Item item_of(const plan::Instr& instr, uint8_t side) {
     it.writes = instr.all_outputs();
     it.side = side;
     return it;
-}
-
-// Small elementwise launches whose work may share a launch with others': a launch costs the host 2.5 us and the device
-// about as much, whatever it does. (Larger ones gain nothing from company, and moving them keeps their operands alive.)
-bool is_mergeable(const plan::Instr& instr) {
-    constexpr size_t kMostBytes = 32u << 20;
-    if (instr.kind() != plan::InstrKind::Pointwise) return false;
-    const auto kernel = std::dynamic_pointer_cast<TileKernel>(instr.kernel());
-    if (!kernel || !kernel->can_join()) return false;
-    size_t bytes = 0;
-    for (const tp::Arg& a : kernel->args()) bytes += storage_bytes(a.dtype, (size_t)a.numel);
-    return bytes <= kMostBytes;
 }
 
 // Joins launches of a one-stream list. Each mergeable launch may run anywhere between the last launch that makes what it
@@ -237,7 +237,7 @@ void build_schedule(Prepared* pr) {
             for (auto& instr : step.instrs) {
                 if (instr->absorbed() || is_view(*instr, g)) continue;
                 Item it = item_of(*instr, 0);
-                it.mergeable = is_mergeable(*instr);
+                it.mergeable = can_share_launch(*instr);
                 items.push_back(std::move(it));
             }
         for (Item& it : items)
@@ -257,7 +257,7 @@ void build_schedule(Prepared* pr) {
             issued[i] = 1;
             if (is_view(*side.order[i], g)) continue;
             Item it = item_of(*side.order[i], 2);
-            it.mergeable = is_mergeable(*side.order[i]);
+            it.mergeable = can_share_launch(*side.order[i]);
             early.push_back(std::move(it));
         }
         for (Item& it : early)

@@ -65,6 +65,35 @@ def test_small_instructions_share_a_launch():
         c.plan.launch_kernel(1)
 
 
+@pytest.mark.parametrize("count,members", [(8, [8]), (12, [12]), (24, [24]), (25, [24, 1]), (30, [24, 6]), (49, [24, 24, 1])])
+def test_a_step_of_many_small_instructions_shares_launches(count, members):
+    """However many there are, as many to a launch as one takes: such a step does not fan out over streams."""
+    c = updates(count, seed=count)
+    kernels = c.launches()
+    assert [len(k.args) for k in kernels] == [2 * m for m in members], [k.description for k in kernels]
+    assert len(c.check(kernels, ["joined_kernels" if m > 1 else "pointwise_kernel" for m in members])) == count
+
+
+def test_a_group_that_takes_too_many_arguments_is_split():
+    c = Case(20)
+    for k in range(10):  # 20 arguments each: a launch takes 160
+        total = c.new([4, 4 + k])
+        for _ in range(18):
+            total = c.g.binary(total, c.new([4, 4 + k]), "add")
+        c.g.new_output(total)
+    kernels = c.launches()
+    assert [len(k.args) for k in kernels] == [160, 40], [k.description for k in kernels]
+    assert len(c.check(kernels, ["joined_kernels"] * 2)) == 10
+
+
+def test_a_step_of_larger_instructions_fans_out():
+    """2 MB each, as many as fan out over streams (HE_OPT_STREAM_FAN_OUT): no launch list."""
+    c = Case()
+    for _ in range(16):
+        c.g.new_output(c.g.unary(c.g.unary(c.g.new_input([512, 512], "f32"), "exp"), "relu"))
+    assert c.launches() == []
+
+
 @pytest.mark.parametrize("terms", [159, 160, 400])
 def test_an_instruction_of_many_arguments_goes_out_alone(terms):
     """A small sum of as many tensors as a shared launch takes arguments, or more, beside instructions that share one."""
