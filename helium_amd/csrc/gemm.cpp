@@ -1875,7 +1875,7 @@ void GemmKernel::execute(void* const* ptrs, hipStream_t stream) {
 }
 
 void GemmKernel::execute_in_scratch(void* const* ptrs, hipStream_t stream, void* scratch, size_t scratch_bytes) {
-    HE_REQUIRE(loaded(), HE_ERR_INVALID, "the kernel's code objects are not loaded on this device yet");
+    require_loaded();
     const size_t need = scratch_bytes_needed();
     HE_REQUIRE(need <= scratch_bytes, HE_ERR_INVALID,
                "the kernel needs %zu bytes of scratch for its partial results, the buffer holds %zu", need, scratch_bytes);
@@ -2208,7 +2208,7 @@ void RepackedConvKernel::execute(void* const* ptrs, hipStream_t stream) {
 }
 
 void RepackedConvKernel::execute_in_scratch(void* const* ptrs, hipStream_t stream, void* scratch, size_t scratch_bytes) {
-    HE_REQUIRE(loaded(), HE_ERR_INVALID, "the kernel's code objects are not loaded on this device yet");
+    require_loaded();
     HE_REQUIRE(scratch_bytes_needed() <= scratch_bytes, HE_ERR_INVALID,
                "the kernel needs %zu bytes of scratch for its repacked operands and partial results, the buffer holds %zu", scratch_bytes_needed(), scratch_bytes);
     HE_REQUIRE(scratch && ((uintptr_t)scratch & 255) == 0, HE_ERR_INVALID, "scratch buffer missing or not 256-byte aligned");

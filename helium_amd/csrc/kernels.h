@@ -33,6 +33,9 @@ public:
     // Loads every code object of the kernel onto the current device.
     virtual void load() = 0;
     virtual bool loaded() const = 0;
+
+protected:
+    void require_loaded() const { HE_REQUIRE(loaded(), HE_ERR_INVALID, "the kernel's code objects are not loaded on this device yet"); }
 };
 
 // Loads the fill kernel's code object (fill_buffers otherwise loads it on its first use).
@@ -95,7 +98,10 @@ public:
     const std::string& source() const override { return source_; }
     const std::string& describe() const override { return describe_; }
     void execute(void* const* ptrs, hipStream_t stream) override;
-    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override {
+        require_loaded();
+        execute(ptrs, stream);
+    }
     size_t scratch_bytes_needed() const override { return 0; }
     void load() override { kernel_->load(); }
     bool loaded() const override { return kernel_->loaded(); }
@@ -230,7 +236,10 @@ public:
     const std::string& source() const override { return source_; }  // of the launch, then of each part by itself
     const std::string& describe() const override { return describe_; }
     void execute(void* const* ptrs, hipStream_t stream) override;
-    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override {
+        require_loaded();
+        execute(ptrs, stream);
+    }
     size_t scratch_bytes_needed() const override { return 0; }
     void load() override { kernel_->load(); }
     bool loaded() const override { return kernel_->loaded(); }
@@ -254,7 +263,10 @@ public:
     const std::string& source() const override { return source_; }
     const std::string& describe() const override { return describe_; }
     void execute(void* const* ptrs, hipStream_t stream) override;
-    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override { execute(ptrs, stream); }
+    void execute_in_scratch(void* const* ptrs, hipStream_t stream, void*, size_t) override {
+        require_loaded();
+        execute(ptrs, stream);
+    }
     size_t scratch_bytes_needed() const override { return 0; }
     void load() override { kernel_->load(); }
     bool loaded() const override { return kernel_->loaded(); }

@@ -104,7 +104,7 @@ bool TileKernel::loaded() const {
 }
 
 void TileKernel::execute_in_scratch(void* const* ptrs, hipStream_t stream, void* scratch, size_t scratch_bytes) {
-    HE_REQUIRE(loaded(), HE_ERR_INVALID, "the kernel's code objects are not loaded on this device yet");
+    require_loaded();
     const size_t need = scratch_bytes_needed();
     HE_REQUIRE(need <= scratch_bytes, HE_ERR_INVALID,
                "the kernel needs %zu bytes of scratch for its partial results, the buffer holds %zu", need, scratch_bytes);

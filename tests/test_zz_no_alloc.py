@@ -78,3 +78,59 @@ def test_a_kernel_that_needs_more_scratch_is_refused(gpu):
     dummy = [ha.DeviceBuffer(256) for _ in k.args]
     with pytest.raises(ha.HeliumError, match="allocation-free entry point holds"):
         k.execute_noalloc(dummy)
+
+
+def _strided_data_gradient():
+    g = ha.ir.OpGraph()
+    params = {"in_channels": 16, "out_channels": 32, "kernel_size": [3, 3], "stride": [2, 2]}
+    dy, w = g.new_input([2, 6, 6, 32], "bf16"), g.new_input([32, 3, 3, 16], "bf16")
+    g.new_output(g.conv_backward_data(dy, w, params, [14, 14]))
+    return g, "composite"
+
+
+def _small_updates():
+    g = ha.ir.OpGraph()
+    for k in range(3):
+        g.new_output(g.unary(g.new_input([5, 7 + k], "f32"), "relu"))
+    return g, "joined members=3"
+
+
+def _two_products():
+    g = ha.ir.OpGraph()
+    for _ in range(2):
+        a, b = g.new_input([96, 64], "bf16"), g.new_input([64, 80], "bf16")
+        g.new_output(g.matmul(a, b, "bf16_f32"))
+    return g, "joined products=2"
+
+
+@pytest.mark.parametrize("graph", [_strided_data_gradient, _small_updates, _two_products])
+def test_a_kernel_of_several_parts_is_refused_until_it_is_loaded(gpu, graph):
+    """The allocation-free entry point loads no code object: a launch of a plan, whose code is loaded by its first ordinary
+    execution, is refused before that and gives the same results after it."""
+    from helium_amd.backend import Plan
+
+    g, described = graph()
+    plan = Plan(g)
+    assert plan.num_launches() == 1, plan.text
+    k = plan.launch_kernel(0)
+    assert k.description.startswith(described), k.description
+    rng = np.random.default_rng(3)
+    bufs = []
+    for a in k.args:
+        values = rng.uniform(-1, 1, a["numel"]).astype(np.float32)
+        values = values if a["dtype"] == "f32" else (values.view(np.uint32) >> 16).astype(np.uint16)
+        bufs.append((ha.DeviceBuffer.from_numpy(values), a, values.dtype))
+
+    def run(execute):
+        for b, a, _ in bufs:
+            if a["is_output"]:
+                b.fill_u8(0xA5)
+        execute([b for b, _, _ in bufs])
+        return [b.to_numpy(dt) for b, a, dt in bufs if a["is_output"]]
+
+    with pytest.raises(ha.HeliumError, match="not loaded") as refused:
+        k.execute_noalloc([b for b, _, _ in bufs])
+    assert refused.value.code == 1  # HE_ERR_INVALID
+    want = run(k.execute)
+    for got, w in zip(run(k.execute_noalloc), want):
+        assert np.array_equal(got, w)
