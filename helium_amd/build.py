@@ -48,8 +48,9 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(link), flush=True)
     subprocess.check_call(link)
-    # (an old-style run path comes before the environment's: the compiler of this toolchain, whatever else is on the path)
-    tool = [hipcc, "-x", "c++", *flags, os.path.join(CSRC, "compiler", "main.cpp"), "-o", COMPILER, f"-L{ROCM}/lib", "-lhiprtc",
+    # (an old-style run path comes before the environment's: the compiler of this toolchain, whatever else is on the path; no HIP
+    # runtime: a compiler has no business with a device)
+    tool = [hipcc, "-no-hip-rt", "-x", "c++", *flags, os.path.join(CSRC, "compiler", "main.cpp"), "-o", COMPILER, f"-L{ROCM}/lib", "-lhiprtc",
             f"-Wl,-rpath,{ROCM}/lib", "-Wl,--disable-new-dtags"]
     if verbose:
         print(" ".join(tool), flush=True)

@@ -98,6 +98,34 @@ private:
     }
 };
 
+// The environment a compiler gets: this process's without a profiler's hooks. A profiler preloads a library that initialises
+// the GPU, which a compiler has no use for (and sixteen at once may not do beside the program under the profiler).
+std::vector<std::string> compiler_environment() {
+    auto starts = [](const std::string& s, std::initializer_list<const char*> with) {
+        for (const char* w : with)
+            if (s.compare(0, strlen(w), w) == 0) return true;
+        return false;
+    };
+    std::vector<std::string> kept;
+    for (char** e = environ; *e; e++) {
+        const std::string var = *e;
+        if (starts(var, {"ROCP_", "ROCPROF", "ROCTRACER_", "HSA_TOOLS_"})) continue;
+        if (!starts(var, {"LD_PRELOAD="})) {
+            kept.push_back(var);
+            continue;
+        }
+        std::string libraries;  // the others that are preloaded stay
+        for (size_t at = strlen("LD_PRELOAD="), end; at < var.size(); at = end + 1) {
+            end = std::min(var.find_first_of(": ", at), var.size());
+            const std::string path = var.substr(at, end - at), file = path.substr(path.rfind('/') + 1);
+            if (path.empty() || starts(file, {"librocprof", "libroctracer", "libroctx"})) continue;
+            libraries += (libraries.empty() ? "" : ":") + path;
+        }
+        if (!libraries.empty()) kept.push_back("LD_PRELOAD=" + libraries);
+    }
+    return kept;
+}
+
 // Compiles in a child process. False: the process could not do its work (the caller compiles in-process). Throws what the
 // compiler has against the source. Text and answer travel in memory files, so that neither side can wait for the other.
 bool compile_in_child(const std::string& source, const std::string& name, const std::vector<std::string>& options, std::vector<char>* code) {
@@ -123,8 +151,12 @@ bool compile_in_child(const std::string& source, const std::string& name, const 
     std::vector<char*> argv{(char*)compiler_path().c_str(), (char*)name.c_str()};
     for (auto& o : options) argv.push_back((char*)o.c_str());
     argv.push_back(nullptr);
+    std::vector<std::string> environment = compiler_environment();
+    std::vector<char*> envp;
+    for (auto& e : environment) envp.push_back(&e[0]);
+    envp.push_back(nullptr);
     pid_t pid = -1;
-    ok = ok && posix_spawn(&pid, compiler_path().c_str(), &actions, nullptr, argv.data(), environ) == 0;
+    ok = ok && posix_spawn(&pid, compiler_path().c_str(), &actions, nullptr, argv.data(), envp.data()) == 0;
     posix_spawn_file_actions_destroy(&actions);
     if (!ok) return false;
     // (a program that ignores SIGCHLD has no status to collect: the answer alone decides)

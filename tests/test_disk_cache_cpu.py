@@ -4,6 +4,8 @@ import os
 import subprocess
 import sys
 
+from helpers import run_with_compiler
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 CHILD = r"""
@@ -76,3 +78,29 @@ def test_what_the_compiler_has_against_a_source_reaches_the_caller():
             "except Exception as e:\n    print(e)\n" % ROOT)
     out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, HELIUM_HIP_CACHE_DIR="off"), capture_output=True, text=True, timeout=300)
     assert out.returncode == 0 and "broken" in out.stdout and "no_such_name" in out.stdout, out.stdout + out.stderr
+
+
+def _probe_with_compiler(tmp_path, script, **env):
+    """Compiles one kernel with that compiler: (compiles, disk hits, bytes of code object) and the process."""
+    out = run_with_compiler(tmp_path, script, CHILD.split("\n", 3)[3], HELIUM_HIP_CACHE_DIR=str(tmp_path / "cache"), **env)
+    assert out.returncode == 0, out.stderr
+    return tuple(int(v) for v in out.stdout.split()), out
+
+
+def test_the_compiler_runs_without_a_profilers_hooks(tmp_path):
+    """What a profiler preloads and sets stays with the program; whatever else is preloaded reaches the compiler as it was."""
+    seen = tmp_path / "environment"
+    preload = ":".join(filter(None, [os.environ.get("LD_PRELOAD"), "/nowhere/librocprofiler-sdk-tool.so", "/nowhere/libother.so", "/nowhere/libroctx64.so"]))
+    _probe_with_compiler(tmp_path, f'env > {seen}; exec "$REAL" "$@"', LD_PRELOAD=preload, ROCP_ONE="1",
+                         ROCPROFILER_TWO="1", HSA_TOOLS_THREE="1", KEPT_ALL_THE_SAME="1")
+    env = dict(line.split("=", 1) for line in seen.read_text().split("\n") if "=" in line)
+    assert not [k for k in env if k.startswith(("ROCP", "HSA_TOOLS"))], env
+    assert env["LD_PRELOAD"] == ":".join(filter(None, [os.environ.get("LD_PRELOAD"), "/nowhere/libother.so"]))
+    assert env["KEPT_ALL_THE_SAME"] == "1" and "PATH" in env
+
+
+def test_the_compiler_does_not_load_the_hip_runtime():
+    import helium_amd
+
+    listed = subprocess.run(["ldd", os.path.join(os.path.dirname(helium_amd.__file__), "helium_rtc")], capture_output=True, text=True).stdout
+    assert "libhiprtc" in listed and "libamdhip64" not in listed and "libhsa" not in listed, listed
