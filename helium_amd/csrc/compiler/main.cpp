@@ -1,13 +1,16 @@
 // The kernel compiler as a process of its own: source text on stdin, `name option...` as arguments, the code object on
-// stdout behind one status byte ('o': code object, 'e': the compiler's log). rtc.cpp says why it is not called in-process.
+// stdout behind one byte ('o': code object, 'e': the compiler's log) and its length in eight. rtc.cpp says why it is not called in-process.
 #include <hip/hiprtc.h>
 #include <unistd.h>
 
+#include <cstdint>
 #include <string>
 #include <vector>
 
 static int answer(char status, const char* data, size_t bytes) {
+    const uint64_t length = bytes;
     std::string out(1, status);
+    out.append((const char*)&length, sizeof length);
     out.append(data, bytes);
     for (size_t done = 0; done < out.size();) {
         const ssize_t n = write(1, out.data() + done, out.size() - done);

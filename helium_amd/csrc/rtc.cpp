@@ -159,20 +159,27 @@ bool compile_in_child(const std::string& source, const std::string& name, const 
     ok = ok && posix_spawn(&pid, compiler_path().c_str(), &actions, nullptr, argv.data(), envp.data()) == 0;
     posix_spawn_file_actions_destroy(&actions);
     if (!ok) return false;
-    // (a program that ignores SIGCHLD has no status to collect: the answer alone decides)
-    while (waitpid(pid, nullptr, 0) < 0 && errno == EINTR) {
+    int status = 0;
+    pid_t ended;
+    while ((ended = waitpid(pid, &status, 0)) < 0 && errno == EINTR) {
     }
+    // (a program that ignores SIGCHLD has no status to collect: the answer, which says how long it is, decides alone)
+    if (ended == pid && !(WIFEXITED(status) && WEXITSTATUS(status) == 0)) return false;
     const off_t bytes = lseek(out.fd, 0, SEEK_END);
-    if (bytes < 2) return false;
+    constexpr off_t kHead = 1 + sizeof(uint64_t);  // the answer's kind and its length
+    if (bytes <= kHead) return false;
     std::vector<char> answer((size_t)bytes);
     for (off_t done = 0; done < bytes;) {
         const ssize_t n = pread(out.fd, answer.data() + done, (size_t)(bytes - done), done);
         if (n <= 0) return false;
         done += n;
     }
-    if (answer[0] == 'e') fail(HE_ERR_RTC, strfmt("hiprtc failed to compile %s: %s", name.c_str(), std::string(answer.begin() + 1, answer.end()).c_str()));
+    uint64_t length;
+    memcpy(&length, answer.data() + 1, sizeof length);
+    if (length != (uint64_t)(bytes - kHead)) return false;
+    if (answer[0] == 'e') fail(HE_ERR_RTC, strfmt("hiprtc failed to compile %s: %s", name.c_str(), std::string(answer.begin() + kHead, answer.end()).c_str()));
     if (answer[0] != 'o') return false;
-    code->assign(answer.begin() + 1, answer.end());
+    code->assign(answer.begin() + kHead, answer.end());
     return true;
 }
 

@@ -4,6 +4,8 @@ import os
 import subprocess
 import sys
 
+import pytest
+
 from helpers import run_with_compiler
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -82,6 +84,7 @@ def test_what_the_compiler_has_against_a_source_reaches_the_caller():
 
 def _probe_with_compiler(tmp_path, script, **env):
     """Compiles one kernel with that compiler: (compiles, disk hits, bytes of code object) and the process."""
+    tmp_path.mkdir(exist_ok=True)
     out = run_with_compiler(tmp_path, script, CHILD.split("\n", 3)[3], HELIUM_HIP_CACHE_DIR=str(tmp_path / "cache"), **env)
     assert out.returncode == 0, out.stderr
     return tuple(int(v) for v in out.stdout.split()), out
@@ -104,3 +107,13 @@ def test_the_compiler_does_not_load_the_hip_runtime():
 
     listed = subprocess.run(["ldd", os.path.join(os.path.dirname(helium_amd.__file__), "helium_rtc")], capture_output=True, text=True).stdout
     assert "libhiprtc" in listed and "libamdhip64" not in listed and "libhsa" not in listed, listed
+
+
+@pytest.mark.parametrize("script", ['"$REAL" "$@" > $0.out; head -c 1000 $0.out', '"$REAL" "$@" > $0.out; head -c 1000 $0.out; exit 2', '"$REAL" "$@"; exit 2',
+                                    '"$REAL" "$@"; kill -9 $$', "exit 0", "printf o"],
+                         ids=["cut_short", "cut_short_with_a_status", "whole_with_a_status", "killed", "nothing", "one_byte"])
+def test_an_answer_that_is_not_whole_is_not_taken(tmp_path, script):
+    """The kernel is compiled in-process instead, to the same code object."""
+    whole, _ = _probe_with_compiler(tmp_path / "sound", 'exec "$REAL" "$@"')
+    got, _ = _probe_with_compiler(tmp_path / "unsound", script)
+    assert got == whole

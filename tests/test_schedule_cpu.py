@@ -157,6 +157,6 @@ for k in range(4):
 plan = Plan(g)
 print(sorted(len(plan.launch_kernel(i).args) for i in range(plan.num_launches())))
 """
-    refuses = run_with_compiler(tmp_path, 'if [ "$1" = joined_kernels ]; then printf "eno registers left"; else exec "$REAL" "$@"; fi', code)
+    refuses = run_with_compiler(tmp_path, 'if [ "$1" = joined_kernels ]; then printf "e\\\\021\\\\0\\\\0\\\\0\\\\0\\\\0\\\\0\\\\0no registers left"; else exec "$REAL" "$@"; fi', code)
     assert refuses.stdout.split("\n")[0] == "[2, 2, 2, 2]", refuses.stdout + refuses.stderr
     assert run_with_compiler(tmp_path, 'exec "$REAL" "$@"', code).stdout.split("\n")[0] == "[8]"
