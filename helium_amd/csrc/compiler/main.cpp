@@ -1,9 +1,14 @@
-// The kernel compiler as a process of its own: source text on stdin, `name option...` as arguments, the code object on
-// stdout behind one byte ('o': code object, 'e': the compiler's log) and its length in eight. rtc.cpp says why it is not called in-process.
+// The kernel compiler as a process of its own: source text on stdin, `name option...` as arguments (or `--version`), the code
+// object (which compiler this is) on stdout behind one byte ('o': code object, 'e': the compiler's log) and its length in eight. rtc.cpp says why it is not called in-process.
 #include <hip/hiprtc.h>
+#include <limits.h>
+#include <link.h>
+#include <sys/stat.h>
 #include <unistd.h>
 
 #include <cstdint>
+#include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -21,8 +26,31 @@ static int answer(char status, const char* data, size_t bytes) {
 }
 static int refuse(const std::string& why) { return answer('e', why.data(), why.size()); }
 
+// The libraries that do the compiling, by the files' names (which carry their versions) and sizes.
+static std::string version() {
+    int major = 0, minor = 0;
+    hiprtcProgram prog;  // (the compiler proper is loaded for the first program)
+    if (hiprtcVersion(&major, &minor) != HIPRTC_SUCCESS || hiprtcCreateProgram(&prog, "// none", "version.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) return "";
+    std::string text = std::to_string(major) + "." + std::to_string(minor);
+    dl_iterate_phdr(
+        [](dl_phdr_info* info, size_t, void* out) {
+            char file[PATH_MAX];
+            struct stat st;
+            if (!strstr(info->dlpi_name, "libhiprtc") && !strstr(info->dlpi_name, "comgr")) return 0;
+            if (!realpath(info->dlpi_name, file) || stat(file, &st) != 0) return 0;
+            *(std::string*)out += " " + std::string(strrchr(file, '/') + 1) + ":" + std::to_string(st.st_size);
+            return 0;
+        },
+        &text);
+    return text;
+}
+
 int main(int argc, char** argv) {
     if (argc < 2) return 2;
+    if (strcmp(argv[1], "--version") == 0) {
+        const std::string v = version();
+        return v.empty() ? 2 : answer('o', v.data(), v.size());
+    }
     std::string source;
     char buf[1 << 16];
     for (ssize_t n; (n = read(0, buf, sizeof buf)) > 0;) source.append(buf, (size_t)n);

@@ -126,9 +126,9 @@ std::vector<std::string> compiler_environment() {
     return kept;
 }
 
-// Compiles in a child process. False: the process could not do its work (the caller compiles in-process). Throws what the
-// compiler has against the source. Text and answer travel in memory files, so that neither side can wait for the other.
-bool compile_in_child(const std::string& source, const std::string& name, const std::vector<std::string>& options, std::vector<char>* code) {
+// Runs the compiler with `args` and the text `in`; its answer's kind and what follows it. False: the process could not do its
+// work. Text and answer travel in memory files, so that neither side can wait for the other.
+bool run_compiler(const std::vector<std::string>& args, const std::string& text, char* kind, std::vector<char>* rest) {
     if (compiler_path().empty()) return false;
     CompilerSlot slot;
     struct Fd {
@@ -138,8 +138,8 @@ bool compile_in_child(const std::string& source, const std::string& name, const 
         }
     } in{memfd_create("helium_rtc_source", MFD_CLOEXEC)}, out{memfd_create("helium_rtc_code", MFD_CLOEXEC)};
     if (in.fd < 0 || out.fd < 0) return false;
-    for (size_t done = 0; done < source.size();) {
-        const ssize_t n = write(in.fd, source.data() + done, source.size() - done);
+    for (size_t done = 0; done < text.size();) {
+        const ssize_t n = write(in.fd, text.data() + done, text.size() - done);
         if (n <= 0) return false;
         done += (size_t)n;
     }
@@ -148,8 +148,8 @@ bool compile_in_child(const std::string& source, const std::string& name, const 
     if (posix_spawn_file_actions_init(&actions) != 0) return false;
     bool ok = posix_spawn_file_actions_adddup2(&actions, in.fd, 0) == 0 && posix_spawn_file_actions_adddup2(&actions, out.fd, 1) == 0 &&
               posix_spawn_file_actions_addclosefrom_np(&actions, 3) == 0;
-    std::vector<char*> argv{(char*)compiler_path().c_str(), (char*)name.c_str()};
-    for (auto& o : options) argv.push_back((char*)o.c_str());
+    std::vector<char*> argv{(char*)compiler_path().c_str()};
+    for (auto& a : args) argv.push_back((char*)a.c_str());
     argv.push_back(nullptr);
     std::vector<std::string> environment = compiler_environment();
     std::vector<char*> envp;
@@ -177,9 +177,22 @@ bool compile_in_child(const std::string& source, const std::string& name, const 
     uint64_t length;
     memcpy(&length, answer.data() + 1, sizeof length);
     if (length != (uint64_t)(bytes - kHead)) return false;
-    if (answer[0] == 'e') fail(HE_ERR_RTC, strfmt("hiprtc failed to compile %s: %s", name.c_str(), std::string(answer.begin() + kHead, answer.end()).c_str()));
-    if (answer[0] != 'o') return false;
-    code->assign(answer.begin() + kHead, answer.end());
+    *kind = answer[0];
+    rest->assign(answer.begin() + kHead, answer.end());
+    return true;
+}
+
+// Compiles in a child process. False: the process could not do its work (the caller compiles in-process). Throws what the
+// compiler has against the source.
+bool compile_in_child(const std::string& source, const std::string& name, const std::vector<std::string>& options, std::vector<char>* code) {
+    std::vector<std::string> args{name};
+    args.insert(args.end(), options.begin(), options.end());
+    char kind = 0;
+    std::vector<char> rest;
+    if (!run_compiler(args, source, &kind, &rest)) return false;
+    if (kind == 'e') fail(HE_ERR_RTC, strfmt("hiprtc failed to compile %s: %s", name.c_str(), std::string(rest.begin(), rest.end()).c_str()));
+    if (kind != 'o') return false;
+    code->swap(rest);
     return true;
 }
 
@@ -208,25 +221,34 @@ void compile_in_process(const std::string& source, const std::string& name, cons
     HE_REQUIRE(r == HIPRTC_SUCCESS, HE_ERR_RTC, "hiprtcGetCode: %s", hiprtcGetErrorString(r));
 }
 
-// What a cached code object depends on besides the source and the options: the compiler that made it.
-const std::string& toolchain_tag() {
+// What a cached code object depends on besides the source and the options: the compiler that made it, which says itself what it
+// is. Empty: there is none of that kind.
+const std::string& child_tag() {
+    static const std::string tag = [] {
+        char kind = 0;
+        std::vector<char> version;
+        if (!run_compiler({"--version"}, "", &kind, &version) || kind != 'o') return std::string();
+        return strfmt("child %s|hip %d|%s", std::string(version.begin(), version.end()).c_str(), (int)HIP_VERSION, he_version());
+    }();
+    return tag;
+}
+const std::string& in_process_tag() {
     static const std::string tag = [] {
         int major = 0, minor = 0;
-        if (!compiler_path().empty()) return strfmt("child|hip %d|%s", (int)HIP_VERSION, he_version());
         if (hiprtcVersion(&major, &minor) != HIPRTC_SUCCESS) major = minor = -1;
         return strfmt("hiprtc %d.%d|hip %d|%s", major, minor, (int)HIP_VERSION, he_version());
     }();
     return tag;
 }
 
-std::string key_of(const std::string& source, const std::vector<std::string>& opts) {
+std::string key_of(const std::string& source, const std::vector<std::string>& opts, const std::string& tag) {
     std::string k = source;
     for (auto& o : opts) {
         k.push_back('\0');
         k += o;
     }
     k.push_back('\0');
-    k += toolchain_tag();
+    k += tag;
     return k;
 }
 
@@ -297,7 +319,8 @@ std::shared_ptr<const std::vector<char>> rtc_compile(const std::string& source, 
                                                      const std::vector<std::string>& extra_options, bool bypass_caches) {
     std::vector<std::string> opts = default_kernel_options();
     for (auto& o : extra_options) opts.push_back(o);
-    std::string key = key_of(source, opts);
+    const bool child = !child_tag().empty();
+    std::string key = key_of(source, opts, child ? child_tag() : in_process_tag());
     if (!bypass_caches) {
         std::lock_guard<std::mutex> lk(g_mu);
         auto it = g_cache.find(key);
@@ -306,22 +329,26 @@ std::shared_ptr<const std::vector<char>> rtc_compile(const std::string& source, 
             return it->second;
         }
     }
+    auto keep = [&](std::vector<char>&& code) {
+        auto sp = std::make_shared<const std::vector<char>>(std::move(code));
+        std::lock_guard<std::mutex> lk(g_mu);
+        g_cache[key] = sp;
+        return sp;
+    };
 
     // Disk cache: the file name is two independent 64-bit hashes of the key.
-    std::string path;
-    std::string dir = cache_dir();
-    if (!dir.empty()) {
-        uint64_t h1 = fnv1a(key.data(), key.size());
-        uint64_t h2 = fnv1a(key.data(), key.size(), 0x9e3779b97f4a7c15ull);
-        path = strfmt("%s/%016llx%016llx.hekc", dir.c_str(), (unsigned long long)h1, (unsigned long long)h2);
-        std::vector<char> blob;
-        if (!bypass_caches && read_cache_file(path, &blob)) {
-            g_disk_hits++;
-            auto sp = std::make_shared<const std::vector<char>>(std::move(blob));
-            std::lock_guard<std::mutex> lk(g_mu);
-            g_cache[key] = sp;
-            return sp;
-        }
+    const std::string dir = cache_dir();
+    auto file_of = [&](const std::string& k) {
+        if (dir.empty()) return std::string();
+        uint64_t h1 = fnv1a(k.data(), k.size());
+        uint64_t h2 = fnv1a(k.data(), k.size(), 0x9e3779b97f4a7c15ull);
+        return strfmt("%s/%016llx%016llx.hekc", dir.c_str(), (unsigned long long)h1, (unsigned long long)h2);
+    };
+    std::string path = file_of(key);
+    std::vector<char> blob;
+    if (!bypass_caches && !path.empty() && read_cache_file(path, &blob)) {
+        g_disk_hits++;
+        return keep(std::move(blob));
     }
 
     if (const char* dump = getenv("HELIUM_HIP_DUMP_DIR")) {
@@ -333,9 +360,18 @@ std::shared_ptr<const std::vector<char>> rtc_compile(const std::string& source, 
         std::ofstream f(strfmt("%s/jit_%s_%d.hip", dump, name.c_str(), id++));
         f << source;
     }
-    std::vector<char> blob;
     try {
-        if (!compile_in_child(source, name, opts, &blob)) compile_in_process(source, name, opts, &blob);
+        if (!child || !compile_in_child(source, name, opts, &blob)) {
+            if (child) {
+                // another compiler's code: kept under that one's name
+                path = file_of(key_of(source, opts, in_process_tag()));
+                if (!bypass_caches && !path.empty() && read_cache_file(path, &blob)) {
+                    g_disk_hits++;
+                    return keep(std::move(blob));
+                }
+            }
+            compile_in_process(source, name, opts, &blob);
+        }
     } catch (...) {
         if (getenv("HELIUM_HIP_DUMP_FAILED")) {
             std::ofstream f(std::string(getenv("HELIUM_HIP_DUMP_FAILED")) + "/" + name + ".failed.hip");
@@ -344,12 +380,8 @@ std::shared_ptr<const std::vector<char>> rtc_compile(const std::string& source, 
         throw;
     }
     g_compiles++;
-
     if (!path.empty()) write_cache_file(path, blob);
-    auto sp = std::make_shared<const std::vector<char>>(std::move(blob));
-    std::lock_guard<std::mutex> lk(g_mu);
-    g_cache[key] = sp;
-    return sp;
+    return keep(std::move(blob));
 }
 
 JitKernel::JitKernel(std::string source, std::string entry, std::vector<std::string> options)

@@ -10,7 +10,7 @@
 
 namespace he {
 
-// Compiles HIP source for gfx950. Cached by (source, options, hiprtc / HIP / library version): in memory, and as a
+// Compiles HIP source for gfx950. Cached by (source, options, compiler / HIP / library version): in memory, and as a
 // checksummed code-object file under the cache directory (HELIUM_HIP_CACHE_DIR, default <library dir>/_kcache) when
 // that directory is usable. `bypass_caches` compiles regardless and replaces both entries.
 std::shared_ptr<const std::vector<char>> rtc_compile(const std::string& source, const std::string& name,

@@ -117,3 +117,29 @@ def test_an_answer_that_is_not_whole_is_not_taken(tmp_path, script):
     whole, _ = _probe_with_compiler(tmp_path / "sound", 'exec "$REAL" "$@"')
     got, _ = _probe_with_compiler(tmp_path / "unsound", script)
     assert got == whole
+
+
+SAYS_OTHER = r"""printf 'o\005\0\0\0\0\0\0\0other'"""
+
+
+def test_the_cache_tells_compilers_apart(tmp_path):
+    """A code object is found by the compiler that made it: not by another version, nor by either what was compiled in-process
+    because the other process could not do its work."""
+    sound, other = 'exec "$REAL" "$@"', 'if [ "$1" = --version ]; then %s; else exec "$REAL" "$@"; fi' % SAYS_OTHER
+    broken = 'if [ "$1" = --version ]; then exec "$REAL" "$@"; else exit 2; fi'
+    counts = lambda script: _probe_with_compiler(tmp_path, script)[0][:2]  # noqa: E731
+    assert counts(sound) == (1, 0)
+    assert counts(other) == (1, 0)    # made by another version: compiled afresh
+    assert counts(broken) == (0, 1)   # nothing to compile
+    for f in os.listdir(tmp_path / "cache"):
+        os.unlink(tmp_path / "cache" / f)
+    assert counts(broken) == (1, 0)   # compiled in-process
+    assert counts(broken) == (0, 1)   # and kept for the next program in the same place
+    assert counts(sound) == (1, 0)    # but not for the other compiler
+    assert len(os.listdir(tmp_path / "cache")) == 2
+
+
+def test_a_compiler_that_cannot_say_what_it_is_is_not_used(tmp_path):
+    (compiles, hits, _), _ = _probe_with_compiler(tmp_path, f"touch {tmp_path}/asked_$1; exit 2")
+    assert (compiles, hits) == (1, 0)
+    assert [f for f in os.listdir(tmp_path) if f.startswith("asked_")] == ["asked_--version"]
