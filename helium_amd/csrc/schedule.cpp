@@ -2,6 +2,8 @@
 // fills in addresses. A small graph's execution is bound by the host, which spent a third of it in maps from nodes to
 // tensors and in one allocation per intermediate value (a training step of 157 launches: 214 of 630 us).
 #include <algorithm>
+#include <functional>
+#include <future>
 #include <map>
 #include <set>
 
@@ -46,6 +48,35 @@ Item item_of(const plan::Instr& instr, uint8_t side) {
     it.writes = instr.all_outputs();
     it.side = side;
     return it;
+}
+
+// Makes the kernels of the groups that have none yet, in parallel. A group without one - it does not compile, or there are no
+// tiles that all members can take - goes out as its members, whose own kernels are there.
+void compile_joins(std::vector<Item>* items, const std::function<std::shared_ptr<KernelBase>(const std::vector<std::shared_ptr<KernelBase>>&)>& join) {
+    std::vector<std::future<std::shared_ptr<KernelBase>>> jobs(items->size());
+    for (size_t i = 0; i < items->size(); i++) {
+        const Item& it = (*items)[i];
+        if (it.instrs.size() < 2 || it.kernel) continue;
+        std::vector<std::shared_ptr<KernelBase>> members;
+        for (auto* instr : it.instrs) members.push_back(instr->kernel());
+        jobs[i] = std::async(std::launch::async, [&join, members]() -> std::shared_ptr<KernelBase> {
+            try {
+                return join(members);
+            } catch (const Error&) {
+                return nullptr;
+            }
+        });
+    }
+    std::vector<Item> list;
+    for (size_t i = 0; i < items->size(); i++) {
+        Item& it = (*items)[i];
+        if (jobs[i].valid() && !(it.kernel = jobs[i].get())) {
+            for (auto* instr : it.instrs) list.push_back(item_of(*instr, it.side));
+            continue;
+        }
+        list.push_back(std::move(it));
+    }
+    *items = std::move(list);
 }
 
 // Joins launches of a one-stream list. Each mergeable launch may run anywhere between the last launch that makes what it
@@ -134,22 +165,12 @@ void join_launches(std::vector<Item>* items) {
         out[i] = 1;
     }
     flush(n);
-    // ---- their kernels; a group whose kernel does not compile goes out as its members' own, which have been compiled
-    items->clear();
-    for (Item& it : list) {
-        if (it.instrs.size() < 2) {
-            items->push_back(std::move(it));
-            continue;
-        }
+    *items = std::move(list);
+    compile_joins(items, [](const std::vector<std::shared_ptr<KernelBase>>& kernels) {
         std::vector<std::shared_ptr<TileKernel>> members;
-        for (auto* i : it.instrs) members.push_back(std::dynamic_pointer_cast<TileKernel>(i->kernel()));
-        try {
-            it.kernel = std::make_shared<JoinedKernel>(members);
-            items->push_back(std::move(it));
-        } catch (const Error&) {
-            for (auto* i : it.instrs) items->push_back(item_of(*i, it.side));
-        }
-    }
+        for (auto& k : kernels) members.push_back(std::dynamic_pointer_cast<TileKernel>(k));
+        return std::make_shared<JoinedKernel>(members);
+    });
 }
 
 // Joins products that follow each other in the list and do not depend on each other: a layer's data gradient and filter
@@ -175,22 +196,8 @@ void join_products(std::vector<Item>* items) {
         group.reads.insert(group.reads.end(), it.reads.begin(), it.reads.end());
         group.writes.insert(group.writes.end(), it.writes.begin(), it.writes.end());
     }
-    items->clear();
-    for (Item& it : list) {
-        if (it.instrs.size() == 1 || it.instrs[0]->kind() != plan::InstrKind::Gemm) {
-            items->push_back(std::move(it));
-            continue;
-        }
-        std::vector<std::shared_ptr<KernelBase>> members;
-        for (auto* i : it.instrs) members.push_back(i->kernel());
-        try {
-            it.kernel = std::make_shared<JoinedProducts>(members);
-            items->push_back(std::move(it));
-        } catch (const Error&) {
-            // no tiles that all of them can take: a launch each, as ever
-            for (auto* i : it.instrs) items->push_back(item_of(*i, it.side));
-        }
-    }
+    *items = std::move(list);
+    compile_joins(items, [](const std::vector<std::shared_ptr<KernelBase>>& kernels) { return std::make_shared<JoinedProducts>(kernels); });
 }
 
 }  // namespace

@@ -160,3 +160,26 @@ print(sorted(len(plan.launch_kernel(i).args) for i in range(plan.num_launches())
     refuses = run_with_compiler(tmp_path, 'if [ "$1" = joined_kernels ]; then printf "e\\\\021\\\\0\\\\0\\\\0\\\\0\\\\0\\\\0\\\\0no registers left"; else exec "$REAL" "$@"; fi', code)
     assert refuses.stdout.split("\n")[0] == "[2, 2, 2, 2]", refuses.stdout + refuses.stderr
     assert run_with_compiler(tmp_path, 'exec "$REAL" "$@"', code).stdout.split("\n")[0] == "[8]"
+
+
+@pytest.mark.parametrize("entry,graph", [
+    ("joined_kernels", "for k in range(30): g.new_output(g.unary(g.new_input([3, 5 + k], 'f32'), 'relu'))"),
+    ("joined_products", "for k in range(8): g.new_output(g.matmul(g.new_input([64, 64], 'bf16'), g.new_input([64, 32 + 8 * k], 'bf16'), 'bf16_f32'))")])
+def test_joins_compile_side_by_side(tmp_path, entry, graph):
+    """Each of two compilations of a joined kernel waits for the other to have begun (and gives up after a while)."""
+    script = f"""if [ "$1" = {entry} ]; then
+mkdir -p {tmp_path}/begun; : > {tmp_path}/begun/$$
+n=0; while [ $(ls {tmp_path}/begun | wc -l) -lt 2 ]; do n=$((n + 1)); if [ $n -gt 200 ]; then : > {tmp_path}/alone; break; fi; sleep 0.1; done
+fi
+exec "$REAL" "$@"
+"""
+    code = f"""
+import helium_amd as ha
+from helium_amd.backend import Plan
+g = ha.ir.OpGraph()
+{graph}
+print(Plan(g).num_launches())
+"""
+    out = run_with_compiler(tmp_path, script, code)
+    assert out.stdout.strip() == "2", out.stdout + out.stderr
+    assert len(list((tmp_path / "begun").iterdir())) == 2 and not (tmp_path / "alone").exists()
