@@ -24,6 +24,7 @@ _ffi._sig("he_plan_describe_planned", C.c_void_p, restype=C.c_char_p)
 _ffi._sig("he_plan_destroy", C.c_void_p)
 _ffi._sig("he_plan_precompile", C.c_void_p)
 _ffi._sig("he_plan_num_launches", C.c_void_p, C.POINTER(C.c_int))
+_ffi._sig("he_plan_blocks", C.c_void_p, C.POINTER(C.c_uint64), C.c_int, C.POINTER(C.c_int))
 _ffi._sig("he_plan_launch_kernel", C.c_void_p, C.c_int, C.POINTER(C.c_void_p))
 _ffi._sig("he_plan_instruction_kernel", C.c_void_p, C.c_int, C.POINTER(C.c_void_p))
 _ffi._sig("he_execute_graph", C.c_void_p, C.POINTER(C.c_uint32), C.POINTER(C.c_void_p), C.c_int, C.POINTER(C.c_uint32),
@@ -135,6 +136,14 @@ class Plan:
         n = C.c_int()
         check(lib.he_plan_num_launches(self.handle, C.byref(n)))
         return n.value
+
+    def blocks(self):
+        """Bytes of each block of device memory that holds values between launches (he_plan_blocks)."""
+        n = C.c_int()
+        check(lib.he_plan_blocks(self.handle, None, 0, C.byref(n)))
+        sizes = (C.c_uint64 * max(n.value, 1))()
+        check(lib.he_plan_blocks(self.handle, sizes, n.value, C.byref(n)))
+        return list(sizes[:n.value])
 
     def launch_kernel(self, index):
         """The kernel of the index-th of them (he_plan_launch_kernel), as `kernel` gives an instruction's."""

@@ -152,6 +152,14 @@ int he_plan_launch_kernel(he_plan_t plan, int index, he_tile_kernel_t* kernel) {
         *kernel = k.release();
     });
 }
+int he_plan_blocks(he_plan_t plan, uint64_t* bytes, int max_blocks, int* num_blocks) {
+    return he::guard([&] {
+        HE_REQUIRE(plan && num_blocks && (bytes || max_blocks == 0), HE_ERR_INVALID, "bad argument");
+        precompile(plan);
+        *num_blocks = plan->schedule ? (int)plan->schedule->blocks.size() : 0;
+        for (int i = 0; i < *num_blocks && i < max_blocks; i++) bytes[i] = plan->schedule->blocks[i];
+    });
+}
 int he_plan_destroy(he_plan_t plan) {
     delete plan;
     return HE_OK;

@@ -325,7 +325,7 @@ struct HostTimer {
         static thread_local int calls = 0;
         for (int i = 0; i < 8; i++) sum[i] += acc[i];
         if (++calls % 100 != 0) return;
-        fprintf(stderr, "[exec timing] per graph, us: setup %.1f, storage %.1f, launches %.1f, finish %.1f\n", sum[2] / 100, sum[3] / 100, sum[4] / 100, sum[5] / 100);
+        fprintf(stderr, "[exec timing] per graph, us: setup %.1f, storage and launches %.1f, finish %.1f\n", sum[2] / 100, sum[4] / 100, sum[5] / 100);
         for (double& v : sum) v = 0;
     }
 };
@@ -546,9 +546,12 @@ std::shared_ptr<const Prepared> prepare(const ir::OpGraph& graph_in) {
             if (!instr->compiled()) jobs.push_back(std::async(std::launch::async, [instr] { instr->precompile(); }));
     for (auto& j : jobs) j.get();
     build_schedule(pr.get());
-    if (getenv("HELIUM_HIP_PLAN_DEBUG") && pr->schedule)
-        fprintf(stderr, "[plan] schedule: %d instructions, %zu launches, %.1f MB of intermediate values\n", pr->schedule->instrs, pr->schedule->launches.size(),
-                pr->schedule->arena_bytes / 1e6);
+    if (getenv("HELIUM_HIP_PLAN_DEBUG") && pr->schedule) {
+        uint64_t bytes = 0;
+        for (uint64_t b : pr->schedule->blocks) bytes += b;
+        fprintf(stderr, "[plan] schedule: %d instructions, %zu launches, %.1f MB of intermediate values in %zu blocks\n", pr->schedule->instrs,
+                pr->schedule->launches.size(), bytes / 1e6, pr->schedule->blocks.size());
+    }
     if (getenv("HELIUM_HIP_PLAN_DEBUG")) {
         size_t fanned = 0, multi = 0;
         for (size_t k = 0; k < pr->plan->steps.size(); k++) {
@@ -644,27 +647,17 @@ NamedTensors execute_scheduled(const Prepared& prepared, const NamedTensors& inp
         local.event_waits++;
         side_joined = true;
     };
-    std::vector<TensorRef> blocks;
+    std::vector<TensorRef> blocks(S.blocks.size());
     try {
         pool.note_uses(tensors, scope);
         ht.lap(2);
-        std::vector<void*> at(S.slots.size(), nullptr);
-        char* arena = nullptr;
-        if (S.arena_bytes) {
-            blocks.push_back(allocate_tensor(HE_U32, (size_t)(S.arena_bytes / 4), scope));
-            arena = (char*)blocks.back()->ptr;
-        }
-        for (size_t i = 0; i < S.slots.size(); i++) {
-            const Schedule::Slot& s = S.slots[i];
-            if (s.where == Schedule::Slot::Result) tensors[i] = allocate_tensor(s.dtype, s.len, scope);
-            at[i] = s.where == Schedule::Slot::Arena ? arena + s.offset : tensors[i]->ptr;
-        }
-        ht.lap(3);
         hipEvent_t main_end = nullptr, early_end = nullptr;  // what the next wait of the other stream is for
         std::vector<void*> ptrs;
         LaunchTimes timing;
         for (size_t i = 0; i < S.launches.size(); i++) {
             const Schedule::Launch& L = S.launches[i];
+            for (uint32_t b : L.opens_blocks) blocks[b] = allocate_tensor(HE_U32, (size_t)(S.blocks[b] / 4), scope);
+            for (uint32_t r : L.opens_results) tensors[r] = allocate_tensor(S.slots[r].dtype, S.slots[r].len, scope);
             const bool on_side = use_side && L.stream == 1;
             const hipStream_t stream = on_side ? st.s[1] : main;
             if (on_side) {
@@ -690,7 +683,10 @@ NamedTensors execute_scheduled(const Prepared& prepared, const NamedTensors& inp
                 set_pending_stop_event(main_end);
             }
             ptrs.resize(L.args.size());
-            for (size_t a = 0; a < L.args.size(); a++) ptrs[a] = at[L.args[a]];
+            for (size_t a = 0; a < L.args.size(); a++) {
+                const Schedule::Slot& s = S.slots[L.args[a]];
+                ptrs[a] = s.where == Schedule::Slot::Arena ? (char*)blocks[s.block]->ptr + s.offset : tensors[L.args[a]]->ptr;
+            }
             if (LaunchTimes::wanted()) timing.start();
             try {
                 if (L.kernel) L.kernel->execute(ptrs.data(), stream);
@@ -705,6 +701,7 @@ NamedTensors execute_scheduled(const Prepared& prepared, const NamedTensors& inp
             if (closes) done_recorded = taken;
             else if (use_side && L.marks_end && !(taken && launch_events)) main_end = record(stream);
             if (use_side && i + 1 == S.early_launches) early_end = record(stream);
+            for (uint32_t b : L.closes_blocks) blocks[b].reset();
         }
         ht.lap(4);
         join_side();

@@ -113,10 +113,11 @@ struct Schedule {
         uint32_t slot;
     };
     struct Slot {
-        // a tensor of the caller's; a tensor the caller gets; or part of the execution's own block, at `offset`
+        // a tensor of the caller's; a tensor the caller gets; or part of one of the execution's own blocks, at `offset`
         enum Where : uint8_t { Input, Result, Arena } where = Arena;
         int dtype = HE_F32;
         size_t len = 0, bytes = 0;
+        uint32_t block = 0;
         uint64_t offset = 0;
     };
     struct Launch {
@@ -124,6 +125,7 @@ struct Schedule {
         std::shared_ptr<Permute> permute;
         std::vector<uint32_t> args;        // slots in the kernel's argument order (permute: source, destination)
         std::vector<uint32_t> new_inputs;  // input slots that this stream reads for the first time
+        std::vector<uint32_t> opens_blocks, opens_results, closes_blocks;  // allocated ahead of the launch, given back behind it
         uint8_t stream = 0;                // 0: the main stream, 1: the side stream
         bool waits_for_main = false;       // the side stream waits for what the main stream has taken so far
         bool marks_end = false;            // ... whose latest launch this is: it carries an event
@@ -134,7 +136,7 @@ struct Schedule {
     std::vector<Slot> slots;
     std::vector<Launch> launches;
     size_t early_launches = 0;  // how many at the head of `launches` are early ones
-    uint64_t arena_bytes = 0;
+    std::vector<uint64_t> blocks;  // bytes of each block that holds values nobody else sees
     int steps = 0, instrs = 0;  // of the plan
     bool uses_side = false;
 };

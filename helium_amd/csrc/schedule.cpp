@@ -345,8 +345,10 @@ void build_schedule(Prepared* pr) {
     }
     // the last launch carries the execution's event when it runs on the main stream
     if (!S.launches.empty() && S.launches.back().stream == 0) S.launches.back().closes = true;
-    // ---- where the values that nobody else sees lie in the execution's one block of memory: the largest first, each at the
-    // lowest address that is free for as long as it is needed. What the side stream touches stays until the streams join.
+    // ---- where the values that nobody else sees lie: the largest first, each at the lowest address of the first block that has
+    // it free for as long as it is needed. What the side stream touches stays until the streams join. A block holds what a page
+    // of the pool does (DevicePool::kMinPage), or one value that is larger: one block for everything took a page of the next
+    // power of two, 64 GB for 33 GB of values.
     const size_t n = S.launches.size();
     std::vector<size_t> from(S.slots.size(), SIZE_MAX), to(S.slots.size(), 0);
     for (size_t i = 0; i < n; i++)
@@ -358,25 +360,54 @@ void build_schedule(Prepared* pr) {
     for (uint32_t s = 0; s < S.slots.size(); s++)
         if (S.slots[s].where == Schedule::Slot::Arena) order.push_back(s);
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return S.slots[a].bytes > S.slots[b].bytes; });
+    const char* env = tuning::get("HELIUM_HIP_ARENA_BLOCK");
+    const uint64_t most = env ? (uint64_t)atoll(env) : DevicePool::kMinPage;
     struct Placed {
         uint64_t start, end;
         size_t from, to;
     };
-    std::vector<Placed> placed;  // by address
+    struct Block {
+        std::vector<Placed> placed;  // by address
+        uint64_t capacity;
+        size_t from, to;
+    };
+    std::vector<Block> blocks;
     for (uint32_t s : order) {
         if (from[s] == SIZE_MAX) from[s] = 0, to[s] = n;  // (written by a launch that names it otherwise: keep it whole)
         const uint64_t size = std::max<uint64_t>((S.slots[s].bytes + DevicePool::kAlign - 1) / DevicePool::kAlign * DevicePool::kAlign, DevicePool::kAlign);
         uint64_t at = 0;
-        for (const Placed& p : placed) {
-            if (p.to < from[s] || p.from > to[s]) continue;
-            if (at + size <= p.start) break;
-            at = std::max(at, p.end);
+        size_t b = 0;
+        for (;; b++) {
+            if (b == blocks.size()) {
+                blocks.push_back({{}, std::max(most, size), SIZE_MAX, 0});
+                S.blocks.push_back(0);
+            }
+            at = 0;
+            for (const Placed& p : blocks[b].placed) {
+                if (p.to < from[s] || p.from > to[s]) continue;
+                if (at + size <= p.start) break;
+                at = std::max(at, p.end);
+            }
+            if (at + size <= blocks[b].capacity) break;
         }
+        Block& block = blocks[b];
+        S.slots[s].block = (uint32_t)b;
         S.slots[s].offset = at;
-        S.arena_bytes = std::max(S.arena_bytes, at + size);
+        S.blocks[b] = std::max(S.blocks[b], at + size);
+        block.from = std::min(block.from, from[s]);
+        block.to = std::max(block.to, to[s]);
         Placed mine{at, at + size, from[s], to[s]};
-        placed.insert(std::upper_bound(placed.begin(), placed.end(), mine, [](const Placed& a, const Placed& b) { return a.start < b.start; }), mine);
+        block.placed.insert(std::upper_bound(block.placed.begin(), block.placed.end(), mine, [](const Placed& a, const Placed& b) { return a.start < b.start; }), mine);
     }
+    // One block (most graphs): everything is allocated ahead of the first launch. Several: blocks and results as they are first
+    // needed, and blocks given back behind their last launch, so that what comes later can have their memory.
+    const bool at_once = S.blocks.size() < 2;
+    for (uint32_t b = 0; b < S.blocks.size(); b++) {
+        S.launches[at_once ? 0 : blocks[b].from].opens_blocks.push_back(b);
+        if (!at_once && blocks[b].to < n) S.launches[blocks[b].to].closes_blocks.push_back(b);
+    }
+    for (uint32_t s = 0; s < S.slots.size(); s++)
+        if (S.slots[s].where == Schedule::Slot::Result) S.launches[at_once || from[s] == SIZE_MAX ? 0 : from[s]].opens_results.push_back(s);
     pr->schedule = std::make_shared<const Schedule>(std::move(S));
 }
 

@@ -328,6 +328,9 @@ int he_plan_num_launches(he_plan_t plan, int* launches);
 /* The kernel of one of them, as he_plan_instruction_kernel gives an instruction's: the arguments of one that several
  * instructions share are theirs one after the other. HE_ERR_INVALID for a permute. */
 int he_plan_launch_kernel(he_plan_t plan, int index, he_tile_kernel_t* kernel);
+/* The blocks of device memory in which an execution keeps the values between its launches: their sizes (as many as `bytes` has
+ * room for), and how many there are. A block holds up to 1 GiB, or one larger value. */
+int he_plan_blocks(he_plan_t plan, uint64_t* bytes, int max_blocks, int* num_blocks);
 int he_plan_destroy(he_plan_t plan);
 
 /* BackendExt::execute_graph (backend.rs:40-80): prunes a copy of the graph, takes the cached plan, compiles its

@@ -196,3 +196,16 @@ def test_two_threads_with_side_streams_give_what_one_thread_gives(gpu, monkeypat
     [t.start() for t in threads]
     [t.join() for t in threads]
     assert not errors, errors[0]
+
+
+@pytest.mark.parametrize("side", [False, True], ids=["one_stream", "side_stream"])
+def test_values_spread_over_many_blocks_change_nothing(gpu, side, monkeypatch):
+    """The values between launches in blocks of 256 KB, allocated and given back as the execution goes, instead of one block: the
+    same bits (as a graph of more than 1 GiB of them runs)."""
+    _, whole, _ = _run("f32", side=side)
+    monkeypatch.setenv("HELIUM_HIP_ARENA_BLOCK", str(256 << 10))
+    r, cut, _ = _run("f32", side=side)
+    assert len(Plan(r["graph"].g).blocks()) > 8
+    assert sorted(whole) == sorted(cut)
+    for o in whole:
+        assert np.array_equal(whole[o], cut[o]), o

@@ -183,3 +183,30 @@ print(Plan(g).num_launches())
     out = run_with_compiler(tmp_path, script, code)
     assert out.stdout.strip() == "2", out.stdout + out.stderr
     assert len(list((tmp_path / "begun").iterdir())) == 2 and not (tmp_path / "alone").exists()
+
+
+def held(shape, count, dtype="f32"):
+    """A graph that holds `count` values of `shape` between its launches: products that other products read."""
+    c = Case()
+    g, precision = c.g, "f32_f32" if dtype == "f32" else "bf16_f32"
+    values = [g.matmul(g.new_input([shape[0], 64], dtype), g.new_input([64, shape[1]], dtype), precision) for _ in range(count)]
+    for v in values:
+        g.new_output(g.matmul(v, g.new_input([shape[1], 32], dtype), precision))
+    return c
+
+
+def test_intermediate_values_lie_in_blocks_of_bounded_size(monkeypatch):
+    GiB = 1 << 30
+    small = held((1024, 1024), 3)
+    small.launches()
+    assert small.plan.blocks() == [3 * 4 << 20]  # one block for everything
+    medium = held((16384, 8192), 5)  # 512 MiB each: two to a block
+    medium.launches()
+    assert medium.plan.blocks() == [GiB, GiB, GiB // 2]
+    large = held((32768, 12288), 3)  # 1.5 GiB each: a block of its own
+    large.launches()
+    assert large.plan.blocks() == [3 * GiB // 2] * 3
+    monkeypatch.setenv("HELIUM_HIP_ARENA_BLOCK", str(8 << 20))
+    cut = held((1024, 1024), 3)
+    cut.launches()
+    assert cut.plan.blocks() == [8 << 20, 4 << 20]
