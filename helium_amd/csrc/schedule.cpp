@@ -238,11 +238,26 @@ void build_schedule(Prepared* pr) {
             if (is_view(*instr, g)) view_of[instr->outputs()[0]] = instr->inputs()[0];
         }
     }
+    // A result is memory of its own, which its owner may write: one that would be another result's or an input's under another
+    // shape is copied after all.
+    for (bool again = true; again;) {
+        again = false;
+        std::map<NodeId, NodeId> held_by;  // storage -> the result that has it
+        for (NodeId in : g.inputs()) held_by[in] = in;
+        for (NodeId out : g.outputs()) {
+            const NodeId n = g.inbound(out)[0], other = held_by.emplace(base(n), n).first->second;
+            if (other == n) continue;
+            view_of.erase(view_of.count(n) ? n : other);
+            again = true;
+            break;
+        }
+    }
+    auto renames = [&](const plan::Instr& instr) { return is_view(instr, g) && view_of.count(instr.outputs()[0]); };
     const Prepared::Side& side = pr->side;
     if (side.side.empty()) {
         for (auto& step : plan.steps)
             for (auto& instr : step.instrs) {
-                if (instr->absorbed() || is_view(*instr, g)) continue;
+                if (instr->absorbed() || renames(*instr)) continue;
                 Item it = item_of(*instr, 0);
                 it.mergeable = can_share_launch(*instr);
                 items.push_back(std::move(it));
@@ -262,7 +277,7 @@ void build_schedule(Prepared* pr) {
         for (size_t i = 0; i < side.order.size(); i++) {
             if (side.side[i] != 2) continue;
             issued[i] = 1;
-            if (is_view(*side.order[i], g)) continue;
+            if (renames(*side.order[i])) continue;
             Item it = item_of(*side.order[i], 2);
             it.mergeable = can_share_launch(*side.order[i]);
             early.push_back(std::move(it));
@@ -274,7 +289,7 @@ void build_schedule(Prepared* pr) {
         items = std::move(early);
         auto issue = [&](auto&& self, size_t i) -> void {
             issued[i] = 1;
-            if (!is_view(*side.order[i], g)) items.push_back(item_of(*side.order[i], side.side[i]));
+            if (!renames(*side.order[i])) items.push_back(item_of(*side.order[i], side.side[i]));
             if (side.side[i] != 1) return;
             for (uint32_t d : side.dependents[i]) {
                 if (issued[d] || side.side[d] != 1) continue;

@@ -336,7 +336,8 @@ int he_plan_destroy(he_plan_t plan);
 /* BackendExt::execute_graph (backend.rs:40-80): prunes a copy of the graph, takes the cached plan, compiles its
  * kernels, and runs the steps over a pool of streams. input_tensors[i] is the storage of Input node input_nodes[i].
  * On return output_nodes / output_tensors hold one (Output node, tensor) pair per Output node of the graph; each
- * tensor is a new reference the caller frees. */
+ * tensor is a new reference the caller frees. Its storage is its own, whatever the graph does to get there, unless Output
+ * nodes name the same node or an Input: those have one storage between them. */
 int he_execute_graph(he_graph_t graph, const uint32_t* input_nodes, const he_tensor_t* input_tensors, int num_inputs,
                      uint32_t* output_nodes, he_tensor_t* output_tensors, int max_outputs, int* num_outputs);
 /* ---- 7. Fusion search over a fusion-IR graph ------------------------------------------------------------

@@ -543,3 +543,18 @@ def test_small_elementwise_launches_share_launches(gpu, count):
     for _ in range(2):
         got, steps = run_graph(g, host)
         check_against_oracle(g, host, got, steps, matmul_rel=1e-2)
+
+
+def test_results_share_no_storage(gpu):
+    """Not with an input, and not with each other, when one is another value under another shape."""
+    g = ha.ir.OpGraph()
+    x = g.new_input([6, 10], "f32")
+    total = g.reduce(x, "sum", 1)
+    outs = [g.new_output(n) for n in (g.reshape(x, [60]), total, g.reshape(total, [6]), g.reshape(g.unary(x, "neg"), [10, 6]))]
+    values = np.arange(60, dtype=np.float32)
+    tx = Tensor.from_numpy(values, "f32")
+    got = execute_graph(g, {x: tx})
+    assert len({t.ptr.value for t in [tx, *got.values()]}) == 5
+    want = [values, values.reshape(6, 10).sum(axis=1), values.reshape(6, 10).sum(axis=1), -values]
+    for o, w in zip(outs, want):
+        assert np.array_equal(got[o].to_numpy(), w)

@@ -210,3 +210,29 @@ def test_intermediate_values_lie_in_blocks_of_bounded_size(monkeypatch):
     cut = held((1024, 1024), 3)
     cut.launches()
     assert cut.plan.blocks() == [8 << 20, 4 << 20]
+
+
+def test_results_have_storage_of_their_own():
+    """Reshapes are no launches where nobody can tell, and copies where two results, or a result and an input, would share."""
+    def launched(build):
+        c = Case()
+        for node in build(c.g, c.g.new_input([6, 10], "f32")):
+            c.g.new_output(node)
+        return sorted(sum(a["is_output"] for a in k.args) for k in c.launches())
+
+    total = lambda g, x: g.reduce(x, "sum", 1)  # noqa: E731
+    assert launched(lambda g, x: [g.reshape(total(g, x), [6])]) == [1]                       # a value between launches
+    assert launched(lambda g, x: [g.reshape(x, [60])]) == [1]                                # an input
+    assert launched(lambda g, x: [g.reshape(g.reshape(x, [60]), [10, 6])]) == [1]
+    assert launched(lambda g, x: [x]) == []                                                  # the input itself
+    def both(g, x):
+        t = total(g, x)
+        return [t, g.reshape(t, [6])]
+    assert launched(both) == [1, 1]
+    assert launched(lambda g, x: both(g, x)[::-1]) == [1, 1]
+
+    def three_shapes(g, x):
+        t = total(g, x)
+        flat = g.reshape(t, [6])
+        return [g.reshape(flat, [2, 3]), flat, g.reshape(t, [3, 2])]
+    assert launched(three_shapes) == [1, 3]  # (one instruction for the shapes)
