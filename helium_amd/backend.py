@@ -6,7 +6,11 @@ import numpy as np
 
 from . import _ffi
 from ._ffi import check, lib
-from . import _native  # (after _ffi: the extension calls the library that it loads)
+try:
+    from . import _native  # (after _ffi: the extension calls the library that it loads)
+except ImportError as e:
+    raise ImportError("helium_amd._native is not built for this Python. Run `python -m helium_amd.build` (or "
+                      "__graft_entry__.build()) with it, which needs its headers.") from e
 from . import device
 from .device import NP_STORAGE, init
 
@@ -49,10 +53,13 @@ class Tensor(_native.Tensor):
 
     _info = None  # (dtype, len, nbytes, ptr), asked for on first use: a result that is only passed on costs no call
 
+    # the he_tensor_t, as every handle of this package: a ctypes.c_void_p, null when freed
+    handle = property(lambda self: C.c_void_p(self._handle), lambda self, handle: setattr(self, "_handle", handle))
+
     def _get(self, i):
         if self._info is None:
             dt, ln, nb, ptr = C.c_int32(), C.c_uint64(), C.c_uint64(), C.c_void_p()
-            check(lib.he_tensor_info(self.handle, C.byref(dt), C.byref(ln), C.byref(nb), C.byref(ptr)))
+            check(lib.he_tensor_info(self._handle, C.byref(dt), C.byref(ln), C.byref(nb), C.byref(ptr)))
             self._info = (_ffi.DTYPE_NAMES[dt.value], ln.value, nb.value, ptr)
         return self._info[i]
 
@@ -78,7 +85,7 @@ class Tensor(_native.Tensor):
         """Backend::download_tensor (blocking): the storage-form array."""
         np_dtype = NP_STORAGE[_ffi.DTYPES[self.dtype]]
         out = np.empty(self.nbytes // np.dtype(np_dtype).itemsize, dtype=np_dtype)
-        check(lib.he_tensor_download(self.handle, out.ctypes.data_as(C.c_void_p)))
+        check(lib.he_tensor_download(self._handle, out.ctypes.data_as(C.c_void_p)))
         return out
 
 

@@ -74,7 +74,7 @@ int set_handle(PyObject* self, PyObject* value, void*) {
     return 0;
 }
 
-PyGetSetDef tensor_getset[] = {{"handle", get_handle, set_handle, "the he_tensor_t, as a number (None: freed)", nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
+PyGetSetDef tensor_getset[] = {{"_handle", get_handle, set_handle, "the he_tensor_t, as a number (None: freed)", nullptr}, {nullptr, nullptr, nullptr, nullptr, nullptr}};
 PyMethodDef tensor_methods[] = {{"free", tensor_free, METH_NOARGS, "lets go of the storage"}, {nullptr, nullptr, 0, nullptr}};
 PyTypeObject tensor_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 

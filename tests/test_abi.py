@@ -50,3 +50,19 @@ def test_rtc_reports_compile_errors():
     with pytest.raises(HeliumError) as e:
         device.rtc_compile('extern "C" __global__ void k(float* p) { p[0] = undefined_symbol; }', "abi_bad")
     assert "undefined_symbol" in str(e.value)
+
+
+def test_a_tensors_handle_is_a_ctypes_pointer():
+    from helium_amd.backend import Tensor
+
+    t = Tensor(ctypes.c_void_p(4096))  # (an address that nothing follows here)
+    try:
+        assert type(t.handle) is ctypes.c_void_p and t.handle.value == 4096 and t.handle
+        t.handle = ctypes.c_void_p()
+        assert type(t.handle) is ctypes.c_void_p and t.handle.value is None and not t.handle
+        t.handle = 4096
+        assert t.handle.value == 4096
+    finally:
+        t.handle = None
+    t.free()
+    assert not t.handle
