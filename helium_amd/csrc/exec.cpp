@@ -194,6 +194,7 @@ struct Staging {
     hipEvent_t done = nullptr;
 };
 struct Streams {
+    int device = 0;
     std::vector<hipStream_t> s;
     EventRef exec_end;  // end of this thread's latest execution (recorded on s[0] after it joined the others)
     bool has_run = false;
@@ -223,22 +224,55 @@ Staging& staging_buffer(Streams& st, size_t bytes) {
     st.staging.push_back(b);
     return st.staging.back();
 }
-Streams& thread_streams() {
-    // a small pool of non-blocking streams per host thread (helium/src/cuda/context.rs:112-125)
-    static thread_local Streams st;
-    if (st.s.empty()) {
-        // HELIUM_HIP_STREAMS=<1..4>: how many streams the independent instructions of a step fan out over
-        const char* env = getenv("HELIUM_HIP_STREAMS");
-        const int n = env ? std::max(1, std::min(4, atoi(env))) : 4;
-        for (int i = 0; i < n; i++) {
-            hipStream_t x;
-            HE_HIP(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
-            st.s.push_back(x);
-        }
-        HE_HIP(hipStreamCreateWithFlags(&st.h2d, hipStreamNonBlocking));
-        HE_HIP(hipStreamCreateWithFlags(&st.d2h, hipStreamNonBlocking));
+std::unique_ptr<Streams> make_streams() {
+    auto st = std::make_unique<Streams>();
+    HE_HIP(hipGetDevice(&st->device));
+    // HELIUM_HIP_STREAMS=<1..4>: how many streams the independent instructions of a step fan out over
+    const char* env = getenv("HELIUM_HIP_STREAMS");
+    const int n = env ? std::max(1, std::min(4, atoi(env))) : 4;
+    for (int i = 0; i < n; i++) {
+        hipStream_t x;
+        HE_HIP(hipStreamCreateWithFlags(&x, hipStreamNonBlocking));
+        st->s.push_back(x);
     }
+    HE_HIP(hipStreamCreateWithFlags(&st->h2d, hipStreamNonBlocking));
+    HE_HIP(hipStreamCreateWithFlags(&st->d2h, hipStreamNonBlocking));
     return st;
+}
+// A small pool of non-blocking streams per host thread (helium/src/cuda/context.rs:112-125), with the pinned buffers that go
+// with it. A thread that ends leaves its own to the next one that begins, which carries on where they are: its executions come
+// after the other's on the same stream, and so may take the memory that those have freed (DevicePool::begin_scope: the pool's
+// thread token is the set's address). A thread's address as the token would be taken up by another thread's, whose streams are
+// in no order with the first one's.
+Streams& thread_streams() {
+    struct Spare {
+        std::mutex mu;
+        std::vector<std::unique_ptr<Streams>> sets;
+    };
+    static Spare* spare = new Spare();  // never destroyed: threads may end after static destruction
+    struct Mine {
+        std::unique_ptr<Streams> st;
+        ~Mine() {
+            if (!st) return;
+            std::lock_guard<std::mutex> lk(spare->mu);
+            spare->sets.push_back(std::move(st));
+        }
+    };
+    static thread_local Mine mine;
+    if (!mine.st) {
+        int device = 0;
+        HE_HIP(hipGetDevice(&device));
+        std::lock_guard<std::mutex> lk(spare->mu);
+        for (auto& set : spare->sets)
+            if (set->device == device) {
+                mine.st = std::move(set);
+                std::swap(set, spare->sets.back());
+                spare->sets.pop_back();
+                break;
+            }
+    }
+    if (!mine.st) mine.st = make_streams();
+    return *mine.st;
 }
 }  // namespace
 

@@ -42,7 +42,7 @@ public:
     static constexpr uint64_t kAlign = 256;             // alignment of every block (device.rs:33)
     static constexpr uint64_t kMinPage = 1ull << 30;    // device.rs:35
     static DevicePool& global();
-    // `thread`: a token of the calling host thread (0: none). The executions of one thread are ordered on the device
+    // `thread`: a token of the calling host thread's streams (0: none). The executions of one thread are ordered on the device
     // (each waits for the end of the one before), so the thread's previous scope is the new scope's parent.
     uint64_t begin_scope(uint64_t thread = 0);
     void end_scope(uint64_t scope);  // called once the scope's device work has finished

@@ -558,3 +558,35 @@ def test_results_share_no_storage(gpu):
     want = [values, values.reshape(6, 10).sum(axis=1), values.reshape(6, 10).sum(axis=1), -values]
     for o, w in zip(outs, want):
         assert np.array_equal(got[o].to_numpy(), w)
+
+
+def test_threads_that_end_with_work_under_way(gpu):
+    """A thread's last execution may still run when the thread has ended and another one begins; neither gets the other's memory."""
+    n = 2048
+    g = ha.ir.OpGraph()
+    x, w = g.new_input([n, n], "f32"), g.new_input([n, n], "f32")
+    v = x
+    for _ in range(3):  # values of 16 MB between the launches
+        v = g.matmul(g.unary(v, "neg"), w, "f32_f32")
+    out = g.new_output(v)
+    rng = np.random.default_rng(4)
+    scale = rng.uniform(0.5, 2.0, n).astype(np.float32)  # w: a scaled permutation, so that every sum has one term
+    order = rng.permutation(n)
+    weights = np.zeros((n, n), np.float32)
+    weights[order, np.arange(n)] = scale
+    tw = Tensor.from_numpy(weights, "f32")
+    xs = [rng.uniform(-1, 1, (n, n)).astype(np.float32) for _ in range(3)]
+    tx = [Tensor.from_numpy(a, "f32") for a in xs]
+    execute_graph(g, {x: tx[0], w: tw})[out].to_numpy()
+    results = []
+    for k in range(24):
+        t = threading.Thread(target=lambda k=k: results.append(execute_graph(g, {x: tx[k % 3], w: tw})[out]))
+        t.start()
+        t.join()
+    want = []
+    for a in xs:
+        for _ in range(3):
+            a = (-a)[:, order] * scale
+        want.append(a)
+    for k, r in enumerate(results):
+        assert np.array_equal(r.to_numpy().reshape(n, n), want[k % 3]), k
