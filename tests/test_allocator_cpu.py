@@ -159,3 +159,43 @@ def test_random_streams_never_hand_out_memory_another_stream_may_use():
         if step % 500 == 0:
             a.stats()
     a.stats()
+
+
+def test_streams_that_branch():
+    """Streams with random parents - chains, several children of one stream, parents that have ended - and one block that goes
+    round: a stream gets it exactly when everything that may still touch it is the stream itself or an ancestor."""
+    for seed in range(20):
+        rng = np.random.default_rng(seed)
+        a = BlockAllocator()
+        a.add_page(1024)
+        ancestors, live, last = {}, [], 0
+        holds = set()  # streams whose work may still touch the block
+        got = refused = 0
+        for _ in range(300):
+            what = rng.random()
+            if not live or what < 0.3:
+                # the latest stream, any live one, one that may have ended, or none
+                parent = int(rng.choice([last, live[int(rng.integers(len(live)))] if live else 0, int(rng.integers(last + 1)), 0], p=[0.5, 0.3, 0.1, 0.1]))
+                s = a.begin_stream(parent)
+                ancestors[s] = (ancestors[parent] | {parent}) if parent in live else set()
+                live.append(s)
+                last = s
+            elif what < 0.5:
+                s = live.pop(0 if rng.random() < 0.7 else int(rng.integers(len(live))))
+                a.end_stream(s)
+                holds.discard(s)
+            else:
+                s = int(rng.choice(live))
+                b = a.allocate(1024, 256, s)
+                assert (b is not None) == (holds <= ancestors[s] | {s}), (seed, s, holds, ancestors[s])
+                if b is None:
+                    refused += 1
+                    continue
+                got += 1
+                holds.add(s)
+                assert b.in_use() == sorted(holds)
+                a.deallocate(b)
+        assert got > 10 and refused > 10, (got, refused)
+        for s in live:
+            a.end_stream(s)
+        assert a.stats() == {"free_blocks": 1, "free_bytes": 1024, "largest_free_block": 1024, "streams": 0}

@@ -590,3 +590,75 @@ def test_threads_that_end_with_work_under_way(gpu):
         want.append(a)
     for k, r in enumerate(results):
         assert np.array_equal(r.to_numpy().reshape(n, n), want[k % 3]), k
+
+
+@pytest.mark.parametrize("length", [1, 3, 255, 257, 32767, 32768, 32769, 100_003])
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+def test_downloads_small_and_large(gpu, length, dtype):
+    """Up to 64 KB leaves through a kernel, more through a copy: of an upload, of the latest execution's result, of an earlier
+    one's, and of another thread's while this thread has none of its own under way, or one."""
+    rng = np.random.default_rng(length)
+    values = nm.to_storage(rng.uniform(0.5, 1, length).astype(np.float32), dtype)
+    t = Tensor.from_numpy(values, dtype, length)
+    assert np.array_equal(t.to_numpy(), values)
+    g = ha.ir.OpGraph()
+    x = g.new_input([length], dtype)
+    out = g.new_output(g.unary(g.unary(x, "relu"), "neg"))
+    want = values ^ np.uint16(0x8000) if dtype == "bf16" else -values
+    earlier = execute_graph(g, {x: t})[out]
+    latest = execute_graph(g, {x: Tensor.from_numpy(values, dtype, length)})[out]
+    assert np.array_equal(latest.to_numpy(), want) and np.array_equal(earlier.to_numpy(), want)
+    for own in (False, True):
+        results = []
+        worker = threading.Thread(target=lambda: results.extend(execute_graph(g, {x: t})[out] for _ in range(8)))
+        worker.start()
+        worker.join()
+        if own:  # relu of what the other thread made is zero
+            assert not nm.from_storage(execute_graph(g, {x: results[-1]})[out].to_numpy(), dtype, [length]).any()
+        for r in results:
+            assert np.array_equal(r.to_numpy(), want)
+
+
+def _outputs_of(kernel, inputs):
+    """One launch on the GPU; {node: bytes of the output}."""
+    bufs = [(ha.DeviceBuffer(max(a["numel"] * (2 if a["dtype"] == "bf16" else 4), 4)) if a["is_output"] else ha.DeviceBuffer.from_numpy(inputs[a["node"]]), a)
+            for a in kernel.args]
+    for b, a in bufs:
+        if a["is_output"]:
+            b.fill_u8(0xA5)
+    kernel.execute([b for b, _ in bufs])
+    return {a["node"]: b.to_numpy(np.uint16 if a["dtype"] == "bf16" else np.uint32) for b, a in bufs if a["is_output"]}
+
+
+def _joined_cases():
+    import test_schedule_cpu as joined
+
+    def products(make):
+        c = joined.Case(11)
+        for node in make(c):
+            c.g.new_output(node)
+        return c
+
+    cases = {name: (lambda make=make: products(make)) for name, make in joined.JOINED.items()}
+    cases["layer_bf16"] = lambda: products(lambda c: joined.linear_backward(c, 256, 512, 384, "bf16", "bf16_f32"))
+    cases["layer_ragged_f32"] = lambda: products(lambda c: joined.linear_backward(c, 203, 511, 333, "f32", "f32_f32"))
+    cases["block"] = lambda: products(lambda c: joined.conv_backward(c, [4, 15, 15, 64], 64, 3, 2))
+    cases["updates"] = lambda: joined.updates(30, seed=5)
+    cases["reductions"] = lambda: joined.reductions(5, (64, 32, 1024), "f32")
+    return cases
+
+
+@pytest.mark.parametrize("name", _joined_cases())
+def test_launches_that_are_shared_make_the_bits_of_their_members(gpu, name):
+    c = _joined_cases()[name]()
+    kernels = c.launches()
+    assert kernels and all(k.description.startswith("joined") for k in kernels), [k.description for k in kernels]
+    origin = {n["id"]: n["origin"] for n in c.plan.graph().nodes}
+    inputs = {n: c.host[o] for n, o in origin.items() if o in c.host}
+    alone = {}
+    for i in range(sum(len(instrs) for instrs, _ in c.plan.steps)):
+        alone.update(_outputs_of(c.plan.kernel(i), inputs))
+    for k in kernels:
+        for node, data in _outputs_of(k, inputs).items():
+            assert np.array_equal(data, alone.pop(node)), (node, k.description)
+    assert not alone

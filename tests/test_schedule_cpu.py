@@ -10,6 +10,7 @@ from helium_amd.backend import Plan
 from oracle import helium_ir as oracle_ir
 from oracle import numerics as nm
 
+from cpu_emul import run_kernel
 from helpers import run_tile_kernel_cpu, run_with_compiler
 
 
@@ -236,3 +237,71 @@ def test_results_have_storage_of_their_own():
         flat = g.reshape(t, [6])
         return [g.reshape(flat, [2, 3]), flat, g.reshape(t, [3, 2])]
     assert launched(three_shapes) == [1, 3]  # (one instruction for the shapes)
+
+
+# ---- joined products -------------------------------------------------------------------------------------------------
+def run_product(kernel, entry, inputs):
+    """A product's launch (one of several products, the classes of a strided data gradient, or one product) on the CPU."""
+    gx = int(re.search(r"grid=(\d+)", kernel.description).group(1))
+    threads = int(re.search(r"threads=(\d+)", kernel.description).group(1))
+    bufs = [(np.full(a["numel"], np.nan, np.float32) if a["dtype"] == "f32" else np.full(a["numel"], 0x7FC0, np.uint16), 2) if a["is_output"]
+            else (inputs[a["node"]], 0) for a in kernel.args]
+    outs = run_kernel(re.split(r"// ---- part \d+ of \d+\n", kernel.source)[0], entry, gx, threads, bufs)
+    return dict(zip([a["node"] for a in kernel.args if a["is_output"]], outs))
+
+
+def conv_backward(c, image, channels, kernel, stride):
+    """A strided convolution's data and filter gradients."""
+    params = {"in_channels": image[3], "out_channels": channels, "kernel_size": [kernel, kernel], "stride": [stride, stride]}
+    out = oracle_ir.conv_output_size(params, image[1:3], [kernel, kernel])
+    dy, w, x = c.new([image[0], *out, channels], "bf16"), c.new([channels, kernel, kernel, image[3]], "bf16"), c.new(image, "bf16")
+    return [c.g.conv_backward_data(dy, w, params, list(image[1:3])), c.g.conv_backward_filter(dy, x, params)]
+
+
+def linear_backward(c, rows, inner, cols, dtype, precision):
+    x, w, dy = c.new([rows, inner], dtype), c.new([inner, cols], dtype), c.new([rows, cols], dtype)
+    return [c.g.matmul(dy, c.g.swap_dims(w, 0, 1), precision), c.g.matmul(c.g.swap_dims(x, 0, 1), dy, precision)]
+
+
+def plain_and_with_an_epilogue(c, count):
+    g, outs = c.g, []
+    for k in range(count):
+        v = g.matmul(c.new([40 + 32 * k, 96], "bf16"), c.new([96, 48 + 8 * k], "bf16"), "bf16_f32")
+        outs.append(g.change_data_type(g.unary(v, "relu"), "bf16") if k % 2 else v)
+    return outs
+
+
+JOINED = {
+    "even_bf16": lambda c: linear_backward(c, 64, 96, 128, "bf16", "bf16_f32"),
+    "ragged_bf16": lambda c: linear_backward(c, 67, 101, 35, "bf16", "bf16_f32"),
+    "ragged_f32": lambda c: linear_backward(c, 33, 70, 47, "f32", "f32_f32"),
+    "epilogues": lambda c: plain_and_with_an_epilogue(c, 4),
+    "strided_convolution": lambda c: conv_backward(c, [1, 9, 9, 16], 16, 3, 2),
+    "convolution_that_leaves_pixels": lambda c: conv_backward(c, [1, 9, 9, 8], 16, 1, 2),
+    "one_row_and_one_column": lambda c: [c.g.matmul(c.new([1, 200], "bf16"), c.new([200, 40], "bf16"), "bf16_f32"),
+                                         c.g.matmul(c.new([50, 200], "bf16"), c.new([200, 1], "bf16"), "bf16_f32")],
+}
+
+
+@pytest.mark.parametrize("name", JOINED)
+def test_joined_products_are_their_members(name):
+    """Products that share a launch: the bits that each makes by itself, and the oracle's values."""
+    c = Case(11)
+    for node in JOINED[name](c):
+        c.g.new_output(node)
+    kernels = c.launches()
+    assert len(kernels) == 1 and kernels[0].description.startswith("joined products="), [k.description for k in kernels]
+    origin = {n["id"]: n["origin"] for n in c.plan.graph().nodes}
+    inputs = {n: c.host[o] for n, o in origin.items() if o in c.host}
+    got = run_product(kernels[0], "joined_products", inputs)
+    alone = {}
+    for i in range(sum(len(instrs) for instrs, _ in c.plan.steps)):
+        k = c.plan.kernel(i)
+        alone.update(run_product(k, "fused_matmul_parts" if k.description.startswith("composite") else "fused_matmul", inputs))
+    assert sorted(got) == sorted(alone) and len(got) >= 2
+    val, desc = oracle_ir.evaluate(c.g.nodes, c.host)
+    for node, data in got.items():
+        assert np.array_equal(data, alone[node]), (node, kernels[0].description)
+        want = np.asarray(val[origin[node]], dtype=np.float64).reshape(-1)
+        have = nm.from_storage(data, desc[origin[node]][1], want.shape).astype(np.float64)
+        assert np.abs(have - want).max() <= (1e-5 if "f32" in name else 2e-2) * np.abs(want).max(), (node, kernels[0].description)
