@@ -777,7 +777,7 @@ GemmProblem gemm_problem_from_fusion(const fir::OpGraph& g) {
     return pr;
 }
 
-int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch, bool f32) {
+int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch) {
     if (tuning::get("HELIUM_HIP_GEMM_NO_SPLIT_K") || batch != 1) return 1;
     if (const char* env = tuning::get("HELIUM_HIP_GEMM_SPLIT_K")) return std::max(1, atoi(env));
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), k_tiles = (K + 63) / 64;
@@ -787,13 +787,6 @@ int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch, bool f32) {
     if (((M + 63) / 64) * ((N + 63) / 64) >= 192) return 1;
     // So do the waves of a workgroup that share a small tile's k range (small_tile): such a product costs about 2.7 us and
     // 0.2 us for every tile that a wave takes, the second launch of a split one 4 us (32 x 512 x 4608: 6.3 us against 10).
-    // An f32 product whose waves' partial sums would be longer than those of a split range (of eight tiles) keeps the split: its
-    // error against 64 bits is no larger for the speed (filter_gradient_split_k has figures).
-    if (f32) {
-        const int64_t split = std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 8, 1024});
-        const int64_t waves = ((M + 31) / 32) * ((N + 31) / 32) <= 256 ? 8 : 1;
-        return split > waves ? (int)split : 1;
-    }
     if (k_tiles <= 192) return 1;
     return (int)std::max<int64_t>(1, std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 96, 1024}));
 }

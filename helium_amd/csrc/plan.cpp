@@ -889,7 +889,7 @@ GemmProblem conv_problem(const ir::OpSubgraph& sg, NodeId conv) {
     pr.M = cv.N * cv.P * cv.Q;
     pr.N = op.conv.out_channels;
     pr.K = cv.R * cv.S * cv.C;
-    pr.split_k = choose_split_k(pr.M, pr.N, pr.K, 1, image.dtype == HE_F32);
+    pr.split_k = choose_split_k(pr.M, pr.N, pr.K, 1);
     HE_REQUIRE(pr.M > 0 && pr.M < (1ll << 31) && ir::num_elements(image.shape) < (1ll << 32), HE_ERR_UNSUPPORTED, "conv too large for 32-bit tile indices");
     pr.mma_dtype = image.dtype == HE_F32 ? HE_F32 : image.dtype == HE_F16 ? HE_F16 : HE_BF16;
     auto operand = [&](tp::Program& p, const ir::Descriptor& d, NodeId node, int64_t rows, int64_t cols) {
@@ -995,7 +995,7 @@ GemmProblem conv_backward_data_problem(const ir::OpSubgraph& sg, NodeId node, in
     pr.M = cv.N * cv.P * cv.Q;
     pr.N = in_channels;
     pr.K = cv.R * cv.S * cv.C;
-    pr.split_k = cls >= 0 ? 1 : choose_split_k(pr.M, pr.N, pr.K, 1, flow.dtype == HE_F32);
+    pr.split_k = cls >= 0 ? 1 : choose_split_k(pr.M, pr.N, pr.K, 1);
     HE_REQUIRE(pr.M > 0 && pr.M < (1ll << 31) && ir::num_elements(flow.shape) < (1ll << 32), HE_ERR_UNSUPPORTED, "conv too large for 32-bit tile indices");
     pr.mma_dtype = flow.dtype == HE_F32 ? HE_F32 : flow.dtype == HE_F16 ? HE_F16 : HE_BF16;
     HE_REQUIRE(in_channels % (pr.mma_dtype == HE_F32 ? 4 : 8) == 0, HE_ERR_UNSUPPORTED,
@@ -1144,12 +1144,9 @@ int filter_gradient_split_k(const GemmProblem& pr, bool element_gather) {
     //  - 512 output channels keep 256x256 tiles, whose count, not that of 128x128 tiles, decides the shares as long as a
     //    share keeps 12 k-tiles: the 7x7x512 layer 36 x 4 = 144 workgroups 77.4 us, 36 x 7 = 252 workgroups 70.3.
     //  - a short k (few pixels) and 32x32 tiles for every CU at most: the waves of a workgroup share the k range, and there are
-    //    no partial tiles to add up (gemm.cpp: small_tile). In f32 only where the waves' sums are shorter than the shares' of
-    //    four k-tiles: up to 96 tiles the error against 64 bits of a 28x28x64 layer at batch 4 was 3.5e-7, with shares
-    //    3.0e-7 (of 16-bit gradients it is the same: their rounding is all of it).
-    const int64_t short_k = pr.mma_dtype == HE_F32 ? 24 : 96;
+    //    no partial tiles to add up (gemm.cpp: small_tile).
     const bool wide128 = !element_gather && pr.M > 64 && pr.M <= 128 && pr.N >= 512;
-    if (!wide128 && !element_gather && ((pr.M + 31) / 32) * ((pr.N + 31) / 32) <= 256 && k_tiles <= short_k) return 1;
+    if (!wide128 && !element_gather && ((pr.M + 31) / 32) * ((pr.N + 31) / 32) <= 256 && k_tiles <= 96) return 1;
     if (tuning::get("HELIUM_HIP_GEMM_NO_WIDE_CONV_TILES")) {
         // (the shares as they were, for comparison)
     } else if (wide128) {
@@ -1207,7 +1204,7 @@ bool over_repacked_image(const GemmProblem& pr, GemmProblem* packed, ConvRepack*
         packed->K = taps;
         resize(packed->op_a, packed->M, packed->K, g.N * g.Hp * g.Wp * 4);
         resize(packed->op_b, packed->N, packed->K, g.O * taps);
-        if (pr.split_k > 1) packed->split_k = choose_split_k(packed->M, packed->N, packed->K, 1, false);
+        if (pr.split_k > 1) packed->split_k = choose_split_k(packed->M, packed->N, packed->K, 1);
     } else {
         packed->N = taps;
         resize(packed->op_b, packed->K, packed->N, g.N * g.Hp * g.Wp * 4);

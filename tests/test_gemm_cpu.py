@@ -673,28 +673,3 @@ def test_epilogue_refuses_what_it_cannot_reduce():
     g.new_output(y); g.new_output(r)
     with pytest.raises(ha.HeliumError):
         ha.backend.matmul_kernel(g, [nd["id"] for nd in g.nodes if nd["node"] == "op"])
-
-
-@pytest.mark.parametrize("image,oc,stride", [((8, 16, 16, 16), 32, 1), ((4, 28, 28, 64), 64, 1), ((8, 32, 32, 32), 64, 2), ((1, 7, 7, 512), 512, 1),
-                                             ((1, 14, 14, 256), 256, 1), ((2, 6, 6, 200), 40, 1), ((1, 4, 4, 2000), 24, 1)])
-@pytest.mark.parametrize("op", ["conv", "conv_backward_data", "conv_backward_filter"])
-def test_partial_sums_of_f32_convolutions_stay_short(image, oc, stride, op):
-    """Each of the f32 sums that a result is added up from covers about eight 64-wide k-tiles (a filter gradient's: four), whether
-    workgroups share the k range or the waves of one, wherever the product leaves most of the chip idle."""
-    params = {"in_channels": image[3], "out_channels": oc, "kernel_size": [3, 3], "stride": [stride, stride]}
-    from oracle import helium_ir as oracle_ir
-
-    flow = [image[0], *oracle_ir.conv_output_size(params, image[1:3], (3, 3)), oc]
-    g = ha.ir.OpGraph()
-    x, w, dy = g.new_input(list(image), "f32"), g.new_input([oc, 3, 3, image[3]], "f32"), g.new_input(flow, "f32")
-    node = {"conv": lambda: g.conv(x, w, params), "conv_backward_data": lambda: g.conv_backward_data(dy, w, params, list(image[1:3])),
-            "conv_backward_filter": lambda: g.conv_backward_filter(dy, x, params)}[op]()
-    g.new_output(node)
-    description = ha.backend.matmul_kernel(g, [node]).description
-    for line in description.split("\n"):
-        if not line.startswith("gemm"):
-            continue
-        k, groups, split = (int(re.search(p, line).group(1)) for p in (r"gemm \[\d+,\d+,(\d+)\]", r"k_groups=(\d+)", r"split_k=(\d+)"))
-        tiles = -(-k // 64)
-        sums = -(-tiles // (split * groups))
-        assert sums <= (4 if op == "conv_backward_filter" else 8) * 1.5 or tiles < 16, line  # (shares are rounded down)
