@@ -777,7 +777,9 @@ GemmProblem gemm_problem_from_fusion(const fir::OpGraph& g) {
     return pr;
 }
 
-int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch) {
+int64_t most_shares(int64_t M, int64_t N) { return std::max<int64_t>(1, HE_NOALLOC_SCRATCH_BYTES / (M * N * 4)); }
+
+int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch, bool f32, bool by_element) {
     if (tuning::get("HELIUM_HIP_GEMM_NO_SPLIT_K") || batch != 1) return 1;
     if (const char* env = tuning::get("HELIUM_HIP_GEMM_SPLIT_K")) return std::max(1, atoi(env));
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128), k_tiles = (K + 63) / 64;
@@ -785,10 +787,26 @@ int choose_split_k(int64_t M, int64_t N, int64_t K, int64_t batch) {
     // 64x64 tiles fill the chip before a split k range has to: the partial tiles of a split cost a second pass over
     // the output (a 3136 x 512 x 4608 convolution: 51 us with 128x128 tiles and four k ranges, 34 us with 64x64 tiles)
     if (((M + 63) / 64) * ((N + 63) / 64) >= 192) return 1;
-    // So do the waves of a workgroup that share a small tile's k range (small_tile): such a product costs about 2.7 us and
-    // 0.2 us for every tile that a wave takes, the second launch of a split one 4 us (32 x 512 x 4608: 6.3 us against 10).
-    if (k_tiles <= 192) return 1;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 96, 1024}));
+    const int64_t split = std::min<int64_t>({(384 + tiles - 1) / tiles, k_tiles / 8, 1024});
+    // So do the waves of a workgroup that share a small tile's k range (small_tile), up to a length: such a product costs about
+    // 2.7 us and 0.2 us for every tile that a wave takes, a split one 10 us however long k is. Measured (us, waves / split) on
+    // 3x3 convolutions, rows x columns, by 64-wide k-tiles:
+    //  - 16 bits: 49x512 72 7.4 / 9.2, 129 11.9 / 11.7, 193 16.6 / 12.1; 196x512 129 12.5 / 16.8, 193 20.2 / 17.6; 784x64 129
+    //    12.2 / 14.8, 193 16.9 / 15.8; 784x512 129 27 / 29, 193 42 / 35;
+    //  - 16 bits gathered element by element (each chain three to six times as long): 49x256 19 16.6 / 24.4, 37 28.1 / 24.4, 73
+    //    51 / 23; 196x256 37 28 / 34, 73 52 / 32, 193 132 / 36;
+    //  - f32, against 64x64 tiles: 196x256 36 16 / 21, 72 27 / 20, 193 72 / 31; 784x256 72 29.5 / 32.5; against 128x128 ones: 49x512
+    //    72 27 / 50, 129 49 / 55, 193 72 / 55; gathered element by element: 49x256 97 62 / 66, 129 81 / 66.
+    const bool split_on_64 = M > 64 && N > 64 && tiles * split < 128;
+    const int64_t waves_up_to = !f32 ? (by_element ? 40 : 160) : split_on_64 ? 56 : by_element ? 112 : 144;
+    if (k_tiles <= waves_up_to || split < 2) return 1;
+    // No more shares than the allocation-free entry point has room for the partial tiles of; where that is fewer, the waves hold
+    // out longer: 392x512, 10 shares, 192 22.6 / 25.2 (24 shares 23.6), 288 27.1 / 28.6; f32 192 72 / 107 (91), 576 190 / 278
+    // (229), but 1568x384, 3 shares, 288 290 / 243 (10 shares 471).
+    const int64_t most = most_shares(M, N);
+    if (split <= most) return (int)split;
+    if (f32 ? ((M + 31) / 32) * ((N + 31) / 32) <= 400 : k_tiles <= (by_element ? 96 : 192)) return 1;
+    return (int)most;
 }
 
 bool operand_b_prefers_nk(const tp::Program& op_b) {

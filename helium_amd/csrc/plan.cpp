@@ -889,7 +889,7 @@ GemmProblem conv_problem(const ir::OpSubgraph& sg, NodeId conv) {
     pr.M = cv.N * cv.P * cv.Q;
     pr.N = op.conv.out_channels;
     pr.K = cv.R * cv.S * cv.C;
-    pr.split_k = choose_split_k(pr.M, pr.N, pr.K, 1);
+    pr.split_k = choose_split_k(pr.M, pr.N, pr.K, 1, image.dtype == HE_F32, cv.C % (image.dtype == HE_F32 ? 4 : 8) != 0);
     HE_REQUIRE(pr.M > 0 && pr.M < (1ll << 31) && ir::num_elements(image.shape) < (1ll << 32), HE_ERR_UNSUPPORTED, "conv too large for 32-bit tile indices");
     pr.mma_dtype = image.dtype == HE_F32 ? HE_F32 : image.dtype == HE_F16 ? HE_F16 : HE_BF16;
     auto operand = [&](tp::Program& p, const ir::Descriptor& d, NodeId node, int64_t rows, int64_t cols) {
@@ -995,7 +995,7 @@ GemmProblem conv_backward_data_problem(const ir::OpSubgraph& sg, NodeId node, in
     pr.M = cv.N * cv.P * cv.Q;
     pr.N = in_channels;
     pr.K = cv.R * cv.S * cv.C;
-    pr.split_k = cls >= 0 ? 1 : choose_split_k(pr.M, pr.N, pr.K, 1);
+    pr.split_k = cls >= 0 ? 1 : choose_split_k(pr.M, pr.N, pr.K, 1, flow.dtype == HE_F32, cv.C % (flow.dtype == HE_F32 ? 4 : 8) != 0);
     HE_REQUIRE(pr.M > 0 && pr.M < (1ll << 31) && ir::num_elements(flow.shape) < (1ll << 32), HE_ERR_UNSUPPORTED, "conv too large for 32-bit tile indices");
     pr.mma_dtype = flow.dtype == HE_F32 ? HE_F32 : flow.dtype == HE_F16 ? HE_F16 : HE_BF16;
     HE_REQUIRE(in_channels % (pr.mma_dtype == HE_F32 ? 4 : 8) == 0, HE_ERR_UNSUPPORTED,
@@ -1144,9 +1144,15 @@ int filter_gradient_split_k(const GemmProblem& pr, bool element_gather) {
     //  - 512 output channels keep 256x256 tiles, whose count, not that of 128x128 tiles, decides the shares as long as a
     //    share keeps 12 k-tiles: the 7x7x512 layer 36 x 4 = 144 workgroups 77.4 us, 36 x 7 = 252 workgroups 70.3.
     //  - a short k (few pixels) and 32x32 tiles for every CU at most: the waves of a workgroup share the k range, and there are
-    //    no partial tiles to add up (gemm.cpp: small_tile).
+    //    no partial tiles to add up (gemm.cpp: small_tile). Waves / shares in us, rows x columns by 64-wide k-tiles: 16 bits 32x288
+    //    36 4.7 / 8.2, 96 8.0 / 8.3; 128x144 64 6.4 / 8.3, 96 8.5 / 8.4; 256x288 96 8.3 / 13.4. f32 against 64x64 tiles 256x288 16
+    //    8.3 / 11.9, 32 13.7 / 12.8, 64 24 / 19, against 128x128 ones 64x576 64 24 / 27, 96 34 / 28, of channels that fill no
+    //    16-byte chunk 64x153 36 23 / 31, 64 37 / 31.
     const bool wide128 = !element_gather && pr.M > 64 && pr.M <= 128 && pr.N >= 512;
-    if (!wide128 && !element_gather && ((pr.M + 31) / 32) * ((pr.N + 31) / 32) <= 256 && k_tiles <= 96) return 1;
+    const bool shares_on_64 = pr.M > 64 && pr.N > 64 && tiles * split < 128;
+    // (f32 gradients of more partial tiles than the allocation-free entry point has room for keep to the waves)
+    const int64_t waves_up_to = pr.mma_dtype != HE_F32 || split > most_shares(pr.M, pr.N) ? 96 : shares_on_64 ? 24 : pr.conv_b.C % 4 ? 48 : 72;
+    if (!wide128 && !element_gather && ((pr.M + 31) / 32) * ((pr.N + 31) / 32) <= 256 && k_tiles <= waves_up_to) return 1;
     if (tuning::get("HELIUM_HIP_GEMM_NO_WIDE_CONV_TILES")) {
         // (the shares as they were, for comparison)
     } else if (wide128) {
@@ -1204,7 +1210,7 @@ bool over_repacked_image(const GemmProblem& pr, GemmProblem* packed, ConvRepack*
         packed->K = taps;
         resize(packed->op_a, packed->M, packed->K, g.N * g.Hp * g.Wp * 4);
         resize(packed->op_b, packed->N, packed->K, g.O * taps);
-        if (pr.split_k > 1) packed->split_k = choose_split_k(packed->M, packed->N, packed->K, 1);
+        if (pr.split_k > 1) packed->split_k = choose_split_k(packed->M, packed->N, packed->K, 1, false, false);
     } else {
         packed->N = taps;
         resize(packed->op_b, packed->K, packed->N, g.N * g.Hp * g.Wp * 4);

@@ -673,3 +673,60 @@ def test_epilogue_refuses_what_it_cannot_reduce():
     g.new_output(y); g.new_output(r)
     with pytest.raises(ha.HeliumError):
         ha.backend.matmul_kernel(g, [nd["id"] for nd in g.nodes if nd["node"] == "op"])
+
+
+def _convolution(op, image, oc, kernel, stride, dtype, make=None):
+    """A convolution's graph: (graph, the op's node, its inputs)."""
+    from oracle import helium_ir as oracle_ir
+
+    params = {"in_channels": image[3], "out_channels": oc, "kernel_size": [kernel, kernel], "stride": [stride, stride]}
+    g = ha.ir.OpGraph()
+    flow = [image[0], *oracle_ir.conv_output_size(params, image[1:3], (kernel, kernel)), oc]
+    x, w, dy = (lambda: g.new_input(list(image), dtype)), (lambda: g.new_input([oc, kernel, kernel, image[3]], dtype)), (lambda: g.new_input(flow, dtype))
+    a, b = {"conv": (x, w), "conv_backward_data": (dy, w), "conv_backward_filter": (dy, x)}[op]
+    a, b = a(), b()
+    node = {"conv": lambda: g.conv(a, b, params), "conv_backward_data": lambda: g.conv_backward_data(a, b, params, list(image[1:3])),
+            "conv_backward_filter": lambda: g.conv_backward_filter(a, b, params)}[op]()
+    g.new_output(node)
+    return g, node, (a, b)
+
+
+def _sharing(description):
+    """(k, k groups, shares) of each product a kernel's description names."""
+    return [tuple(int(re.search(p, line).group(1)) for p in (r"gemm \[\d+,\d+,(\d+)\]", r"k_groups=(\d+)", r"split_k=(\d+)"))
+            for line in description.split("\n") if line.startswith("gemm")]
+
+
+# the longest k of each line and one beyond it: channels of a 3x3 convolution (its k is nine times as long)
+@pytest.mark.parametrize("dtype,pixels,oc,waves,shares", [
+    ("bf16", 7, 512, 1136, 1144), ("bf16", 7, 256, 284, 285), ("f16", 4, 64, 1136, 1144),
+    ("f32", 7, 512, 1024, 1028), ("f32", 7, 256, 795, 797), ("f32", 14, 256, 396, 400)])
+@pytest.mark.parametrize("op", ["conv", "conv_backward_data"])
+def test_long_k_ranges_are_shared_by_workgroups(dtype, pixels, oc, waves, shares, op):
+    """Up to a length by the waves of a workgroup, beyond it by workgroups, in shares of eight 64-wide k-tiles."""
+    for channels, split in ((waves, False), (shares, True), (4 * shares, True)):
+        image, out = ((1, pixels, pixels, channels), oc) if op == "conv" else ((1, pixels, pixels, oc), channels)
+        g, node, _ = _convolution(op, image, out, 3, 1, dtype)
+        ((k, groups, got),) = _sharing(ha.backend.matmul_kernel(g, [node]).description)
+        tiles = -(-pixels * pixels // 128) * -(-oc // 128)
+        assert k == 9 * channels and got == (min(-(-384 // tiles), -(-k // 64) // 8) if split else 1), (channels, k, got)
+        assert (groups > 1) == (not split)
+
+
+@pytest.mark.parametrize("dtype,pixels,oc,waves,shares", [("bf16", 28, 512, 1360, 1400), ("f32", 28, 512, 4000, 4000), ("f32", 40, 384, 0, 1400)])
+def test_partial_tiles_fit_the_allocation_free_entry_point(dtype, pixels, oc, waves, shares):
+    """Shares of so large a result that its partial tiles would not fit: the waves keep the k range for longer, then as many as fit."""
+    for channels, split in ((waves, 1), (shares, 1 if waves == shares else (8 << 20) // (pixels * pixels * oc * 4))):
+        if not channels:
+            continue
+        g, node, _ = _convolution("conv", (1, pixels, pixels, channels), oc, 3, 1, dtype)
+        ((k, groups, got),) = _sharing(ha.backend.matmul_kernel(g, [node]).description)
+        assert got == split and (split > 1) == (groups == 1), (channels, k, got, groups)
+
+
+@pytest.mark.parametrize("dtype,oc,channels,line", [("bf16", 64, 32, 96), ("f32", 64, 32, 72), ("f32", 64, 17, 48), ("f32", 256, 32, 24)])
+def test_filter_gradients_of_many_pixels_are_shared_by_workgroups(dtype, oc, channels, line):
+    for tiles, split in ((line, False), (line + 1, True)):
+        g, node, _ = _convolution("conv_backward_filter", (tiles, 8, 8, channels), oc, 3, 1, dtype)
+        ((k, groups, got),) = _sharing(ha.backend.matmul_kernel(g, [node]).description)
+        assert k == 64 * tiles and (got > 1) == split and (groups > 1) == (not split), (tiles, got, groups)
