@@ -108,6 +108,14 @@ const char* kGemmBody = R"HIP(
 #endif
 #define KT_ALL ((GK + BK - 1) / BK)
 #define KT_PER_SPLIT ((KT_ALL + SPLIT_K - 1) / SPLIT_K)
+/* An f32 convolution whose k range the waves share (or workgroups, in long shares) adds up partial sums of this many k-tiles, as
+   many as the shares of a range that is split over workgroups have (eight 64-wide ones, a filter gradient's four): with one sum
+   per wave the error against 64 bits grew with the waves' share, 2.9e-7 to 4.1e-7 for the filter gradient of a 16x16x32 layer at
+   batch 16. (16-bit ones keep one sum: their operands' rounding is a thousand times that. Plain products were never split: one
+   sum per wave is a third of their error.) It costs 1 to 4%: 64 -> 64 channels of 28x28 at batch 4 20.2 -> 20.3 us, a 7x7x512
+   convolution 25.9 -> 27.0. */
+#define SUM_TILES (CONV_B ? 8 : 16)
+#define TWO_SUMS (MMA_F32 && (CONV_A || CONV_B) && (WAVES_K > 1 || SPLIT_K > 1) && (KT_PER_SPLIT + WAVES_K - 1) / WAVES_K > (SPLIT_K > 1 ? 32 : SUM_TILES))
 
 __device__ __forceinline__ u32 a_off(u32 m, u32 kc) { return m * (BK * ESZ) + ((kc ^ ((m >> A_SWZ_SHIFT) & (A_CHUNKS - 1))) << 4); }
 // B rows keep their memory order; the chunk index is XORed with 4 * (k % 4) for the transposing 16-bit reads
@@ -466,6 +474,24 @@ void fused_matmul(KERNEL_PARAMS) {
         for (int j = 0; j < NB; j++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+#if TWO_SUMS
+    f32x16 total[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) total[i][j] = acc[i][j];
+    auto take_sum = [&] {
+#pragma unroll
+        for (int i = 0; i < MB; i++)
+#pragma unroll
+            for (int j = 0; j < NB; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    total[i][j][e] += acc[i][j][e];
+                    acc[i][j][e] = 0.0f;
+                }
+    };
+#endif
 
     // Register staging of the operands that do not travel by direct global->LDS loads. A raw operand waits in
     // registers as the 16-byte chunk it was loaded as; a mainloop-fused one as its undecoded source vectors, which
@@ -658,9 +684,19 @@ void fused_matmul(KERNEL_PARAMS) {
         STAGE_SCHED_BARRIER
         if (more) stage_store(next, next % NSTAGES);
 #endif
+#if TWO_SUMS
+        if ((kt & (SUM_TILES - 1)) == SUM_TILES - 1) take_sum();
+#endif
         __builtin_amdgcn_sched_barrier(0);
     }
     finish_tiles(acc, frags);
+#if TWO_SUMS
+    take_sum();
+#pragma unroll
+    for (int i = 0; i < MB; i++)
+#pragma unroll
+        for (int j = 0; j < NB; j++) acc[i][j] = total[i][j];
+#endif
     __syncthreads();
 
     // ---- epilogue: accumulators -> wave-private LDS strip -> row-major NV-wide vectors -----------------------

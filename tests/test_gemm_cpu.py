@@ -2,6 +2,7 @@
 AddressSanitizer) against the oracle: index arithmetic, edge predication, mainloop and epilogue fusion."""
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -11,7 +12,7 @@ from oracle import fusion_ir as oracle
 from oracle import numerics as nm
 
 import gemm_cases
-from cpu_emul import run_kernel
+from cpu_emul import CLANG, run_kernel
 
 
 def launch_gemm(k, bufs):
@@ -697,6 +698,22 @@ def _sharing(description):
             for line in description.split("\n") if line.startswith("gemm")]
 
 
+@pytest.mark.parametrize("image,oc,stride", [((8, 16, 16, 16), 32, 1), ((4, 28, 28, 64), 64, 1), ((8, 32, 32, 32), 64, 2), ((1, 7, 7, 512), 512, 1),
+                                             ((1, 14, 14, 256), 256, 1), ((2, 6, 6, 200), 40, 1), ((1, 4, 4, 2000), 24, 1)])
+@pytest.mark.parametrize("op", ["conv", "conv_backward_data", "conv_backward_filter"])
+def test_partial_sums_of_f32_convolutions_stay_short(image, oc, stride, op):
+    """Each of the f32 sums that a result is added up from covers at most eight 64-wide k-tiles (a filter gradient's: four), whether the
+    waves of a workgroup share the k range or workgroups do (whose shares are rounded down)."""
+    g, node, _ = _convolution(op, image, oc, 3, stride, "f32")
+    kernel = ha.backend.matmul_kernel(g, [node])
+    sources = re.split(r"// ---- part \d+ of \d+\n", kernel.source)
+    for (k, groups, split), source in zip(_sharing(kernel.description), sources[1:] or sources):
+        assert "#define BK 32\n" in source and "#define MMA_F32 1" in source
+        text = subprocess.run([CLANG, "-E", "-P", "-x", "c++", "-"], input=source, capture_output=True, text=True, check=True).stdout
+        assert ("take_sum" in text) == (groups > 1 and -(-k // 32) > (8 if op == "conv_backward_filter" else 16) * groups), kernel.description
+        assert split == 1 or -(-k // 64) <= 12 * split, kernel.description
+
+
 # the longest k of each line and one beyond it: channels of a 3x3 convolution (its k is nine times as long)
 @pytest.mark.parametrize("dtype,pixels,oc,waves,shares", [
     ("bf16", 7, 512, 1136, 1144), ("bf16", 7, 256, 284, 285), ("f16", 4, 64, 1136, 1144),
@@ -730,3 +747,38 @@ def test_filter_gradients_of_many_pixels_are_shared_by_workgroups(dtype, oc, cha
         g, node, _ = _convolution("conv_backward_filter", (tiles, 8, 8, channels), oc, 3, 1, dtype)
         ((k, groups, got),) = _sharing(ha.backend.matmul_kernel(g, [node]).description)
         assert k == 64 * tiles and (got > 1) == split and (groups > 1) == (not split), (tiles, got, groups)
+
+
+@pytest.mark.parametrize("pixels,channels,oc", [((3, 11), 4096, 40), ((4, 8), 4100, 32), ((4, 5), 4400, 64), ((8, 8), 8196, 31)])
+def test_f32_convolutions_of_long_sums_on_cpu(pixels, channels, oc):
+    """The waves' second accumulators: k ranges that end with a partial sum of 16 k-tiles, right behind one, and in between."""
+    rng = np.random.default_rng(channels)
+    m, k = pixels[0] * pixels[1], channels
+    g, node, (x, w) = _convolution("conv", (1, *pixels, channels), oc, 1, 1, "f32")
+    values = rng.uniform(-1, 1, (m, k)).astype(np.float32), rng.uniform(-1, 1, (oc, k)).astype(np.float32)
+    _check_long_sums(g, node, (x, w), values, lambda a, b: a @ b.T, k, 512)
+
+
+@pytest.mark.parametrize("images,oc,channels", [(32, 32, 16), (33, 40, 12), (37, 24, 20), (48, 64, 8)])
+def test_f32_filter_gradients_of_long_sums_on_cpu(images, oc, channels):
+    """... of 8 k-tiles, over all pixels."""
+    rng = np.random.default_rng(images)
+    k = images * 64
+    g, node, (dy, x) = _convolution("conv_backward_filter", (images, 8, 8, channels), oc, 1, 1, "f32")
+    values = rng.uniform(-1, 1, (k, oc)).astype(np.float32), rng.uniform(-1, 1, (k, channels)).astype(np.float32)
+    _check_long_sums(g, node, (dy, x), values, lambda a, b: a.T @ b, k, 256)
+
+
+def _check_long_sums(g, node, nodes, values, product, k, most):
+    """`most`: how many products one sum may take."""
+    kernel, got = run_ir_kernel_on_cpu(g, [node], dict(zip(nodes, values)))
+    assert "k_groups=8" in kernel.description, kernel.description
+    want = product(*(v.astype(np.float64) for v in values))
+    # `most` products to a sum, k / `most` sums: each addition rounds by at most 2^-24 of a partial sum of terms below 1 (std 1/3)
+    assert np.abs(got[node].reshape(want.shape) - want).max() <= 2.0 ** -24 * (most + k / most) * np.sqrt(k) / 3
+    # a first term of 2^25 swallows the pairs of ones that come to the same sum, which are fewer than `most`
+    values = [np.ones_like(v) for v in values]
+    (values[0].T if values[0].shape[0] == k else values[0])[:, 0] = 2.0 ** 25
+    _, got = run_ir_kernel_on_cpu(g, [node], dict(zip(nodes, values)))
+    lost = 2.0 ** 25 + k - 1 - got[node]
+    assert (lost <= most + 4 * (k / most + 8)).all(), lost.max()  # (and each further addition rounds to a multiple of 4)
