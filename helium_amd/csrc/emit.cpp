@@ -628,7 +628,19 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
     // than half as much. A wave that moves 4 bytes per lane keeps too little in flight: a [5000 x 3001] f32 chain with four
     // operands, its values and two reductions of them 87.6 -> 68.5 us. (Small tensors are not bound by that.)
     const int nv_aligned = pick_nv(p, 16), nv_any = pick_nv(p, 16, true);
-    const bool guarded = nv_aligned * 4 <= nv_any && ir::num_elements(p.dims) >= 1 << 16 && !tuning::get("HELIUM_HIP_POINTWISE_NO_GUARD");
+    bool any_col = false, any_scalar = false, any_row = false;
+    for (auto& o : p.outs) {
+        if (!o.reduce) continue;
+        if (o.fold_m && !o.fold_n) any_col = true;
+        if (o.fold_m && o.fold_n) any_scalar = true;
+        if (!o.fold_m) any_row = true;
+    }
+    // Reductions that fold columns leave that many more partial results to the block that folds them, one element at a time: below
+    // a million elements that is longer than what the vectors save (a chain of ten operations with two such reductions, vectors /
+    // one element, us: 67x1001 6.6 / 5.6, 131x501 7.7 / 5.9, 200x3541 9.7 / 7.0; 150x8191 8.6 / 10.0, 600x3001 9.8 / 12.0), but for
+    // rows so short that a block spans several (8001x17 8.0 / 8.7), and where rows are reduced too, which a block then holds whole.
+    const bool folds = (any_col || any_scalar) && !any_row, worth = ir::num_elements(p.dims) >= (folds && N > 64 ? 1 << 20 : 1 << 16);
+    const bool guarded = nv_aligned * 4 <= nv_any && worth && !tuning::get("HELIUM_HIP_POINTWISE_NO_GUARD");
     const int NV = guarded ? nv_any : nv_aligned;
     const std::string row_end = guarded ? "(DIM_N - n0)" : "", row_inside = guarded ? "(u32)NV" : "";
     const int threads = 256;
@@ -638,12 +650,6 @@ PointwiseLaunch emit_pointwise(const Program& p, const std::string& entry) {
     auto scaled = [](const Out& o, const std::string& x) {
         return o.rop == ROp::Mean ? strfmt("(float)((double)(%s) * %.17g)", x.c_str(), o.mean_scale) : x;
     };
-    bool any_col = false, any_scalar = false;
-    for (auto& o : p.outs) {
-        if (!o.reduce) continue;
-        if (o.fold_m && !o.fold_n) any_col = true;
-        if (o.fold_m && o.fold_n) any_scalar = true;
-    }
     // Threads along a row. With a column reduction a block should be tall rather than wide: its TY row groups are
     // combined in LDS, so every block leaves one partial per column it spans, not one per column per row group.
     int tx_cap = any_col ? 64 : threads;

@@ -91,3 +91,10 @@ def test_rows_of_odd_length_move_as_guarded_vectors(shape):
 @pytest.mark.parametrize("axis", [1, 2])
 def test_c3_chain_of_odd_rows_on_cpu(axis):
     test_c3_chain_on_cpu(93, 707, axis)
+
+
+@pytest.mark.parametrize("rows,cols,width", [(67, 1001, 1), (200, 3541, 1), (600, 3001, 4), (8001, 17, 4), (1024, 64, 4), (60, 1001, 1)])
+def test_odd_rows_under_column_reductions_are_vectors_where_those_pay(rows, cols, width):
+    """Below a million elements the partial results of wider lanes cost more than the lanes save, but for short rows."""
+    g, _, _ = configs.c3_chain(rows, cols, make_inputs=False)
+    assert f" NV={width} " in ha.TileKernel.auxiliary(g).description
