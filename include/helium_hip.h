@@ -409,8 +409,9 @@ int he_fgraph_subdivide(he_fgraph_t graph, uint64_t* nodes, int32_t* portions, i
  * HE_OPT_STREAM_FAN_OUT (default 1): how the independent instructions of a plan step are spread over the calling
  * thread's streams. 2: every step with several instructions fans out and the next step waits for all of its streams
  * (helium/src/cuda.rs:190-221). 1: only steps whose instructions are too small to fill the device and numerous enough to
- * outweigh the joins (each costs the host 15-20 us here), those of up to 1 MB that share launches counted as one; all others run on the first stream in plan order. 0: one
- * stream. Takes effect from the next he_execute_graph; results do not depend on it. */
+ * outweigh the joins (each costs the host 15-20 us here), those of up to 1 MB that share launches counted as one; all
+ * others run on the first stream in plan order. 0: one stream. Takes effect from the next he_execute_graph; results do
+ * not depend on it. */
 enum { HE_OPT_FUSE_MATMUL_EPILOGUE = 0, HE_OPT_FOLD_SWAP_INTO_REDUCE = 1, HE_OPT_REMATERIALIZE = 2, HE_OPT_CANCEL_TRANSPOSES = 3,
        HE_OPT_HOIST_BROADCASTS = 4, HE_OPT_STREAM_FAN_OUT = 5 };
 int he_backend_set_option(int option, int64_t value);
