@@ -1,5 +1,6 @@
-// The kernel compiler as a process of its own: source text on stdin, `name option...` as arguments (or `--version`), the code
-// object (which compiler this is) on stdout behind one byte ('o': code object, 'e': the compiler's log) and its length in eight. rtc.cpp says why it is not called in-process.
+// The kernel compiler as a process of its own: source text on stdin and `name option...` as arguments, or `--version` alone. The
+// answer goes to stdout: a byte for its kind ('o': the code object, or which compiler this is; 'e': the compiler's log), its
+// length in eight bytes, and itself. rtc.cpp says why the compiler is not called in-process.
 #include <hip/hiprtc.h>
 #include <limits.h>
 #include <link.h>
